@@ -100,7 +100,7 @@ struct smac_ctx {
   double* fstage = nullptr;  // 3*1024 lane sums of the two-stage reductions
   std::vector<Level> lev;
   double* cinv = nullptr;
-  double* cinv_ws = nullptr;  // the factor of the coarsest operator (n x n)
+  double* cinv_ws = nullptr;  // work array of the coarsest inverse
   int cinv_n = 0;
   // the coarsest inverse is rebuilt on a second stream (default priority),
   // next to the predictor; the solve waits for ev_side_out before its first
@@ -951,7 +951,7 @@ static int mg_coeffs(smac_ctx* c) {
     if (rc) return rc;
   }
   if (!c->cinv_ws) {
-    int rc = dalloc(&c->cinv_ws, (size_t)n * n);
+    int rc = dalloc(&c->cinv_ws, dense_pinv_work(n));
     if (rc) return rc;
   }
   // an outlet makes the operator regular: a plain inverse, else the

@@ -291,7 +291,8 @@ void launch_fill(const Lv& L, T* x, hipStream_t st);
 // coarse face coefficients of axis d on level C from level F (k_mg_coarsen_beta)
 void launch_mg_coarsen_beta(const Lv& F, const Lv& C, int d, double* cb, hipStream_t st);
 // dense (pseudo-)inverse of the coarsest level's operator into out (n x n,
-// n = cells of C; work: n x n scratch), on the device
+// n = cells of C <= 1024; work: dense_pinv_work(n) doubles), on the device
+size_t dense_pinv_work(int n);
 void launch_dense_pinv(const Lv& C, int singular, double* work, double* out, hipStream_t st);
 
 // the reference's multigrid (smac_refgmg.hip); fb == nullptr: coefficients

@@ -1521,14 +1521,8 @@ void launch_mg_coarsen_beta(const Lv& F, const Lv& C, int d, double* cb, hipStre
   hipLaunchKernelGGL(k_mg_coarsen_beta, g, dim3(64, 4), 0, st, F, C, d, cb);
 }
 
-// Dense (pseudo-)inverse of the coarsest operator in one workgroup: the
-// operator from the level's coefficients (the uniform rule, or the face
-// coefficient arrays), shifted by c J (c = A00 / n) when singular, its
-// Cholesky factor column by column, the inverse column by column by forward
-// and back substitution, minus J / (c n^2). Every sum runs in the order of
-// the sequential algorithm (dot products in increasing k), with one thread per
-// row (factor) or per column (substitution), so the result is that of the
-// plain host loops bit for bit. A and out are n x n, row-major.
+// the six off-diagonal terms and the diagonal of a coarsest cell, from the
+// uniform rule or the face coefficient arrays
 __device__ void coarsest_coef(const Lv& L, int i, int j, int k, double a6[6], double* diag) {
   const int q[3] = {i, j, k};
 #pragma unroll
@@ -1558,180 +1552,256 @@ __device__ void coarsest_coef(const Lv& L, int i, int j, int k, double a6[6], do
   }
 }
 
-constexpr int PINV_LN = 128, PINV_LB = 64;
-__device__ __forceinline__ int tri(int i, int k) { return i * (i + 1) / 2 + k; }
-// acc - a(k0) b(k0) - a(k0+1) b(k0+1) - ... - a(k1-1) b(k1-1), subtracted in
-// that order; the operands are read 16 at a time ahead of the subtractions
-template <class FA, class FB>
-__device__ __forceinline__ double sub_dot(double acc, int k0, int k1, const FA& a, const FB& b) {
-  int k = k0;
-  for (; k + 16 <= k1; k += 16) {
-    double x[16], y[16];
-#pragma unroll
-    for (int u = 0; u < 16; u++) {
-      x[u] = a(k + u);
-      y[u] = b(k + u);
-    }
-#pragma unroll
-    for (int u = 0; u < 16; u++) acc -= x[u] * y[u];
-  }
-  for (; k < k1; k++) acc -= a(k) * b(k);
-  return acc;
-}
-constexpr int PINV_T = 1024;
-__global__ __launch_bounds__(PINV_T) void k_dense_pinv(Lv L, int singular, double* __restrict__ A,
-                                                    double* __restrict__ out) {
+// ---- dense (pseudo-)inverse of the coarsest operator (up to 1024 cells), in
+// the order of the sequential algorithm: every sum runs over increasing k,
+// rounded term by term, so the result is that of plain host loops bit for bit.
+//
+// The matrix M is the operator (shifted by c J, c = A00 / n, when singular)
+// with the identity below it, 2n x n row-major. Its Cholesky factorization by
+// right-looking panels of 32 columns leaves L on top and, in the rows below,
+// the forward substitutions of the identity's columns (row n + r, entry j =
+// y_j of column r: the same products and order as a factor row). A launch per
+// panel updates all trailing 32 x 32 tiles at once; each tile's block factors
+// the panel's diagonal block again for itself (the two waves that need it
+// hold a row per lane in registers and broadcast by readlane, no barrier),
+// which costs less than a launch of its own per panel. The back substitution
+// subtracts l_ki x_k in increasing k, newest first, so it is one serial chain
+// of n^2/2 subtractions per column: a wave owns a few columns with x in LDS
+// and the other three waves stage the rows of L^T ahead of it. That chain is
+// the bound. One workgroup for everything (a column at a time, operands from
+// the L2) took 29.6 ms for 480 cells and 0.53 ms for 90.
+constexpr int PB = 32;       // panel and tile width
+constexpr int PINV_MAX = 1024;
+
+// M <- [A + c J; I], and c behind the matrices
+__global__ __launch_bounds__(128) void k_pinv_assemble(Lv L, int singular, double* __restrict__ M,
+                                                       double* __restrict__ cshift_out) {
   const int n = L.n[0] * L.n[1] * L.n[2];
-  const int t = (int)threadIdx.x;
-  const size_t nn = (size_t)n * n;
-  __shared__ double djj_s, cshift_s;
-  for (size_t e = t; e < nn; e += PINV_T) A[e] = 0.0;
+  const int row = (int)blockIdx.x, t = (int)threadIdx.x;
+  double* m = M + (size_t)row * n;
+  if (row >= n) {
+    for (int e = t; e < n; e += 128) m[e] = e == row - n ? 1.0 : 0.0;
+    return;
+  }
+  __shared__ double a[PINV_MAX];
+  __shared__ double cs;
+  for (int e = t; e < n; e += 128) a[e] = 0.0;
   __syncthreads();
-  for (int row = t; row < n; row += PINV_T) {
-    const int i = row % L.n[0] + 1, j = (row / L.n[0]) % L.n[1] + 1, k = row / (L.n[0] * L.n[1]) + 1;
-    double a6[6], diag;
+  // thread 0: this row; thread 64: A00, from row 0's terms in the same order
+  if (t == 0 || t == 64) {
+    const int r = t == 0 ? row : 0;
+    const int i = r % L.n[0] + 1, j = (r / L.n[0]) % L.n[1] + 1, k = r / (L.n[0] * L.n[1]) + 1;
+    double a6[6], diag, a00 = 0.0;
     coarsest_coef(L, i, j, k, a6, &diag);
-    A[(size_t)row * n + row] += diag;
+    if (t == 0) a[r] += diag;
+    a00 += diag;
     const int nb[6][3] = {{i + 1, j, k}, {i - 1, j, k}, {i, j + 1, k}, {i, j - 1, k}, {i, j, k + 1}, {i, j, k - 1}};
-    for (int m = 0; m < 6; m++) {
-      if (a6[m] == 0.) continue;
-      int q[3] = {nb[m][0], nb[m][1], nb[m][2]};
+#pragma unroll
+    for (int q6 = 0; q6 < 6; q6++) {
+      if (a6[q6] == 0.) continue;
+      int q[3] = {nb[q6][0], nb[q6][1], nb[q6][2]};
+#pragma unroll
       for (int d = 0; d < 3; d++)
         if (L.per[d]) q[d] = wrapi(q[d], L.n[d]);
       const int col = ((q[2] - 1) * L.n[1] + (q[1] - 1)) * L.n[0] + (q[0] - 1);
-      A[(size_t)row * n + col] -= a6[m];
+      if (t == 0) a[col] -= a6[q6];
+      if (col == 0) a00 -= a6[q6];
+    }
+    if (t == 64) {
+      cs = singular ? a00 / (double)n : 0.0;
+      if (row == 0) *cshift_out = cs;
     }
   }
   __syncthreads();
-  if (t == 0) cshift_s = singular ? A[0] / (double)n : 0.0;
+  const double c = cs;
+  for (int e = t; e < n; e += 128) m[e] = singular ? a[e] + c : a[e];
+}
+
+__device__ __forceinline__ double rdlane(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Panel c0 .. c0+31: block (I, J) owns the trailing tile of rows
+// c1 + 32 I .., columns c1 + 32 J .. (c1 = min(c0 + 32, n)). The J = 0 blocks write
+// their rows of the panel's factor, and block (0, 0) the diagonal block, to
+// LT (n x 2n, LT[c][r] = l_rc).
+__global__ __launch_bounds__(256) void k_pinv_panel(double* __restrict__ M, double* __restrict__ LT, int n, int c0) {
+  const int c1 = min(c0 + PB, n);
+  const int r0 = c1 + PB * (int)blockIdx.x, k0 = c1 + PB * (int)blockIdx.y;
+  const int last = r0 + PB - 1;  // last row of the strip
+  // tiles above the diagonal, and identity rows whose first entry is still to come
+  if (last < n && blockIdx.x < blockIdx.y) return;
+  if (r0 - n >= c1) return;
+  __shared__ double LI[PB][PB + 1], LJ[PB][PB + 1], LD[PB][PB + 1];
+  const int t = (int)threadIdx.x, w = t >> 6, lane = t & 63, l32 = t & 31;
+  if (w < 2) {
+    // lanes 0..31: the diagonal block's rows; 32..63: the strip's (wave 0) or
+    // the tile columns' rows (wave 1)
+    const bool dia = lane < PB;
+    const int row = dia ? c0 + l32 : (w == 0 ? r0 + l32 : k0 + l32);
+    const bool ok = dia ? row < n : (w == 0 ? row < 2 * n : row < n);
+    double v[PB];
+#pragma unroll
+    for (int c = 0; c < PB; c++)
+      v[c] = ok && c0 + c < n ? M[(size_t)row * n + c0 + c] : (dia && c == l32 ? 1.0 : 0.0);
+#pragma unroll
+    for (int jc = 0; jc < PB; jc++) {
+      const double d = sqrt(rdlane(v[jc], jc));
+      const double q = v[jc] / d;
+      v[jc] = lane == jc ? d : q;
+#pragma unroll
+      for (int c = jc + 1; c < PB; c++) v[c] -= v[jc] * rdlane(v[jc], c);
+    }
+    if (!dia) {
+#pragma unroll
+      for (int c = 0; c < PB; c++) (w == 0 ? LI : LJ)[l32][c] = v[c];
+    } else if (w == 0) {
+#pragma unroll
+      for (int c = 0; c < PB; c++) LD[l32][c] = v[c];
+    }
+  }
   __syncthreads();
-  const double cshift = cshift_s;
-  if (singular) {
-    for (size_t e = t; e < nn; e += PINV_T) A[e] += cshift;
-    __syncthreads();
-  }
-  for (int jc = 0; jc < n; jc++) {
-    if (t == 0) {
-      const double* aj = A + (size_t)jc * n;
-      auto lj = [&](int k) { return aj[k]; };
-      const double s = sub_dot(aj[jc], 0, jc, lj, lj);
-      const double d = sqrt(s);
-      A[(size_t)jc * n + jc] = d;
-      djj_s = d;
-    }
-    __syncthreads();
-    const double djj = djj_s;
-    const double* aj = A + (size_t)jc * n;
-    for (int i = jc + 1 + t; i < n; i += PINV_T) {
-      double* ai = A + (size_t)i * n;
-      const double tt = sub_dot(ai[jc], 0, jc, [&](int k) { return ai[k]; }, [&](int k) { return aj[k]; });
-      ai[jc] = tt / djj;
-    }
-    __syncthreads();
-  }
-  for (int col = t; col < n; col += PINV_T) {
-    // y = the column of the inverse, kept in out's column col
-    auto yk = [&](int k) { return out[(size_t)k * n + col]; };
-    for (int i = 0; i < n; i++) {
-      const double* ai = A + (size_t)i * n;
-      const double tt = sub_dot((i == col) ? 1.0 : 0.0, 0, i, [&](int k) { return ai[k]; }, yk);
-      out[(size_t)i * n + col] = tt / ai[i];
-    }
-    for (int i = n - 1; i >= 0; i--) {
-      const double tt = sub_dot(out[(size_t)i * n + col], i + 1, n, [&](int k) { return A[(size_t)k * n + i]; }, yk);
-      out[(size_t)i * n + col] = tt / A[(size_t)i * n + i];
+  if (blockIdx.y == 0) {
+    for (int c = t >> 5; c < PB && c0 + c < n; c += 8) {
+      double* o = LT + (size_t)(c0 + c) * (2 * (size_t)n);
+      if (r0 + l32 < 2 * n) o[r0 + l32] = LI[l32][c];
+      if (blockIdx.x == 0 && l32 >= c && c0 + l32 < n) o[c0 + l32] = LD[l32][c];
     }
   }
-  if (singular) {
+  const int col = k0 + l32;
+  if (col >= n) return;
+  double acc[4];
+  bool in[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int r = r0 + (t >> 5) + 8 * q;
+    in[q] = r < 2 * n && (r >= n || col <= r);
+    acc[q] = in[q] ? M[(size_t)r * n + col] : 0.0;
+  }
+#pragma unroll 8
+  for (int k = 0; k < PB; k++) {
+    const double lj = LJ[l32][k];
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc[q] -= LI[(t >> 5) + 8 * q][k] * lj;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (in[q]) M[(size_t)(r0 + (t >> 5) + 8 * q) * n + col] = acc[q];
+}
+
+// x_i = (y_i - l_{i+1,i} x_{i+1} - ... - l_{n-1,i} x_{n-1}) / l_ii, i = n-1..0,
+// for the CB columns c = CB blockIdx.x + lane of wave 0 (n CB <= 8192); waves
+// 1..3 stage the next G rows of L^T and of y (2 G n <= 8192).
+template <int CB, int G>
+__global__ __launch_bounds__(256) void k_pinv_back(const double* __restrict__ LT, const double* __restrict__ cshift,
+                                                   int n, int singular, double* __restrict__ out) {
+  __shared__ double xs[8192];
+  __shared__ double ls[8192];
+  __shared__ double ys[2 * G * CB];
+  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+  const int c = CB * (int)blockIdx.x + lane;
+  const size_t ld = 2 * (size_t)n;
+  // group g holds the rows i = hi(g) .. hi(g)-G+1, hi(g) = n-1-G g (row i at
+  // slot hi - i); wave wi of nw takes every nw-th row
+  auto stage = [&](int g, int wi, int nw) {
+    const int hi = n - 1 - G * g;
+    double* lb = ls + (g & 1) * G * n;
+    double* yb = ys + (g & 1) * G * CB;
+    for (int s = wi; s < G && hi - s >= 0; s += nw) {
+      const int i = hi - s;
+      const double* src = LT + (size_t)i * ld;
+      for (int k = i + lane; k < n; k += 256) {
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = k + 64 * u < n ? src[k + 64 * u] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (k + 64 * u < n) lb[s * n + k + 64 * u] = v[u];
+      }
+    }
+    for (int e = 64 * wi + lane; e < G * CB; e += 64 * nw) {
+      const int i = hi - e / CB, r = CB * (int)blockIdx.x + e % CB;
+      // y_i of column r is 0 before its own row
+      yb[e] = i >= r && r < n && i >= 0 ? LT[(size_t)i * ld + n + r] : 0.0;
+    }
+  };
+  stage(0, w, 4);
+  __syncthreads();
+  const double corr = singular ? 1.0 / (*cshift * (double)n * (double)n) : 0.0;
+  const int ng = (n + G - 1) / G;
+  double xl = 0.0;  // x_{i+1}
+  for (int g = 0; g < ng; g++) {
+    if (w > 0) {
+      if (g + 1 < ng) stage(g + 1, w - 1, 3);
+    } else if (lane < CB) {
+      const int hi = n - 1 - G * g;
+      const double* yb = ys + (g & 1) * G * CB + lane;
+      const double* xb = xs + lane;
+      for (int s = 0; s < G && hi - s >= 0; s++) {
+        const int i = hi - s;
+        const double* l = ls + (g & 1) * G * n + s * n;
+        double acc = yb[s * CB];
+        int k = i + 1;
+        if (k < n) acc -= l[k] * xl;
+        k++;
+        constexpr int U = 16;
+        double a[U], b[U];
+        if (k + U <= n) {
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            a[u] = l[k + u];
+            b[u] = xb[(k + u) * CB];
+          }
+          for (; k + 2 * U <= n; k += U) {
+            double a2[U], b2[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+              a2[u] = l[k + U + u];
+              b2[u] = xb[(k + U + u) * CB];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) acc -= a[u] * b[u];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+              a[u] = a2[u];
+              b[u] = b2[u];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; u++) acc -= a[u] * b[u];
+          k += U;
+        }
+        for (; k < n; k++) acc -= l[k] * xb[k * CB];
+        xl = acc / l[i];
+        xs[i * CB + lane] = xl;
+        if (c < n) out[(size_t)i * n + c] = singular ? xl - corr : xl;
+      }
+    }
     __syncthreads();
-    const double corr = 1.0 / (cshift * (double)n * (double)n);
-    for (size_t e = t; e < nn; e += PINV_T) out[e] -= corr;
   }
 }
-// The same for n <= 128 (a coarsest level of up to 128 cells, rebuilt with
-// every change of the coefficients) with the operations on LDS: the packed
-// lower triangle (all the factorization reads; the assembled operator is
-// symmetric entry for entry) and the solution columns 64 at a time (k-major,
-// so the column threads read consecutive words). Same arithmetic, same order.
-__global__ __launch_bounds__(PINV_T) void k_dense_pinv_lds(Lv L, int singular, double* __restrict__ out) {
-  __shared__ double Ls[PINV_LN * (PINV_LN + 1) / 2];
-  __shared__ double Ys[PINV_LN * PINV_LB];
-  __shared__ double djj_s, cshift_s;
-  const int n = L.n[0] * L.n[1] * L.n[2];
-  const int t = (int)threadIdx.x;
-  const int ntri = n * (n + 1) / 2;
-  for (int e = t; e < ntri; e += PINV_T) Ls[e] = 0.0;
-  __syncthreads();
-  for (int row = t; row < n; row += PINV_T) {
-    const int i = row % L.n[0] + 1, j = (row / L.n[0]) % L.n[1] + 1, k = row / (L.n[0] * L.n[1]) + 1;
-    double a6[6], diag;
-    coarsest_coef(L, i, j, k, a6, &diag);
-    Ls[tri(row, row)] += diag;
-    const int nb[6][3] = {{i + 1, j, k}, {i - 1, j, k}, {i, j + 1, k}, {i, j - 1, k}, {i, j, k + 1}, {i, j, k - 1}};
-    for (int m = 0; m < 6; m++) {
-      if (a6[m] == 0.) continue;
-      int q[3] = {nb[m][0], nb[m][1], nb[m][2]};
-      for (int d = 0; d < 3; d++)
-        if (L.per[d]) q[d] = wrapi(q[d], L.n[d]);
-      const int col = ((q[2] - 1) * L.n[1] + (q[1] - 1)) * L.n[0] + (q[0] - 1);
-      if (col <= row) Ls[tri(row, col)] -= a6[m];
-    }
-  }
-  __syncthreads();
-  if (t == 0) cshift_s = singular ? Ls[0] / (double)n : 0.0;
-  __syncthreads();
-  const double cshift = cshift_s;
-  if (singular) {
-    for (int e = t; e < ntri; e += PINV_T) Ls[e] += cshift;
-    __syncthreads();
-  }
-  for (int jc = 0; jc < n; jc++) {
-    if (t == 0) {
-      const int rj = tri(jc, 0);
-      auto lj = [&](int k) { return Ls[rj + k]; };
-      const double s = sub_dot(Ls[tri(jc, jc)], 0, jc, lj, lj);
-      const double d = sqrt(s);
-      Ls[tri(jc, jc)] = d;
-      djj_s = d;
-    }
-    __syncthreads();
-    const double djj = djj_s;
-    const int rj = tri(jc, 0);
-    for (int i = jc + 1 + t; i < n; i += PINV_T) {
-      const int ri = tri(i, 0);
-      const double tt = sub_dot(Ls[ri + jc], 0, jc, [&](int k) { return Ls[ri + k]; }, [&](int k) { return Ls[rj + k]; });
-      Ls[ri + jc] = tt / djj;
-    }
-    __syncthreads();
-  }
-  for (int c0 = 0; c0 < n; c0 += PINV_LB) {
-    const int cl = t, col = c0 + t;
-    if (t < PINV_LB && col < n) {
-      auto yk = [&](int k) { return Ys[k * PINV_LB + cl]; };
-      for (int i = 0; i < n; i++) {
-        const int ri = tri(i, 0);
-        const double tt = sub_dot((i == col) ? 1.0 : 0.0, 0, i, [&](int k) { return Ls[ri + k]; }, yk);
-        Ys[i * PINV_LB + cl] = tt / Ls[ri + i];
-      }
-      for (int i = n - 1; i >= 0; i--) {
-        const double tt = sub_dot(Ys[i * PINV_LB + cl], i + 1, n, [&](int k) { return Ls[tri(k, i)]; }, yk);
-        Ys[i * PINV_LB + cl] = tt / Ls[tri(i, i)];
-      }
-      for (int i = 0; i < n; i++) out[(size_t)i * n + col] = Ys[i * PINV_LB + cl];
-    }
-  }
-  if (singular) {
-    __syncthreads();
-    const double corr = 1.0 / (cshift * (double)n * (double)n);
-    for (size_t e = t; e < (size_t)n * n; e += PINV_T) out[e] -= corr;
-  }
-}
+
+size_t dense_pinv_work(int n) { return 4 * (size_t)n * n + 1; }
 void launch_dense_pinv(const Lv& C, int singular, double* work, double* out, hipStream_t st) {
   const int n = C.n[0] * C.n[1] * C.n[2];
-  if (n <= PINV_LN)
-    hipLaunchKernelGGL(k_dense_pinv_lds, dim3(1), dim3(PINV_T), 0, st, C, singular, out);
-  else
-    hipLaunchKernelGGL(k_dense_pinv, dim3(1), dim3(PINV_T), 0, st, C, singular, work, out);
+  double* LT = work + 2 * (size_t)n * n;
+  double* cs = work + 4 * (size_t)n * n;
+  hipLaunchKernelGGL(k_pinv_assemble, dim3((unsigned)(2 * n)), dim3(128), 0, st, C, singular, work, cs);
+  for (int c0 = 0; c0 < n; c0 += PB) {
+    const int c1 = c0 + PB < n ? c0 + PB : n;
+    const int ni = (2 * n - c1 + PB - 1) / PB, nj = c1 < n ? (n - c1 + PB - 1) / PB : 1;
+    hipLaunchKernelGGL(k_pinv_panel, dim3((unsigned)ni, (unsigned)nj), dim3(256), 0, st, work, LT, n, c0);
+  }
+  // the columns per wave and the rows staged ahead that fit the LDS
+#define SMAC_PBACK(CB, G) \
+  hipLaunchKernelGGL((k_pinv_back<CB, G>), dim3((unsigned)((n + CB - 1) / CB)), dim3(256), 0, st, LT, cs, n, singular, out)
+  if (n <= 256) SMAC_PBACK(32, 16);
+  else if (n <= 512) SMAC_PBACK(16, 8);
+  else SMAC_PBACK(8, 4);
+#undef SMAC_PBACK
 }
 
 template <typename T>
