@@ -1568,8 +1568,10 @@ __device__ void coarsest_coef(const Lv& L, int i, int j, int k, double a6[6], do
 // subtracts l_ki x_k in increasing k, newest first, so it is one serial chain
 // of n^2/2 subtractions per column: a wave owns a few columns with x in LDS
 // and the other three waves stage the rows of L^T ahead of it. That chain is
-// the bound. One workgroup for everything (a column at a time, operands from
-// the L2) took 29.6 ms for 480 cells and 0.53 ms for 90.
+// the bound (12 ns a step of a lone wave). 512 cells 1.8 ms (16 panels of 14 to
+// 20 us, then 1.55 ms), 128 cells 0.23 ms, 90 cells 0.14 ms; one workgroup for
+// everything (a column at a time, operands from the L2) took 29.6 ms for 480
+// cells, 0.99 ms for 128 and 0.53 ms for 90.
 constexpr int PB = 32;       // panel and tile width
 constexpr int PINV_MAX = 1024;
 
@@ -1693,22 +1695,29 @@ __global__ __launch_bounds__(256) void k_pinv_panel(double* __restrict__ M, doub
 }
 
 // x_i = (y_i - l_{i+1,i} x_{i+1} - ... - l_{n-1,i} x_{n-1}) / l_ii, i = n-1..0,
-// for the CB columns c = CB blockIdx.x + lane of wave 0 (n CB <= 8192); waves
-// 1..3 stage the next G rows of L^T and of y (2 G n <= 8192).
-template <int CB, int G>
+// for the CB columns c = CB blockIdx.x + lane of wave 0 (n <= NM); waves 1..3
+// stage the next G rows of L^T and of y. The chain's operands are read two
+// chunks of 16 ahead and its products formed one chunk ahead, past the end of a
+// row into zeros, so that its steps are subtractions only; of the newest x only
+// x_{i+1}, kept in a register, is younger than the loads.
+template <int CB, int G, int NM>
 __global__ __launch_bounds__(256) void k_pinv_back(const double* __restrict__ LT, const double* __restrict__ cshift,
                                                    int n, int singular, double* __restrict__ out) {
-  __shared__ double xs[8192];
-  __shared__ double ls[8192];
+  constexpr int U = 16, ST = NM + 5 * U;
+  __shared__ double xs[ST * CB];
+  __shared__ double ls[2 * G * ST];
   __shared__ double ys[2 * G * CB];
   const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
   const int c = CB * (int)blockIdx.x + lane;
   const size_t ld = 2 * (size_t)n;
+  for (int e = (int)threadIdx.x; e < ST * CB; e += 256) xs[e] = 0.0;
+  for (int e = (int)threadIdx.x; e < 2 * G * ST; e += 256) ls[e] = 0.0;
+  __syncthreads();
   // group g holds the rows i = hi(g) .. hi(g)-G+1, hi(g) = n-1-G g (row i at
   // slot hi - i); wave wi of nw takes every nw-th row
   auto stage = [&](int g, int wi, int nw) {
     const int hi = n - 1 - G * g;
-    double* lb = ls + (g & 1) * G * n;
+    double* lb = ls + (g & 1) * G * ST;
     double* yb = ys + (g & 1) * G * CB;
     for (int s = wi; s < G && hi - s >= 0; s += nw) {
       const int i = hi - s;
@@ -1719,7 +1728,7 @@ __global__ __launch_bounds__(256) void k_pinv_back(const double* __restrict__ LT
         for (int u = 0; u < 4; u++) v[u] = k + 64 * u < n ? src[k + 64 * u] : 0.0;
 #pragma unroll
         for (int u = 0; u < 4; u++)
-          if (k + 64 * u < n) lb[s * n + k + 64 * u] = v[u];
+          if (k + 64 * u < n) lb[s * ST + k + 64 * u] = v[u];
       }
     }
     for (int e = 64 * wi + lane; e < G * CB; e += 64 * nw) {
@@ -1739,43 +1748,43 @@ __global__ __launch_bounds__(256) void k_pinv_back(const double* __restrict__ LT
     } else if (lane < CB) {
       const int hi = n - 1 - G * g;
       const double* yb = ys + (g & 1) * G * CB + lane;
-      const double* xb = xs + lane;
       for (int s = 0; s < G && hi - s >= 0; s++) {
         const int i = hi - s;
-        const double* l = ls + (g & 1) * G * n + s * n;
-        double acc = yb[s * CB];
-        int k = i + 1;
-        if (k < n) acc -= l[k] * xl;
-        k++;
-        constexpr int U = 16;
-        double a[U], b[U];
-        if (k + U <= n) {
+        const double* l = ls + (g & 1) * G * ST + s * ST + i;
+        const double* x = xs + i * CB + lane;
+        double a0[U], b0[U], a1[U], b1[U], p0[U], p1[U];
+        auto rd = [&](double* a, double* b, int k) {
 #pragma unroll
           for (int u = 0; u < U; u++) {
             a[u] = l[k + u];
-            b[u] = xb[(k + u) * CB];
+            b[u] = x[(k + u) * CB];
           }
-          for (; k + 2 * U <= n; k += U) {
-            double a2[U], b2[U];
+        };
+        double acc = yb[s * CB];
+        auto mul = [&](double* p, const double* a, const double* b) {
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-              a2[u] = l[k + U + u];
-              b2[u] = xb[(k + U + u) * CB];
-            }
+          for (int u = 0; u < U; u++) p[u] = a[u] * b[u];
+        };
+        auto sub = [&](const double* p) {
 #pragma unroll
-            for (int u = 0; u < U; u++) acc -= a[u] * b[u];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-              a[u] = a2[u];
-              b[u] = b2[u];
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < U; u++) acc -= a[u] * b[u];
-          k += U;
+          for (int u = 0; u < U; u++) acc -= p[u];
+        };
+        const double dii = l[0];
+        rd(a0, b0, 2);
+        rd(a1, b1, 2 + U);
+        acc -= l[1] * xl;  // i = n-1: l[1] is 0
+        mul(p0, a0, b0);
+        for (int k = 2; k < n - i; k += 2 * U) {
+          rd(a0, b0, k + 2 * U);
+          mul(p1, a1, b1);
+          sub(p0);
+          __builtin_amdgcn_sched_barrier(0);
+          rd(a1, b1, k + 3 * U);
+          mul(p0, a0, b0);
+          sub(p1);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        for (; k < n; k++) acc -= l[k] * xb[k * CB];
-        xl = acc / l[i];
+        xl = acc / dii;
         xs[i * CB + lane] = xl;
         if (c < n) out[(size_t)i * n + c] = singular ? xl - corr : xl;
       }
@@ -1796,11 +1805,13 @@ void launch_dense_pinv(const Lv& C, int singular, double* work, double* out, hip
     hipLaunchKernelGGL(k_pinv_panel, dim3((unsigned)ni, (unsigned)nj), dim3(256), 0, st, work, LT, n, c0);
   }
   // the columns per wave and the rows staged ahead that fit the LDS
-#define SMAC_PBACK(CB, G) \
-  hipLaunchKernelGGL((k_pinv_back<CB, G>), dim3((unsigned)((n + CB - 1) / CB)), dim3(256), 0, st, LT, cs, n, singular, out)
-  if (n <= 256) SMAC_PBACK(32, 16);
-  else if (n <= 512) SMAC_PBACK(16, 8);
-  else SMAC_PBACK(8, 4);
+#define SMAC_PBACK(CB, G, NM)                                                                                    \
+  hipLaunchKernelGGL((k_pinv_back<CB, G, NM>), dim3((unsigned)((n + CB - 1) / CB)), dim3(256), 0, st, LT, cs, n, \
+                     singular, out)
+  if (n <= 128) SMAC_PBACK(32, 16, 128);
+  else if (n <= 256) SMAC_PBACK(32, 8, 256);
+  else if (n <= 512) SMAC_PBACK(16, 8, 512);
+  else SMAC_PBACK(8, 4, 1024);
 #undef SMAC_PBACK
 }
 
