@@ -1093,6 +1093,18 @@ static void vcycle(smac_ctx* c, int l, int nu1, int nu2) {
     KT(c, "mg_coarse_solve", launch_mg_coarse<T>(V.lv, c->cinv, f, e, c->st));
     return;
   }
+  if (nu1 == 2 && nu2 == 2 && mg_tile_applies<T>(V.lv)) {
+    // small levels: one launch down and one up; tb holds e between the two
+    Level& C = c->lev[l + 1];
+    T* ep = (T*)V.tb;
+    const int rcp = mg_zs_division<T>(V.lv, e, f) == 2;
+    c->zs_done = false;
+    KT(c, fine ? "mg_down_l0" : "mg_coarse_levels", launch_mg_down<T>(V.lv, C.lv, f, ep, (T*)C.f, rcp, c->st));
+    vcycle<T>(c, l + 1, nu1, nu2);
+    KT(c, fine ? "mg_up_l0" : "mg_coarse_levels",
+       launch_mg_up<T>(C.lv, V.lv, (const T*)C.e, ep, f, e, rcp, c->st));
+    return;
+  }
   // the first red half sweep starts from e = 0 and writes every red cell; the
   // black half sweep that follows reads only red cells, so no fill is needed
   if (nu1 == 0) KT(c, fine ? "mg_fill_l0" : "mg_coarse_levels", launch_fill<T>(V.lv, e, c->st));
@@ -1424,7 +1436,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   const bool fuse = c->dv2 && dir_spmv_applies<T>(g, z, c->dv, c->dv2, c->dp, c->Ad);
   // the zero-start red half sweep of level 0 rides on the residual update
   // (uniform coefficients: pointwise f/diag)
-  const int zs_mode = (mg && !var && o.nu1 >= 1)
+  const int zs_mode = (mg && !var && o.nu1 >= 1 && !(o.nu1 == 2 && o.nu2 == 2 && mg_tile_applies<T>(c->lev[0].lv)))
                           ? mg_zs_division<T>(c->lev[0].lv, (const T*)c->lev[0].e, (const T*)c->lev[0].f)
                           : 0;
   c->zs_done = false;

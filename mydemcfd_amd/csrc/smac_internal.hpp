@@ -288,6 +288,18 @@ template <typename T>
 void launch_mg_coarse(const Lv& C, const double* ainv, const T* f, T* e, hipStream_t st);
 template <typename T>
 void launch_fill(const Lv& L, T* x, hipStream_t st);
+// a level's half of the V-cycle in one launch (smac_mgtile.hip), nu = 2, for a
+// level of up to MG_TILE_CELLS cells: down = the four half sweeps from zero (e
+// in ep), the residual and its restriction to fc; up = the prolongation of ec
+// onto ep and the four half sweeps, into e. rcp: the FP32 reciprocal in place
+// of the division (mg_zs_division(L) == 2)
+constexpr size_t MG_TILE_CELLS = (size_t)1 << 18;
+template <typename T>
+bool mg_tile_applies(const Lv& L);
+template <typename T>
+void launch_mg_down(const Lv& F, const Lv& C, const T* f, T* ep, T* fc, int rcp, hipStream_t st);
+template <typename T>
+void launch_mg_up(const Lv& C, const Lv& F, const T* ec, const T* ep, const T* f, T* e, int rcp, hipStream_t st);
 // coarse face coefficients of axis d on level C from level F (k_mg_coarsen_beta)
 void launch_mg_coarsen_beta(const Lv& F, const Lv& C, int d, double* cb, hipStream_t st);
 // dense (pseudo-)inverse of the coarsest level's operator into out (n x n,
