@@ -1441,11 +1441,17 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
                           : 0;
   c->zs_done = false;
   bool ad_ready = first_fused;
+  // small grids: two passes an iteration around the preconditioner, r.z
+  // alternating between two slots
+  const bool small = !stat && !fuse && c->dv2 && pcg_small_applies(g);
+  const bool jac = small && !mg && !refg;  // Jacobi and its dots ride on the residual update
+  int rz = S_RZ, rzn = S_RZN;
+  bool fresh = false;  // S_RR and S_LINF on the host are those of the last update
   for (iter = 0; iter < o.max_iter && !conv && !nan; ++iter) {
-    if (!ad_ready) KT(c, "spmv_dot", launch_spmv_dot(g, bfp, c->dv, c->Ad, P[0], s));
-    double* pap = ad_ready ? P[4] : P[0];
+    if (!ad_ready) KT(c, "spmv_dot", launch_spmv_dot(g, bfp, c->dv, c->Ad, small ? P[4] : P[0], s));
+    double* pap = ad_ready || small ? P[4] : P[0];
     ad_ready = false;
-    if (!stat) {
+    if (!stat && !small) {
       FinalizeArgs fa = fin(c);
       fin_add(fa, pap, 0, S_PAP);
       fa.op = OP_DIV;
@@ -1454,7 +1460,10 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
       fa.sb = S_PAP;
       launch_finalize(fa, c->S, s);
     }
-    if (zs_mode)
+    fresh = false;
+    if (small)
+      KT(c, "update", launch_pcg_res<T>(g, bfp, jac, pap, c->S, rz, c->r, c->Ad, f0, c->z, o.flexible, P, s));
+    else if (zs_mode)
       KT(c, "update_zs",
          c->zs_done = launch_update<T>(g, c->r, c->Ad, c->S, S_ALPHA, P[0], P[1], f0, s, z, zs_mode, &c->lev[0].lv));
     else
@@ -1477,12 +1486,13 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     c->dot_flex = o.flexible;
     c->dot_p0 = P[2];
     c->dot_p1 = P[3];
-    precond();
+    if (!jac) precond();
     c->dot_req = false;
-    if (!stat && !c->dot_done) KT(c, "dot2", launch_dot2<T>(g, c->r, z, c->Ad, o.flexible, P[2], P[3], s));
+    if (!stat && !c->dot_done && !jac)
+      KT(c, "dot2", launch_dot2<T>(g, c->r, z, c->Ad, o.flexible, P[2], P[3], s));
     bool check = (iter % o.check_every) == 0;
     {
-      if (!stat) {
+      if (!stat && !small) {
         FinalizeArgs fa = fin(c);
         fin_add(fa, P[2], 0, S_RZN);
         if (o.flexible) fin_add(fa, P[3], 0, S_ZAD);
@@ -1493,8 +1503,9 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
         fin_add(fb, P[0], 0, S_RR);
         fin_add(fb, P[1], 1, S_LINF);
       }
-      if (stat) {
-        // no scalar operation: alpha and beta stay 1 and 0
+      if (stat || small) {
+        // no scalar operation: alpha and beta stay 1 and 0, or are formed by
+        // the pass that uses them
       } else if (o.flexible) {
         fb.op = OP_BETA_PR;
         fb.dst = S_BETA;
@@ -1513,6 +1524,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
       HIPOK(hipGetLastError());
       rc = read_scalars(c);
       if (rc) return rc;
+      fresh = true;
       if (!std::isfinite(c->Sh[S_RR]) || !std::isfinite(c->Sh[S_LINF])) {
         iter++;
         nan = true;
@@ -1534,6 +1546,18 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
         }
       }
     }
+    if (small && iter + 1 < o.max_iter) {
+      KT(c, "dir_spmv", launch_pcg_dir<T>(g, bfp, P[2], P[3], o.flexible, c->S, rz, rzn, z, c->dv, c->dv2, c->dp, c->Ad,
+                                          P[4], s));
+      std::swap(c->dv, c->dv2);
+      std::swap(rz, rzn);
+      ad_ready = true;
+      dp_pending = false;
+      continue;
+    }
+    // (small grids, the last iteration: no direction is needed any more, and
+    // the flush below adds its alpha d)
+    if (small) continue;
     if (fuse && iter + 1 < o.max_iter) {
       KT(c, "dir_spmv", launch_dir_spmv<T>(g, bfp, z, c->dv, c->dv2, c->dp, c->Ad, P[4], c->S, S_ALPHA, S_BETA, s));
       std::swap(c->dv, c->dv2);
@@ -1558,12 +1582,14 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     st->mg_levels = (mg || refg) ? L : 0;
     st->bnorm = bnorm;
     if (have_update) {
-      FinalizeArgs fa = fin(c);
-      fin_add(fa, P[0], 0, S_RR);
-      fin_add(fa, P[1], 1, S_LINF);
-      launch_finalize(fa, c->S, s);
-      rc = read_scalars(c);
-      if (rc) return rc;
+      if (!fresh) {  // the last update was not checked
+        FinalizeArgs fa = fin(c);
+        fin_add(fa, P[0], 0, S_RR);
+        fin_add(fa, P[1], 1, S_LINF);
+        launch_finalize(fa, c->S, s);
+        rc = read_scalars(c);
+        if (rc) return rc;
+      }
       rr = c->Sh[S_RR];
       st->linf_res_dt = c->Sh[S_LINF] * dt;
     } else {

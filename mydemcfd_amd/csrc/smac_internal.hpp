@@ -212,6 +212,21 @@ void launch_dot2(const Geo& g, const double* r, const Z* z, const double* Ad, in
 template <typename Z>
 void launch_xpay(const Geo& g, const Z* z, double* d, double* dp, const double* S, int slot_alpha, int slot_beta,
                  hipStream_t st);
+// the PCG iteration on small grids, where launches bound it: the direction
+// update with its SpMV, and the residual update (Jacobi: with the
+// preconditioner and its dots), each forming the scalars it needs from the row
+// partials. p_rz, p_zad: partials of r.z, z.Ad; p_pap: of d.Ad; slots rz_in,
+// rz_out of S: r.z of this and of the next iteration. launch_pcg_res: P[0..3]
+// <- |r|^2, max |r|, r.z, z.Ad (the last two with Jacobi)
+constexpr size_t PCG_SMALL_ROWS = 8192, PCG_SMALL_CELLS = (size_t)1 << 19;
+bool pcg_small_applies(const Geo& g);
+template <typename Z>
+void launch_pcg_dir(const Geo& g, const BetaF* bf, const double* p_rz, const double* p_zad, int flexible, double* S,
+                    int rz_in, int rz_out, const Z* z, const double* dold, double* dnew, double* dp, double* Ad,
+                    double* part, hipStream_t st);
+template <typename F>
+void launch_pcg_res(const Geo& g, const BetaF* bf, int jacobi, const double* p_pap, double* S, int rz_in, double* r,
+                    const double* Ad, F* f0, double* z, int flexible, double* const P[4], hipStream_t st);
 void launch_finalize(const FinalizeArgs& fa, double* S, hipStream_t st);
 void launch_scalar_copy(double* S, int dst, int src, hipStream_t st);
 void launch_scalar_set(double* S, int dst, double v, hipStream_t st);

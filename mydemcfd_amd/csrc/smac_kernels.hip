@@ -8,6 +8,8 @@
 //   Poisson RHS      k_rhs, k_rhs_eps  b = -(1/dt) div u* (+ the volume-fraction form)
 //   PCG vectors      k_init_r, k_add_scalar, k_jacobi, k_copy_dot, k_sum,
 //                    k_spmv_dot, k_update, k_dot2, k_xpay, k_dp_flush
+//                    k_pcg_dir, k_pcg_res   the iteration's passes on small
+//                                      grids, scalars formed in each block
 //   reductions       k_finalize        canonical 1024-lane tree + scalar ops
 //   (multigrid kernels: smac_mg.hip)
 //   correction       k_correct_all, k_zero_dp
@@ -1470,6 +1472,162 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs fa, double* __re
   }
 }
 
+// ------------------------------------------------- PCG iteration, small grids
+// Up to PCG_SMALL_ROWS rows an iteration's launches cost more than its work:
+// with Jacobi nine kernels of 1.7 to 5.5 us each on 64^3, three of them
+// reductions of a few thousand row partials in one block. Here every block of
+// the two kernels that need a scalar forms it for itself from the row partials
+// (32 KB at most 256 times from the L2), in the canonical order, so an
+// iteration is k_pcg_dir and k_pcg_res, with the V-cycle and its dots between
+// them when there is one. Block 0 leaves the scalars in S for the next kernel;
+// r.z alternates between two slots, since its old value is read by every block
+// that may still be running.
+//
+// The canonical sums of up to two row-partial arrays, in every thread: 256
+// threads take the lanes t, t+256, t+512, t+768 of the 1024-lane tree (its
+// first two steps are theirs), and every wave finishes it from LDS.
+template <int CNT>
+__device__ __forceinline__ void block_sums(const double* const (&part)[CNT], int nrows, double (&out)[CNT]) {
+  __shared__ double lds[CNT][256];
+  const int t = (int)threadIdx.x, lane = t & 63;
+  if (t < 256) {
+#pragma unroll
+    for (int m = 0; m < CNT; m++) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[u] = fin_lane<4>(part[m], 0, nrows, t + 256 * u);
+      lds[m][t] = (v[0] + v[2]) + (v[1] + v[3]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < CNT; m++) {
+    const double v = (lds[m][lane] + lds[m][lane + 128]) + (lds[m][lane + 64] + lds[m][lane + 192]);
+    out[m] = __shfl(wave_tree_sum(v), 0, 64);
+  }
+}
+
+// row of this wave (canonical row index and j, k), NT / 64 rows a block
+#define SMALL_ROW(NT)                                                                        \
+  const int lane = (int)threadIdx.x & 63;                                                    \
+  const int vrow_ = xcd_block((int)blockIdx.x, (int)gridDim.x) * ((NT) / 64) + ((int)threadIdx.x >> 6); \
+  if (vrow_ >= g.n[1] * g.n[2]) return;                                                      \
+  int j, k;                                                                                  \
+  band_jk(vrow_, g.n[1], g.n[2], j, k);                                                      \
+  const int row = (k - 1) * g.n[1] + (j - 1);                                                \
+  const size_t rb = ((size_t)k * (size_t)g.py + (size_t)j) * (size_t)g.px;
+
+// beta from the partials of r.z (and z.Ad, flexible), d = z + beta d_old,
+// dp += alpha d_old, Ad = A d, part <- d.Ad (k_finalize's OP_DIV / OP_BETA_PR,
+// k_xpay and k_spmv_dot)
+template <bool VAR, typename Z, int NT>
+__global__ __launch_bounds__(NT) void k_pcg_dir(Geo g, BetaF bf, const double* __restrict__ p_rz,
+                                                const double* __restrict__ p_zad, int flexible, double* __restrict__ S,
+                                                int rz_in, int rz_out, const Z* __restrict__ z,
+                                                const double* __restrict__ dold, double* __restrict__ dnew,
+                                                double* __restrict__ dp, double* __restrict__ Ad,
+                                                double* __restrict__ part) {
+  const int nrows = g.n[1] * g.n[2];
+  const double* const pp[2] = {p_rz, flexible ? p_zad : p_rz};
+  double sums[2];
+  block_sums<2>(pp, nrows, sums);
+  const double alpha = S[S_ALPHA], rz = S[rz_in];
+  const double beta = flexible ? (-alpha * sums[1]) / rz : sums[0] / rz;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[rz_out] = sums[0];
+    S[S_BETA] = beta;
+  }
+  SMALL_ROW(NT)
+  const int nx = g.n[0], nh = nx >> 1;
+  const size_t ypr = idx(g, 0, W(g, 1, j + 1), k), ymr = idx(g, 0, W(g, 1, j - 1), k);
+  const size_t zpr = idx(g, 0, j, W(g, 2, k + 1)), zmr = idx(g, 0, j, W(g, 2, k - 1));
+  auto dv = [&](size_t o) { return (double)St<Z>::ld(z, o) + beta * dold[o]; };
+  double acc = 0.0;
+  for (int q0 = 1 + 2 * lane; q0 <= nx; q0 += 128) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int q = q0 + t;
+      if (q > nx) continue;
+      const int i = q <= nh ? 2 * q : 2 * (q - nh) - 1;
+      const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k);
+      const double od = dold[rb + q];
+      const double xc = (double)St<Z>::ld(z, rb + q) + beta * od;
+      const double xp = dv(rb + spos(W(g, 0, i + 1), nx)), xm = dv(rb + spos(W(g, 0, i - 1), nx));
+      const double yp = dv(ypr + q), ym = dv(ymr + q), zp = dv(zpr + q), zm = dv(zmr + q);
+      const double s = c.a[0] * xp + c.a[1] * xm + c.a[2] * yp + c.a[3] * ym + c.a[4] * zp + c.a[5] * zm;
+      const double v = c.diag * xc - s;
+      dp[rb + i] = dp[rb + i] + alpha * od;
+      dnew[rb + q] = xc;
+      Ad[rb + q] = v;
+      acc += xc * v;
+    }
+  }
+  acc = wave_tree_sum(acc);
+  if (lane == 0) part[row] = acc;
+}
+
+// alpha from the partials of d.Ad, r -= alpha Ad with |r|^2 and max |r|, f0 =
+// (F) r; JAC: also z = r / diag with the partials of r.z and z.Ad (k_finalize's
+// OP_DIV, k_update, k_jacobi and k_dot2)
+template <bool VAR, bool JAC, typename F, int NT>
+__global__ __launch_bounds__(NT) void k_pcg_res(Geo g, BetaF bf, const double* __restrict__ p_pap,
+                                                double* __restrict__ S, int rz_in, double* __restrict__ r,
+                                                const double* __restrict__ Ad, F* __restrict__ f0,
+                                                double* __restrict__ z, int flexible, double* __restrict__ part0,
+                                                double* __restrict__ part1, double* __restrict__ part2,
+                                                double* __restrict__ part3) {
+  const int nrows = g.n[1] * g.n[2];
+  const double* const pp[1] = {p_pap};
+  double sums[1];
+  block_sums<1>(pp, nrows, sums);
+  const double alpha = S[rz_in] / sums[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S[S_PAP] = sums[0];
+    S[S_ALPHA] = alpha;
+  }
+  SMALL_ROW(NT)
+  const int nx = g.n[0], nh = nx >> 1;
+  double a0 = 0.0, mx = 0.0, a2 = 0.0, a3 = 0.0;
+  for (int q0 = 1 + 2 * lane; q0 <= nx; q0 += 128) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int q = q0 + t;
+      if (q > nx) continue;
+      const size_t o = rb + q;
+      const double ad = Ad[o];
+      const double rn = r[o] - alpha * ad;
+      r[o] = rn;
+      a0 += rn * rn;
+      const double ar = fabs(rn);
+      if (ar > mx || ar != ar) mx = ar;
+      if constexpr (JAC) {
+        const int i = q <= nh ? 2 * q : 2 * (q - nh) - 1;
+        const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k);
+        const double zz = (1. / c.diag) * rn;
+        z[o] = zz;
+        a2 += rn * zz;
+        if (flexible) a3 += zz * ad;
+      } else if (f0) {
+        St<F>::st(f0, o, (typename St<F>::C)rn);
+      }
+    }
+  }
+  a0 = wave_tree_sum(a0);
+  mx = wave_max(mx);
+  if (JAC) {
+    a2 = wave_tree_sum(a2);
+    if (flexible) a3 = wave_tree_sum(a3);
+  }
+  if (lane == 0) {
+    part0[row] = a0;
+    part1[row] = mx;
+    if (JAC) {
+      part2[row] = a2;
+      if (flexible) part3[row] = a3;
+    }
+  }
+}
+
 // S[dst] = S[src] (e.g. rz <- rz_new)
 __global__ void k_scalar_copy(double* S, int dst, int src) { S[dst] = S[src]; }
 __global__ void k_scalar_set(double* S, int dst, double v) { S[dst] = v; }
@@ -1965,6 +2123,58 @@ void launch_finalize(const FinalizeArgs& fa, double* S, hipStream_t st) {
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, st, f1, S);
   }
 }
+// 16 rows a block where there are rows enough for every CU, 4 below
+static inline int small_nt(const Geo& g) { return g.n[1] * g.n[2] > 1024 ? 1024 : 256; }
+static inline dim3 small_grid(const Geo& g, int nt) {
+  return dim3((unsigned)((g.n[1] * g.n[2] + nt / 64 - 1) / (nt / 64)));
+}
+bool pcg_small_applies(const Geo& g) {
+  const size_t rows = (size_t)g.n[1] * (size_t)g.n[2];
+  return rows <= PCG_SMALL_ROWS && rows * (size_t)g.n[0] <= PCG_SMALL_CELLS;
+}
+template <typename Z>
+void launch_pcg_dir(const Geo& g, const BetaF* bf, const double* p_rz, const double* p_zad, int flexible, double* S,
+                    int rz_in, int rz_out, const Z* z, const double* dold, double* dnew, double* dp, double* Ad,
+                    double* part, hipStream_t st) {
+  const int nt = small_nt(g);
+#define SMAC_PD(V, N)                                                                                              \
+  hipLaunchKernelGGL((k_pcg_dir<V, Z, N>), small_grid(g, N), dim3(N), 0, st, g, bf ? *bf : BetaF{}, p_rz, p_zad, \
+                     flexible, S, rz_in, rz_out, z, dold, dnew, dp, Ad, part)
+  if (bf) {
+    if (nt == 256) SMAC_PD(true, 256);
+    else SMAC_PD(true, 1024);
+  } else {
+    if (nt == 256) SMAC_PD(false, 256);
+    else SMAC_PD(false, 1024);
+  }
+#undef SMAC_PD
+}
+template <typename F>
+void launch_pcg_res(const Geo& g, const BetaF* bf, int jacobi, const double* p_pap, double* S, int rz_in, double* r,
+                    const double* Ad, F* f0, double* z, int flexible, double* const P[4], hipStream_t st) {
+  const int nt = small_nt(g);
+#define SMAC_PR(V, J, N)                                                                                         \
+  hipLaunchKernelGGL((k_pcg_res<V, J, F, N>), small_grid(g, N), dim3(N), 0, st, g, bf ? *bf : BetaF{}, p_pap, S, \
+                     rz_in, r, Ad, f0, z, flexible, P[0], P[1], P[2], P[3])
+#define SMAC_PR_N(V, J)             \
+  do {                              \
+    if (nt == 256) SMAC_PR(V, J, 256); \
+    else SMAC_PR(V, J, 1024);       \
+  } while (0)
+  if (!jacobi) SMAC_PR_N(false, false);
+  else if (bf) SMAC_PR_N(true, true);
+  else SMAC_PR_N(false, true);
+#undef SMAC_PR_N
+#undef SMAC_PR
+}
+#define SMAC_INST_PCG(Z)                                                                                          \
+  template void launch_pcg_dir<Z>(const Geo&, const BetaF*, const double*, const double*, int, double*, int, int,  \
+                                  const Z*, const double*, double*, double*, double*, double*, hipStream_t);       \
+  template void launch_pcg_res<Z>(const Geo&, const BetaF*, int, const double*, double*, int, double*, const double*, \
+                                  Z*, double*, int, double* const[4], hipStream_t);
+SMAC_INST_PCG(double)
+SMAC_INST_PCG(float)
+SMAC_INST_PCG(bf16s)
 void launch_scalar_copy(double* S, int dst, int src, hipStream_t st) {
   hipLaunchKernelGGL(k_scalar_copy, dim3(1), dim3(1), 0, st, S, dst, src);
 }
