@@ -404,20 +404,48 @@ struct Vec<bf16s, N> {
   }
 };
 
+// the value of lane l + s in lane l, s = 32, 16 (the halves and rows of 16
+// swapped by the permlane instructions) or 8, 4, 2, 1 (inside a row, DPP row
+// shift), valid in the lanes below s -- all the halving tree reads; register
+// moves, where __shfl_down goes through the LDS pipe (a tree of six steps is
+// some 400 cycles shorter). All 64 lanes must be active.
+template <int S>
+__device__ __forceinline__ unsigned lane_down32(unsigned v) {
+  if constexpr (S == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  else if constexpr (S == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  else return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + S, 0xf, 0xf, true);
+}
+template <int S>
+__device__ __forceinline__ double lane_down(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = lane_down32<S>((unsigned)b), hi = lane_down32<S>((unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
 // Canonical wave64 halving tree: lane l += lane l+s, s = 32..1; lane 0 holds
 // the result. Identical association to the CPU oracle's tree().
 __device__ __forceinline__ double wave_tree_sum(double v) {
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) v = v + __shfl_down(v, s, 64);
-  return v;
+  v = v + lane_down<32>(v);
+  v = v + lane_down<16>(v);
+  v = v + lane_down<8>(v);
+  v = v + lane_down<4>(v);
+  v = v + lane_down<2>(v);
+  return v + lane_down<1>(v);
 }
+__device__ __forceinline__ double max_step(double v, double o) { return o > v || o != o ? o : v; }
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) {
-    double o = __shfl_down(v, s, 64);
-    if (o > v || o != o) v = o;
-  }
-  return v;
+  v = max_step(v, lane_down<32>(v));
+  v = max_step(v, lane_down<16>(v));
+  v = max_step(v, lane_down<8>(v));
+  v = max_step(v, lane_down<4>(v));
+  v = max_step(v, lane_down<2>(v));
+  return max_step(v, lane_down<1>(v));
+}
+// the value of lane `lane` (the same for the whole wave)
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
 }  // namespace smac

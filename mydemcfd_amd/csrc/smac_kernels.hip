@@ -1483,39 +1483,117 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs fa, double* __re
 // r.z alternates between two slots, since its old value is read by every block
 // that may still be running.
 //
-// The canonical sums of up to two row-partial arrays, in every thread: 256
-// threads take the lanes t, t+256, t+512, t+768 of the 1024-lane tree (its
-// first two steps are theirs), and every wave finishes it from LDS.
-template <int CNT>
-__device__ __forceinline__ void block_sums(const double* const (&part)[CNT], int nrows, double (&out)[CNT]) {
-  __shared__ double lds[CNT][256];
+// The canonical sums of up to two row-partial arrays (the second only when
+// `both`), in every thread: the block's threads form the 1024 lane sums, every
+// wave finishes the tree from LDS.
+template <int CNT, int NT>
+__device__ __forceinline__ void block_sums(const double* const (&part)[CNT], bool both, int nrows,
+                                           double (&out)[CNT]) {
+  __shared__ double lds[CNT][1024];
   const int t = (int)threadIdx.x, lane = t & 63;
-  if (t < 256) {
+  constexpr int LT = 1024 / NT, B = 4;  // lanes per thread, rows per lane in flight
+  double acc[CNT][LT];
 #pragma unroll
-    for (int m = 0; m < CNT; m++) {
-      double v[4];
+  for (int m = 0; m < CNT; m++)
 #pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = fin_lane<4>(part[m], 0, nrows, t + 256 * u);
-      lds[m][t] = (v[0] + v[2]) + (v[1] + v[3]);
-    }
+    for (int u = 0; u < LT; u++) acc[m][u] = 0.0;
+  for (int r0 = t; r0 < nrows; r0 += 1024 * B) {
+    double v[CNT][LT][B];
+#pragma unroll
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < LT; u++)
+#pragma unroll
+        for (int q = 0; q < B; q++) {
+          const int r = r0 + NT * u + 1024 * q;
+          v[m][u][q] = r < nrows && (m == 0 || both) ? part[m][r] : 0.0;
+        }
+#pragma unroll
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < LT; u++)
+#pragma unroll
+        for (int q = 0; q < B; q++)
+          if (r0 + NT * u + 1024 * q < nrows) acc[m][u] += v[m][u][q];
   }
+#pragma unroll
+  for (int m = 0; m < CNT; m++)
+#pragma unroll
+    for (int u = 0; u < LT; u++) lds[m][t + NT * u] = acc[m][u];
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < CNT; m++) {
-    const double v = (lds[m][lane] + lds[m][lane + 128]) + (lds[m][lane + 64] + lds[m][lane + 192]);
-    out[m] = __shfl(wave_tree_sum(v), 0, 64);
+    if (m > 0 && !both) {
+      out[m] = 0.0;
+      continue;
+    }
+    double x[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) x[u] = lds[m][lane + 64 * u];
+#pragma unroll
+    for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+      for (int u = 0; u < h; u++) x[u] = x[u] + x[u + h];
+    out[m] = lane_value(wave_tree_sum(x[0]), 0);
   }
 }
 
 // row of this wave (canonical row index and j, k), NT / 64 rows a block
 #define SMALL_ROW(NT)                                                                        \
   const int lane = (int)threadIdx.x & 63;                                                    \
-  const int vrow_ = xcd_block((int)blockIdx.x, (int)gridDim.x) * ((NT) / 64) + ((int)threadIdx.x >> 6); \
+  const int vrow_ = xcd_block((int)blockIdx.x, (int)gridDim.x) * ((NT) / 64) +               \
+                    __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);                   \
   if (vrow_ >= g.n[1] * g.n[2]) return;                                                      \
   int j, k;                                                                                  \
   band_jk(vrow_, g.n[1], g.n[2], j, k);                                                      \
   const int row = (k - 1) * g.n[1] + (j - 1);                                                \
   const size_t rb = ((size_t)k * (size_t)g.py + (size_t)j) * (size_t)g.px;
+
+// The lanes take the cells of a 128-position chunk one by one (lane l the
+// positions l and 64 + l), so that rows of up to 64 cells keep every lane busy;
+// pair_add then adds a product per cell to the lane sums in pair order: lane l
+// the values of positions 2l and 2l + 1 (zero past the row's end).
+__device__ __forceinline__ double pair_add(double acc, const double p[2], bool upper, int lane) {
+  const int src = (2 * lane) & 63;
+  double v0 = __shfl(p[0], src), v1 = __shfl(p[0], src + 1);
+  if (upper) {
+    const double w0 = __shfl(p[1], src), w1 = __shfl(p[1], src + 1);
+    v0 = lane < 32 ? v0 : w0;
+    v1 = lane < 32 ? v1 : w1;
+  } else {
+    v0 = lane < 32 ? v0 : 0.0;
+    v1 = lane < 32 ? v1 : 0.0;
+  }
+  acc += v0;
+  acc += v1;
+  return acc;
+}
+// coefficients of cell i of the row (coef_uniform)
+struct RowCoef {
+  double a0, ay[4];
+  bool perx;
+  int nx;
+  __device__ __forceinline__ RowCoef(const Geo& g, int j, int k) {
+    a0 = g.beta0 * g.inv_d2[0];
+    ay[0] = wall_face(g.per[1], j + 1, g.n[1]) ? 0.0 : g.beta0 * g.inv_d2[1];
+    ay[1] = wall_face(g.per[1], j, g.n[1]) ? 0.0 : g.beta0 * g.inv_d2[1];
+    ay[2] = wall_face(g.per[2], k + 1, g.n[2]) ? 0.0 : g.beta0 * g.inv_d2[2];
+    ay[3] = wall_face(g.per[2], k, g.n[2]) ? 0.0 : g.beta0 * g.inv_d2[2];
+    perx = g.per[0] != 0;
+    nx = g.n[0];
+  }
+  __device__ __forceinline__ Coef at(int i) const {
+    Coef c;
+    c.a[0] = !perx && i == nx ? 0.0 : a0;
+    c.a[1] = !perx && i == 1 ? 0.0 : a0;
+    c.a[2] = ay[0];
+    c.a[3] = ay[1];
+    c.a[4] = ay[2];
+    c.a[5] = ay[3];
+    c.diag = c.a[0] + c.a[1] + c.a[2] + c.a[3] + c.a[4] + c.a[5];
+    return c;
+  }
+};
 
 // beta from the partials of r.z (and z.Ad, flexible), d = z + beta d_old,
 // dp += alpha d_old, Ad = A d, part <- d.Ad (k_finalize's OP_DIV / OP_BETA_PR,
@@ -1528,10 +1606,10 @@ __global__ __launch_bounds__(NT) void k_pcg_dir(Geo g, BetaF bf, const double* _
                                                 double* __restrict__ dp, double* __restrict__ Ad,
                                                 double* __restrict__ part) {
   const int nrows = g.n[1] * g.n[2];
-  const double* const pp[2] = {p_rz, flexible ? p_zad : p_rz};
+  const double* const pp[2] = {p_rz, p_zad};
   double sums[2];
-  block_sums<2>(pp, nrows, sums);
   const double alpha = S[S_ALPHA], rz = S[rz_in];
+  block_sums<2, NT>(pp, flexible != 0, nrows, sums);
   const double beta = flexible ? (-alpha * sums[1]) / rz : sums[0] / rz;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S[rz_out] = sums[0];
@@ -1541,26 +1619,31 @@ __global__ __launch_bounds__(NT) void k_pcg_dir(Geo g, BetaF bf, const double* _
   const int nx = g.n[0], nh = nx >> 1;
   const size_t ypr = idx(g, 0, W(g, 1, j + 1), k), ymr = idx(g, 0, W(g, 1, j - 1), k);
   const size_t zpr = idx(g, 0, j, W(g, 2, k + 1)), zmr = idx(g, 0, j, W(g, 2, k - 1));
-  auto dv = [&](size_t o) { return (double)St<Z>::ld(z, o) + beta * dold[o]; };
+  const RowCoef rc(g, j, k);
+  auto dv = [&](size_t base, unsigned q) { return (double)St<Z>::ld(z + base, q) + beta * dold[base + q]; };
   double acc = 0.0;
-  for (int q0 = 1 + 2 * lane; q0 <= nx; q0 += 128) {
+  for (int c0 = 0; c0 < nx; c0 += 128) {
+    const bool upper = c0 + 64 < nx;
+    double p[2] = {0.0, 0.0};
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int q = q0 + t;
-      if (q > nx) continue;
+    for (int m = 0; m < 2; m++) {
+      const int q = c0 + 64 * m + lane + 1;
+      if ((m == 1 && !upper) || q > nx) continue;
       const int i = q <= nh ? 2 * q : 2 * (q - nh) - 1;
-      const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k);
-      const double od = dold[rb + q];
-      const double xc = (double)St<Z>::ld(z, rb + q) + beta * od;
-      const double xp = dv(rb + spos(W(g, 0, i + 1), nx)), xm = dv(rb + spos(W(g, 0, i - 1), nx));
-      const double yp = dv(ypr + q), ym = dv(ymr + q), zp = dv(zpr + q), zm = dv(zmr + q);
+      const unsigned u = (unsigned)q;
+      const double od = dold[rb + u];
+      const double xc = (double)St<Z>::ld(z + rb, u) + beta * od;
+      const double xp = dv(rb, (unsigned)spos(W(g, 0, i + 1), nx)), xm = dv(rb, (unsigned)spos(W(g, 0, i - 1), nx));
+      const double yp = dv(ypr, u), ym = dv(ymr, u), zp = dv(zpr, u), zm = dv(zmr, u);
+      const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : rc.at(i);
       const double s = c.a[0] * xp + c.a[1] * xm + c.a[2] * yp + c.a[3] * ym + c.a[4] * zp + c.a[5] * zm;
       const double v = c.diag * xc - s;
-      dp[rb + i] = dp[rb + i] + alpha * od;
-      dnew[rb + q] = xc;
-      Ad[rb + q] = v;
-      acc += xc * v;
+      dp[rb + (unsigned)i] = dp[rb + (unsigned)i] + alpha * od;
+      dnew[rb + u] = xc;
+      Ad[rb + u] = v;
+      p[m] = xc * v;
     }
+    acc = pair_add(acc, p, upper, lane);
   }
   acc = wave_tree_sum(acc);
   if (lane == 0) part[row] = acc;
@@ -1579,37 +1662,46 @@ __global__ __launch_bounds__(NT) void k_pcg_res(Geo g, BetaF bf, const double* _
   const int nrows = g.n[1] * g.n[2];
   const double* const pp[1] = {p_pap};
   double sums[1];
-  block_sums<1>(pp, nrows, sums);
-  const double alpha = S[rz_in] / sums[0];
+  const double rz = S[rz_in];
+  block_sums<1, NT>(pp, false, nrows, sums);
+  const double alpha = rz / sums[0];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S[S_PAP] = sums[0];
     S[S_ALPHA] = alpha;
   }
   SMALL_ROW(NT)
   const int nx = g.n[0], nh = nx >> 1;
+  const RowCoef rc(g, j, k);
   double a0 = 0.0, mx = 0.0, a2 = 0.0, a3 = 0.0;
-  for (int q0 = 1 + 2 * lane; q0 <= nx; q0 += 128) {
+  for (int c0 = 0; c0 < nx; c0 += 128) {
+    const bool upper = c0 + 64 < nx;
+    double p0[2] = {0.0, 0.0}, p2[2] = {0.0, 0.0}, p3[2] = {0.0, 0.0};
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-      const int q = q0 + t;
-      if (q > nx) continue;
-      const size_t o = rb + q;
-      const double ad = Ad[o];
-      const double rn = r[o] - alpha * ad;
-      r[o] = rn;
-      a0 += rn * rn;
+    for (int m = 0; m < 2; m++) {
+      const int q = c0 + 64 * m + lane + 1;
+      if ((m == 1 && !upper) || q > nx) continue;
+      const unsigned u = (unsigned)q;
+      const double ad = Ad[rb + u];
+      const double rn = r[rb + u] - alpha * ad;
+      r[rb + u] = rn;
+      p0[m] = rn * rn;
       const double ar = fabs(rn);
       if (ar > mx || ar != ar) mx = ar;
       if constexpr (JAC) {
         const int i = q <= nh ? 2 * q : 2 * (q - nh) - 1;
-        const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k);
+        const Coef c = VAR ? coef_var(g, bf.b, i, j, k) : rc.at(i);
         const double zz = (1. / c.diag) * rn;
-        z[o] = zz;
-        a2 += rn * zz;
-        if (flexible) a3 += zz * ad;
+        z[rb + u] = zz;
+        p2[m] = rn * zz;
+        if (flexible) p3[m] = zz * ad;
       } else if (f0) {
-        St<F>::st(f0, o, (typename St<F>::C)rn);
+        St<F>::st(f0 + rb, u, (typename St<F>::C)rn);
       }
+    }
+    a0 = pair_add(a0, p0, upper, lane);
+    if (JAC) {
+      a2 = pair_add(a2, p2, upper, lane);
+      if (flexible) a3 = pair_add(a3, p3, upper, lane);
     }
   }
   a0 = wave_tree_sum(a0);

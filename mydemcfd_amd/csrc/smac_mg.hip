@@ -1619,13 +1619,6 @@ __global__ __launch_bounds__(128) void k_pinv_assemble(Lv L, int singular, doubl
   for (int e = t; e < n; e += 128) m[e] = singular ? a[e] + c : a[e];
 }
 
-__device__ __forceinline__ double rdlane(double v, int lane) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
 // Panel c0 .. c0+31: block (I, J) owns the trailing tile of rows
 // c1 + 32 I .., columns c1 + 32 J .. (c1 = min(c0 + 32, n)). The J = 0 blocks write
 // their rows of the panel's factor, and block (0, 0) the diagonal block, to
@@ -1651,11 +1644,11 @@ __global__ __launch_bounds__(256) void k_pinv_panel(double* __restrict__ M, doub
       v[c] = ok && c0 + c < n ? M[(size_t)row * n + c0 + c] : (dia && c == l32 ? 1.0 : 0.0);
 #pragma unroll
     for (int jc = 0; jc < PB; jc++) {
-      const double d = sqrt(rdlane(v[jc], jc));
+      const double d = sqrt(lane_value(v[jc], jc));
       const double q = v[jc] / d;
       v[jc] = lane == jc ? d : q;
 #pragma unroll
-      for (int c = jc + 1; c < PB; c++) v[c] -= v[jc] * rdlane(v[jc], c);
+      for (int c = jc + 1; c < PB; c++) v[c] -= v[jc] * lane_value(v[jc], c);
     }
     if (!dia) {
 #pragma unroll
