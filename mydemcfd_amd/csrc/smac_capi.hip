@@ -96,7 +96,10 @@ struct smac_ctx {
   double* part[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   int nrows = 0;
   double* S = nullptr;
+  // pinned host copy of the scalars that reductions publish, and behind it the
+  // number of the last publication (waited for by wait_scalars)
   double* Sh = nullptr;
+  uint64_t seq = 0;
   double* fstage = nullptr;  // 3*1024 lane sums of the two-stage reductions
   std::vector<Level> lev;
   double* cinv = nullptr;
@@ -475,7 +478,8 @@ extern "C" int smac_create(const smac_grid_desc* gd, const smac_fluid_desc* fl, 
   for (int m = 0; m < 5 && rc == SMAC_OK; m++) rc = dalloc(&c->part[m], (size_t)c->nrows);
   if (rc == SMAC_OK) rc = dalloc(&c->S, S_COUNT);
   if (rc == SMAC_OK) rc = dalloc(&c->fstage, 3 * 1024);
-  if (rc == SMAC_OK && hipHostMalloc((void**)&c->Sh, S_COUNT * sizeof(double)) != hipSuccess) rc = SMAC_ERR_OOM;
+  if (rc == SMAC_OK && hipHostMalloc((void**)&c->Sh, (S_COUNT + 1) * sizeof(double)) != hipSuccess) rc = SMAC_ERR_OOM;
+  if (rc == SMAC_OK) memset(c->Sh, 0, (S_COUNT + 1) * sizeof(double));
   if (rc == SMAC_OK) {
     c->ev_ok = true;
     for (int e = 0; e < 8; e++)
@@ -1284,10 +1288,32 @@ static void fin_add(FinalizeArgs& fa, const double* part, int kind, int out) {
   fa.out[fa.count] = out;
   fa.count++;
 }
-static int read_scalars(smac_ctx* c) {
-  HIPOK(hipMemcpyAsync(c->Sh, c->S, S_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->st));
-  HIPOK(hipStreamSynchronize(c->st));
-  return SMAC_OK;
+// The reduction fa also leaves its results in c->Sh: the host reads them after
+// wait_scalars, which waits for this kernel alone, not for what is queued
+// behind it.
+static void fin_publish(smac_ctx* c, FinalizeArgs& fa) {
+  fa.host = c->Sh;
+  fa.seq = ++c->seq;
+}
+// Wait for the last published reduction. The stream is asked now and then, so
+// that an error on it, or its end without the number, ends the wait.
+static int wait_scalars(smac_ctx* c) {
+  const uint64_t* f = reinterpret_cast<const uint64_t*>(c->Sh + S_COUNT);
+  for (unsigned n = 1;; n++) {
+    if (__atomic_load_n(f, __ATOMIC_ACQUIRE) == c->seq) return SMAC_OK;
+    if ((n & 0x3fffu) == 0) {
+      const hipError_t e = hipStreamQuery(c->st);
+      if (e != hipErrorNotReady) {
+        if (e == hipSuccess && __atomic_load_n(f, __ATOMIC_ACQUIRE) == c->seq) return SMAC_OK;
+        fprintf(stderr, "smac: a reduction's result did not arrive: %s\n", hipGetErrorString(e));
+        return SMAC_ERR_HIP;
+      }
+      (void)hipGetLastError();  // not ready is no error
+    }
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+  }
 }
 
 extern "C" void smac_default_opts(smac_solver_opts* o) {
@@ -1377,6 +1403,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   // r = b - mean b; |r|^2 and sum r; then (pure Neumann) r -= mean r, and
   // f0 = (T) r. dp is zeroed only when the last correction has not cleared it.
   double size_inv = 1. / Ncell;
+  c->zs_done = false;
   const int zero_dp = c->dp_zero ? 0 : 1;
   c->dp_zero = false;
   launch_init_r<T>(g, c->rhs, c->r, f0, c->dp, zero_dp, c->S, pure ? S_MEANB : -1, 0.0, -1, P[0], P[1], 1,
@@ -1385,6 +1412,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     FinalizeArgs fa = fin(c);
     fin_add(fa, P[0], 0, S_BB);
     fin_add(fa, P[1], 0, S_SUMR);
+    fin_publish(c, fa);  // read below, while the first V-cycle runs
     launch_finalize(fa, c->S, s);
   }
   if (pure)
@@ -1411,7 +1439,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     launch_finalize(fa, c->S, s);
   }
   HIPOK(hipGetLastError());
-  int rc = read_scalars(c);
+  int rc = wait_scalars(c);
   if (rc) return rc;
   double bb = c->Sh[S_BB];
   double bnorm = sqrt(bb);
@@ -1447,6 +1475,8 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   const bool jac = small && !mg && !refg;  // Jacobi and its dots ride on the residual update
   int rz = S_RZ, rzn = S_RZN;
   bool fresh = false;  // S_RR and S_LINF on the host are those of the last update
+  bool near_end = false;
+  double last = o.stop_rule == SMAC_STOP_REF_LINF_DT ? 0.0 : bnorm;  // the last check's norm
   for (iter = 0; iter < o.max_iter && !conv && !nan; ++iter) {
     if (!ad_ready) KT(c, "spmv_dot", launch_spmv_dot(g, bfp, c->dv, c->Ad, small ? P[4] : P[0], s));
     double* pap = ad_ready || small ? P[4] : P[0];
@@ -1479,6 +1509,53 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
       launch_finalize(fa, c->S, s);
       KT(c, "add_scalar_norms", launch_add_scalar_norms(g, c->r, -1. * size_inv, c->S, S_SUMR, P[0], P[1], s));
     }
+    // The check of the new residual's norms. They are on the host some
+    // microseconds after the update: where the last checks' rate says that the
+    // solve may end here, the host waits for them first, so that no V-cycle
+    // runs after the last update; elsewhere it queues the V-cycle (or the next
+    // direction pass) and reads them while that runs. What is queued behind a
+    // check that ends the solve changes nothing that is read afterwards, but
+    // for the direction pass' dp += alpha d, which is the flush's.
+    const bool check = (iter % o.check_every) == 0;
+    if (check) {
+      FinalizeArgs fa = fin(c);
+      fin_add(fa, P[0], 0, S_RR);
+      fin_add(fa, P[1], 1, S_LINF);
+      fin_publish(c, fa);
+      launch_finalize(fa, c->S, s);
+    }
+    auto judge = [&]() -> int {  // 1: the solve ends, 0: not, < 0: an error
+      HIPOK(hipGetLastError());
+      const int w = wait_scalars(c);
+      if (w) return w;
+      fresh = true;
+      nan = !std::isfinite(c->Sh[S_RR]) || !std::isfinite(c->Sh[S_LINF]);
+      if (nan) return 1;
+      double m, target;
+      if (o.stop_rule == SMAC_STOP_REF_LINF_DT) {
+        m = linf = c->Sh[S_LINF] * dt;
+        target = o.tol;
+      } else {
+        rr = c->Sh[S_RR];
+        m = sqrt(rr);
+        target = o.tol * bnorm;
+      }
+      conv = m < target;
+      // the next check's norm at the rate of the last two, and a factor of 3
+      near_end = last > 0.0 && m < last && m * (m / last) < 3.0 * target;
+      last = m;
+      return conv;
+    };
+    bool judged = false;
+    if (check && near_end && !jac) {
+      const int e = judge();
+      if (e < 0) return e;
+      if (e) {
+        iter++;
+        break;
+      }
+      judged = true;
+    }
     c->dot_req = !stat;
     c->dot_done = false;
     c->dot_r = c->r;
@@ -1490,63 +1567,43 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     c->dot_req = false;
     if (!stat && !c->dot_done && !jac)
       KT(c, "dot2", launch_dot2<T>(g, c->r, z, c->Ad, o.flexible, P[2], P[3], s));
-    bool check = (iter % o.check_every) == 0;
-    {
-      if (!stat && !small) {
-        FinalizeArgs fa = fin(c);
-        fin_add(fa, P[2], 0, S_RZN);
-        if (o.flexible) fin_add(fa, P[3], 0, S_ZAD);
-        launch_finalize(fa, c->S, s);
-      }
-      FinalizeArgs fb = fin(c);
-      if (check) {
-        fin_add(fb, P[0], 0, S_RR);
-        fin_add(fb, P[1], 1, S_LINF);
-      }
-      if (stat || small) {
-        // no scalar operation: alpha and beta stay 1 and 0, or are formed by
-        // the pass that uses them
-      } else if (o.flexible) {
-        fb.op = OP_BETA_PR;
-        fb.dst = S_BETA;
-        fb.sa = S_ALPHA;
-        fb.sb = S_ZAD;
-        fb.sc = S_RZ;
+    if (!stat && !small) {
+      FinalizeArgs fa = fin(c);
+      fin_add(fa, P[2], 0, S_RZN);
+      if (o.flexible) fin_add(fa, P[3], 0, S_ZAD);
+      if (o.flexible) {
+        fa.op = OP_BETA_PR;
+        fa.dst = S_BETA;
+        fa.sa = S_ALPHA;
+        fa.sb = S_ZAD;
+        fa.sc = S_RZ;
       } else {
-        fb.op = OP_DIV;
-        fb.dst = S_BETA;
-        fb.sa = S_RZN;
-        fb.sb = S_RZ;
+        fa.op = OP_DIV;
+        fa.dst = S_BETA;
+        fa.sa = S_RZN;
+        fa.sb = S_RZ;
       }
-      if (fb.count > 0 || fb.op != OP_NONE) launch_finalize(fb, c->S, s);
+      launch_finalize(fa, c->S, s);
     }
-    if (check) {
-      HIPOK(hipGetLastError());
-      rc = read_scalars(c);
-      if (rc) return rc;
-      fresh = true;
-      if (!std::isfinite(c->Sh[S_RR]) || !std::isfinite(c->Sh[S_LINF])) {
+    const bool more = iter + 1 < o.max_iter;
+    if (jac && more) {
+      KT(c, "dir_spmv", launch_pcg_dir<T>(g, bfp, P[2], P[3], o.flexible, c->S, rz, rzn, z, c->dv, c->dv2, c->dp, c->Ad,
+                                          P[4], s));
+      std::swap(c->dv, c->dv2);
+      std::swap(rz, rzn);
+      ad_ready = true;
+      dp_pending = false;
+    }
+    if (check && !judged) {
+      const int e = judge();
+      if (e < 0) return e;
+      if (e) {
         iter++;
-        nan = true;
         break;
       }
-      if (o.stop_rule == SMAC_STOP_REF_LINF_DT) {
-        linf = c->Sh[S_LINF] * dt;
-        if (linf < o.tol) {
-          iter++;
-          conv = 1;
-          break;
-        }
-      } else {
-        rr = c->Sh[S_RR];
-        if (sqrt(rr) < o.tol * bnorm) {
-          iter++;
-          conv = 1;
-          break;
-        }
-      }
     }
-    if (small && iter + 1 < o.max_iter) {
+    if (jac) continue;
+    if (small && more) {
       KT(c, "dir_spmv", launch_pcg_dir<T>(g, bfp, P[2], P[3], o.flexible, c->S, rz, rzn, z, c->dv, c->dv2, c->dp, c->Ad,
                                           P[4], s));
       std::swap(c->dv, c->dv2);
@@ -1558,7 +1615,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     // (small grids, the last iteration: no direction is needed any more, and
     // the flush below adds its alpha d)
     if (small) continue;
-    if (fuse && iter + 1 < o.max_iter) {
+    if (fuse && more) {
       KT(c, "dir_spmv", launch_dir_spmv<T>(g, bfp, z, c->dv, c->dv2, c->dp, c->Ad, P[4], c->S, S_ALPHA, S_BETA, s));
       std::swap(c->dv, c->dv2);
       ad_ready = true;
@@ -1568,6 +1625,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     dp_pending = false;
     if (!stat) launch_scalar_copy(c->S, S_RZ, S_RZN, s);
   }
+  c->zs_done = false;  // a half sweep ahead of a V-cycle that was not taken
   // the last update's dp += alpha d (S_ALPHA still holds its alpha)
   if (dp_pending) {
     if (c->defer_dp) c->dp_deferred = true;
@@ -1586,8 +1644,9 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
         FinalizeArgs fa = fin(c);
         fin_add(fa, P[0], 0, S_RR);
         fin_add(fa, P[1], 1, S_LINF);
+        fin_publish(c, fa);
         launch_finalize(fa, c->S, s);
-        rc = read_scalars(c);
+        rc = wait_scalars(c);
         if (rc) return rc;
       }
       rr = c->Sh[S_RR];
@@ -1996,9 +2055,10 @@ extern "C" int smac_calc_cfl(smac_ctx* c, double dt, double* cc, double* cv) {
   FinalizeArgs fa = fin(c);
   fin_add(fa, c->part[0], 1, S_CFLC);
   fin_add(fa, c->part[1], 1, S_CFLV);
+  fin_publish(c, fa);
   launch_finalize(fa, c->S, c->st);
   HIPOK(hipGetLastError());
-  rc = read_scalars(c);
+  rc = wait_scalars(c);
   if (rc) return rc;
   if (cc) *cc = c->Sh[S_CFLC];
   if (cv) *cv = c->Sh[S_CFLV];

@@ -111,6 +111,10 @@ struct FinalizeArgs {
   int op, dst, sa, sb, sc;
   double c;
   double* stage;  // 3*1024 doubles: per-lane sums of large reductions (may be null)
+  // host != nullptr (pinned): the results also go to host[out[m]], then the
+  // number `seq` to the word host[S_COUNT]
+  double* host;
+  uint64_t seq;
 };
 
 // device scalar slots

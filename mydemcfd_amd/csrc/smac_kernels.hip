@@ -1451,10 +1451,16 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs fa, double* __re
     if (t < 64) {
       double v = lds[t];
       v = kind == 0 ? wave_tree_sum(v) : wave_max(v);
-      if (t == 0) S[fa.out[m]] = v;
+      if (t == 0) {
+        S[fa.out[m]] = v;
+        if (fa.host) fa.host[fa.out[m]] = v;
+      }
     }
     __syncthreads();
   }
+  if (t == 0 && fa.host)  // the values above before the number the host waits for
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(fa.host + S_COUNT), fa.seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   if (t == 0) {
     switch (fa.op) {
       case OP_MEAN:  // S[dst] = S[a] / c
