@@ -627,8 +627,20 @@ extern "C" size_t smac_field_count(const smac_ctx* c, int32_t f) {
   return (size_t)sh[0] * (size_t)sh[1] * (size_t)sh[2];
 }
 
-// copy between the reference layout (src pitch sh0, plane sh0*sh1) and the
-// padded box, one 2-D copy per z-plane
+// a device field between the reference layout and the box, queued on the
+// context stream
+static int move_field(smac_ctx* c, int f, double* box, const double* ref, bool to_box) {
+  int sh[3];
+  field_shape(c, f, sh);
+  launch_field_copy(box, const_cast<double*>(ref), c->g.px, c->g.py, sh, to_box ? 1 : 0, c->st);
+  HIPOK(hipGetLastError());
+  return SMAC_OK;
+}
+static int field_in(smac_ctx* c, int f, double* box, const double* ref) { return move_field(c, f, box, ref, true); }
+static int field_out(smac_ctx* c, int f, double* ref, double* box) { return move_field(c, f, box, ref, false); }
+
+// copy between a host array in the reference layout (src pitch sh0, plane
+// sh0*sh1) and the padded box, one 2-D copy per z-plane
 static int copy_field(smac_ctx* c, int f, double* dst_box, const double* src_ref, bool to_box, hipMemcpyKind kind,
                       double* dst_ref, const double* src_box) {
   int sh[3];
@@ -727,7 +739,10 @@ extern "C" int smac_upload_device(smac_ctx* c, int32_t f, const double* dsrc, si
     c->props_ready = false;
     c->props_ver++;
   }
-  return copy_field(c, f, *slot, dsrc, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+  const int rc = field_in(c, f, *slot, dsrc);
+  if (rc) return rc;
+  HIPOK(hipStreamSynchronize(c->st));
+  return SMAC_OK;
 }
 
 extern "C" int smac_device_layout(const smac_ctx* c, int64_t* pitch_x, int64_t* pitch_y, int64_t* planes) {
@@ -782,7 +797,10 @@ extern "C" int smac_download_device(smac_ctx* c, int32_t f, double* ddst, size_t
   if (count != smac_field_count(c, f)) return SMAC_ERR_INVALID_ARG;
   double** slot = field_slot(c, f);
   if (!*slot) return SMAC_ERR_INVALID_ARG;
-  return copy_field(c, f, nullptr, nullptr, false, hipMemcpyDeviceToDevice, ddst, *slot);
+  const int rc = field_out(c, f, ddst, *slot);
+  if (rc) return rc;
+  HIPOK(hipStreamSynchronize(c->st));
+  return SMAC_OK;
 }
 
 // ------------------------------------------------------------------ the step
@@ -1889,11 +1907,11 @@ extern "C" int smac_adjoint_step(smac_ctx* c, double dt, const smac_solver_opts*
   hipStream_t s = c->st;
   // the state of the step and the cotangents of its output, in the box layout
   for (int a = 0; a < 3; a++) {
-    rc = copy_field(c, SMAC_FIELD_U + a, c->u[a], u_n[a], true, hipMemcpyDeviceToDevice, nullptr, nullptr);
-    if (!rc) rc = copy_field(c, SMAC_FIELD_U + a, ubn[a], ubar[a], true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+    rc = field_in(c, SMAC_FIELD_U + a, c->u[a], u_n[a]);
+    if (!rc) rc = field_in(c, SMAC_FIELD_U + a, ubn[a], ubar[a]);
     if (rc) return rc;
   }
-  rc = copy_field(c, SMAC_FIELD_P, pb, pbar, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+  rc = field_in(c, SMAC_FIELD_P, pb, pbar);
   if (rc) return rc;
   const bool var = var_props(c);
   const BetaF bf = beta_of(c);
@@ -1915,10 +1933,13 @@ extern "C" int smac_adjoint_step(smac_ctx* c, double dt, const smac_solver_opts*
   launch_rg_zero(c->dp, c->tot, s);
   HIPOK(hipGetLastError());
   for (int a = 0; a < 3; a++) {
-    rc = copy_field(c, SMAC_FIELD_U + a, nullptr, nullptr, false, hipMemcpyDeviceToDevice, ubar[a], un[a]);
+    rc = field_out(c, SMAC_FIELD_U + a, ubar[a], un[a]);
     if (rc) return rc;
   }
-  return copy_field(c, SMAC_FIELD_P, nullptr, nullptr, false, hipMemcpyDeviceToDevice, pbar, pbo);
+  rc = field_out(c, SMAC_FIELD_P, pbar, pbo);
+  if (rc) return rc;
+  HIPOK(hipStreamSynchronize(c->st));
+  return SMAC_OK;
 }
 
 // Adjoint of one step of the VoF loop (smac_transport_alpha(dt, S, step) then
@@ -1966,10 +1987,10 @@ extern "C" int smac_adjoint_vof_step(smac_ctx* c, double dt, int32_t S, int32_t 
   hipStream_t s = c->st;
   const size_t bytes = c->tot * sizeof(double);
   // ---- the step again, from (alpha^n, u^n, p^n)
-  rc = copy_field(c, SMAC_FIELD_ALPHA, ral[0], alpha_n, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+  rc = field_in(c, SMAC_FIELD_ALPHA, ral[0], alpha_n);
   for (int a = 0; a < 3 && !rc; a++)
-    rc = copy_field(c, SMAC_FIELD_U + a, c->u[a], u_n[a], true, hipMemcpyDeviceToDevice, nullptr, nullptr);
-  if (!rc) rc = copy_field(c, SMAC_FIELD_P, c->p, p_n, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+    rc = field_in(c, SMAC_FIELD_U + a, c->u[a], u_n[a]);
+  if (!rc) rc = field_in(c, SMAC_FIELD_P, c->p, p_n);
   if (rc) return rc;
   HIPOK(hipMemcpyAsync(c->alpha, ral[0], bytes, hipMemcpyDeviceToDevice, s));
   c->alpha_nonzero = true;  // the property arrays of a two-phase grid
@@ -1992,9 +2013,9 @@ extern "C" int smac_adjoint_vof_step(smac_ctx* c, double dt, int32_t S, int32_t 
   HIPOK(hipMemcpyAsync(dpf, c->dp, bytes, hipMemcpyDeviceToDevice, s));
   // ---- cotangents of the step's output, box layout
   for (int a = 0; a < 3 && !rc; a++)
-    rc = copy_field(c, SMAC_FIELD_U + a, ubn[a], ubar[a], true, hipMemcpyDeviceToDevice, nullptr, nullptr);
-  if (!rc) rc = copy_field(c, SMAC_FIELD_P, pb, pbar, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
-  if (!rc) rc = copy_field(c, SMAC_FIELD_ALPHA, X, alpha_bar, true, hipMemcpyDeviceToDevice, nullptr, nullptr);
+    rc = field_in(c, SMAC_FIELD_U + a, ubn[a], ubar[a]);
+  if (!rc) rc = field_in(c, SMAC_FIELD_P, pb, pbar);
+  if (!rc) rc = field_in(c, SMAC_FIELD_ALPHA, X, alpha_bar);
   if (rc) return rc;
   launch_rg_zero(anx, c->tot, s);
   for (int a = 0; a < 3; a++) launch_rg_zero(Fb[a], c->tot, s);
@@ -2037,10 +2058,12 @@ extern "C" int smac_adjoint_vof_step(smac_ctx* c, double dt, int32_t S, int32_t 
   launch_rg_zero(c->dp, c->tot, s);
   HIPOK(hipGetLastError());
   for (int a = 0; a < 3 && !rc; a++)
-    rc = copy_field(c, SMAC_FIELD_U + a, nullptr, nullptr, false, hipMemcpyDeviceToDevice, ubar[a], un[a]);
-  if (!rc) rc = copy_field(c, SMAC_FIELD_P, nullptr, nullptr, false, hipMemcpyDeviceToDevice, pbar, pbo);
-  if (!rc) rc = copy_field(c, SMAC_FIELD_ALPHA, nullptr, nullptr, false, hipMemcpyDeviceToDevice, alpha_bar, X);
-  return rc;
+    rc = field_out(c, SMAC_FIELD_U + a, ubar[a], un[a]);
+  if (!rc) rc = field_out(c, SMAC_FIELD_P, pbar, pbo);
+  if (!rc) rc = field_out(c, SMAC_FIELD_ALPHA, alpha_bar, X);
+  if (rc) return rc;
+  HIPOK(hipStreamSynchronize(c->st));
+  return SMAC_OK;
 }
 
 extern "C" int smac_calc_cfl(smac_ctx* c, double dt, double* cc, double* cv) {

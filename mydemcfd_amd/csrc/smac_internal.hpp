@@ -260,6 +260,8 @@ void launch_ghost_velocity(const Geo& g, double* const u[3], hipStream_t st);
 void launch_outlet_faces(const Geo& g, const double* const us[3], const double* const beta[3], const double* dp,
                          double* const u[3], double dt, hipStream_t st);
 void launch_face_gradp(const Geo& g, const double* p, double* const gp[3], hipStream_t st);
+// a field between the box and the dense reference layout (sh cells), on the device
+void launch_field_copy(double* box, double* ref, int px, int py, const int sh[3], int to_box, hipStream_t st);
 // VTI cell data: p[n], alpha[n] (al == nullptr: 0), velocity[3n] as float
 void launch_pack_cells(const Geo& g, const double* p, const double* al, const double* const u[3], float* out,
                        hipStream_t st);
