@@ -11,6 +11,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <string>
 #include <type_traits>
@@ -117,6 +118,12 @@ struct smac_ctx {
   int rg_req = 0;
   double rg_beta0 = 0.0;
   uint64_t rg_ver = ~0ull;
+  // levels rg_first.. of the reference's multigrid run in one workgroup
+  // (rg_first = the level count: none do); rg_tail describes the levels on the
+  // device
+  int rg_first = 0;
+  int rg_tail_small = 0;
+  RgTailLv* rg_tail = nullptr;
   // two-phase properties (allocated on first use; natural layout)
   double *rho = nullptr, *rho_old = nullptr, *inv_rho = nullptr, *mu = nullptr;
   double* beta[3] = {nullptr, nullptr, nullptr};
@@ -532,6 +539,8 @@ static void rg_free(smac_ctx* c) {
   c->rg_req = 0;
   dfree(c->rgt);
   c->rgt = nullptr;
+  dfree(c->rg_tail);
+  c->rg_tail = nullptr;
 }
 
 static double** field_slot(smac_ctx* c, int f);
@@ -1183,14 +1192,8 @@ static void vcycle(smac_ctx* c, int l, int nu1, int nu2) {
   }
 }
 
-// G_GMGSolver::initialize + create_coeffs (CFD/pressure_solver/G_GMGSolver.cu:10-147,913-922).
-// Returns the level count or a negative status: an odd size in a coarsened
-// direction (the reference aborts) or a single level (the reference then
-// prolongs through levels_[-1], G_GMGSolver.cu:971).
-static int rg_setup(smac_ctx* c, int req) {
-  if (req < 1 || req > 16) return SMAC_ERR_INVALID_ARG;
-  const uint64_t ver = pois_var(c) ? c->props_ver : 0;
-  if (!c->rg.empty() && c->rg_req == req && c->rg_beta0 == c->g.beta0 && c->rg_ver == ver) return (int)c->rg.size();
+// the levels and their arrays; 0 or a negative status
+static int rg_alloc(smac_ctx* c, int req) {
   rg_free(c);
   std::vector<RgLv> lv;
   int prev[3] = {c->n[0], c->n[1], c->n[2]};
@@ -1232,6 +1235,43 @@ static int rg_setup(smac_ctx* c, int req) {
     rg_free(c);
     return rc;
   }
+  {
+    const int nl = (int)lv.size();
+    c->rg_first = nl;
+    while (c->rg_first > 0 && rg_tail_applies(lv[c->rg_first - 1])) c->rg_first--;
+    c->rg_tail_small = 1;
+    std::vector<RgTailLv> T((size_t)nl);
+    for (int l = 0; l < nl; l++) {
+      RgLevel& V = c->rg[l];
+      T[l].L = V.lv;
+      T[l].q = V.q;
+      T[l].rhs = V.rhs;
+      for (int d = 0; d < 3; d++) T[l].b[d] = V.b[d];
+      if (l >= c->rg_first && V.lv.n[0] * V.lv.n[1] * V.lv.n[2] > 1024) c->rg_tail_small = 0;
+    }
+    rc = balloc((void**)&c->rg_tail, T.size() * sizeof(RgTailLv));
+    if (rc) {
+      rg_free(c);
+      return rc;
+    }
+    HIPOK(hipMemcpy(c->rg_tail, T.data(), T.size() * sizeof(RgTailLv), hipMemcpyHostToDevice));
+  }
+  return SMAC_OK;
+}
+// G_GMGSolver::initialize + create_coeffs (CFD/pressure_solver/G_GMGSolver.cu:10-147,913-922).
+// Returns the level count or a negative status: an odd size in a coarsened
+// direction (the reference aborts) or a single level (the reference then
+// prolongs through levels_[-1], G_GMGSolver.cu:971).
+static int rg_setup(smac_ctx* c, int req) {
+  if (req < 1 || req > 16) return SMAC_ERR_INVALID_ARG;
+  const uint64_t ver = pois_var(c) ? c->props_ver : 0;
+  if (!c->rg.empty() && c->rg_req == req && c->rg_beta0 == c->g.beta0 && c->rg_ver == ver) return (int)c->rg.size();
+  // the levels depend on the grid alone; new coefficients need new face
+  // coefficients only
+  if (c->rg.empty() || c->rg_req != req) {
+    const int rc = rg_alloc(c, req);
+    if (rc) return rc;
+  }
   // face coefficients (create_coeffs); rebuilt when the grid's coefficients change
   const BetaF gb = pois_of(c);
   for (size_t l = 0; l < c->rg.size(); l++)
@@ -1254,38 +1294,63 @@ static void rg_vcycle(smac_ctx* c, const smac_solver_opts& o) {
   const BetaF* gbp = pois_var(c) ? &gb : nullptr;
   double* x = c->z;
   double* t = c->rgt;
-  for (auto& V : c->rg) KT(c, "rg_levels", launch_rg_zero(V.q, V.tot, s));
-  if (nf == 0) KT(c, "rg_fine", launch_rg_zero(x, c->tot, s));
-  for (int it = 0; it < nf; it++) {
-    KT(c, "rg_fine_jacobi", launch_rg_fine_jacobi(g, gbp, x, t, c->r, it == 0, s));
-    std::swap(x, t);
+  // the finest grid and the levels that take one launch down and one up; the
+  // levels from rg_first on run in one workgroup
+  const bool fine_tile = nf == 4 && rg_tile_applies(g.n);
+  auto tile = [&](int l) { return nf == 4 && rg_tile_applies(c->rg[l].lv.n); };
+  const int tail = c->rg_first;
+  if (fine_tile) {
+    KT(c, "rg_fine_down", launch_rg_fine_down(g, gbp, c->r, t, c->rg[0].lv, c->rg[0].rhs, s));
+  } else {
+    if (nf == 0) KT(c, "rg_fine", launch_rg_zero(x, c->tot, s));
+    for (int it = 0; it < nf; it++) {
+      KT(c, "rg_fine_jacobi", launch_rg_fine_jacobi(g, gbp, x, t, c->r, it == 0, s));
+      std::swap(x, t);
+    }
+    KT(c, "rg_fine_restrict", launch_rg_fine_res_restrict(g, gbp, x, c->r, c->rg[0].lv, c->rg[0].rhs, s));
   }
-  KT(c, "rg_fine_restrict", launch_rg_fine_res_restrict(g, gbp, x, c->r, c->rg[0].lv, c->rg[0].rhs, s));
-  for (int l = 0; l < L - 1; l++) {
+  for (int l = 0; l < std::min(tail, L - 1); l++) {
     RgLevel& V = c->rg[l];
+    if (tile(l)) {
+      KT(c, "rg_levels", launch_rg_down(V.lv, V.b, V.rhs, V.q, c->rg[l + 1].lv, c->rg[l + 1].rhs, s));
+      continue;
+    }
+    KT(c, "rg_levels", launch_rg_zero(V.q, V.tot, s));
     for (int it = 0; it < nf; it++) {
       KT(c, "rg_levels", launch_rg_jacobi(V.lv, V.b, V.q, V.qt, V.rhs, s));
       std::swap(V.q, V.qt);
     }
     KT(c, "rg_levels", launch_rg_res_restrict(V.lv, V.b, V.q, V.rhs, c->rg[l + 1].lv, c->rg[l + 1].rhs, s));
   }
-  {
+  if (tail < L) {
+    KT(c, "rg_levels", launch_rg_tail(c->rg_tail, tail, L - 1, nf, nc, c->rg_tail_small, s));
+  } else {
     RgLevel& V = c->rg[L - 1];
+    KT(c, "rg_levels", launch_rg_zero(V.q, V.tot, s));
     for (int it = 0; it < nc; it++) {
       KT(c, "rg_levels", launch_rg_jacobi(V.lv, V.b, V.q, V.qt, V.rhs, s));
       std::swap(V.q, V.qt);
     }
-    KT(c, "rg_levels", launch_rg_prolong(V.lv, V.q, c->rg[L - 2].lv, c->rg[L - 2].q, s));
   }
-  for (int l = L - 2; l >= 0; l--) {
+  for (int l = std::min(tail, L - 1) - 1; l >= 0; l--) {
     RgLevel& V = c->rg[l];
+    const RgLevel& C = c->rg[l + 1];
+    if (tile(l)) {
+      KT(c, "rg_levels", launch_rg_up(V.lv, V.b, C.lv, C.q, V.q, V.rhs, V.qt, s));
+      std::swap(V.q, V.qt);
+      continue;
+    }
+    KT(c, "rg_levels", launch_rg_prolong(C.lv, C.q, V.lv, V.q, s));
     for (int it = 0; it < nf; it++) {
       KT(c, "rg_levels", launch_rg_jacobi(V.lv, V.b, V.q, V.qt, V.rhs, s));
       std::swap(V.q, V.qt);
     }
-    if (l != 0) KT(c, "rg_levels", launch_rg_prolong(V.lv, V.q, c->rg[l - 1].lv, c->rg[l - 1].q, s));
-    else KT(c, "rg_fine_prolong", launch_rg_prolong_fine(V.lv, V.q, g, x, s));
   }
+  if (fine_tile) {
+    KT(c, "rg_fine_up", launch_rg_fine_up(g, gbp, c->rg[0].lv, c->rg[0].q, t, c->r, x, s));
+    return;
+  }
+  KT(c, "rg_fine_prolong", launch_rg_prolong_fine(c->rg[0].lv, c->rg[0].q, g, x, s));
   for (int it = 0; it < nf; it++) {
     KT(c, "rg_fine_jacobi", launch_rg_fine_jacobi(g, gbp, x, t, c->r, 0, s));
     std::swap(x, t);

@@ -342,6 +342,28 @@ void launch_rg_fine_jacobi(const Geo& g, const BetaF* gb, const double* x, doubl
 void launch_rg_fine_res_restrict(const Geo& g, const BetaF* gb, const double* x, const double* r, const RgLv& C,
                                  double* crhs, hipStream_t st);
 void launch_rg_prolong_fine(const RgLv& C, const double* cq, const Geo& g, double* x, hipStream_t st);
+// small levels: the four sweeps of a level (or of the finest grid) from zero
+// with the residual's restriction, or after the prolongation, in one launch;
+// and all levels from `first` to the coarsest and back in one workgroup
+struct RgTailLv {
+  RgLv L;
+  double *q, *rhs;
+  const double* b[3];
+};
+constexpr size_t RG_TILE_CELLS = (size_t)1 << 17;
+constexpr int RG_TAIL_CELLS = 4096, RG_TAIL_PAD = 8192;
+bool rg_tile_applies(const int n[3]);
+bool rg_tail_applies(const RgLv& L);
+void launch_rg_down(const RgLv& L, double* const b[3], const double* rhs, double* q, const RgLv& C, double* crhs,
+                    hipStream_t st);
+void launch_rg_up(const RgLv& L, double* const b[3], const RgLv& C, const double* cq, const double* qi,
+                  const double* rhs, double* qo, hipStream_t st);
+void launch_rg_fine_down(const Geo& g, const BetaF* gb, const double* r, double* x, const RgLv& C, double* crhs,
+                         hipStream_t st);
+void launch_rg_fine_up(const Geo& g, const BetaF* gb, const RgLv& C, const double* cq, const double* xi,
+                       const double* r, double* xo, hipStream_t st);
+// T: the levels on the device; small: none of them has over 1024 cells
+void launch_rg_tail(const RgTailLv* T, int first, int last, int nf, int nc, int small, hipStream_t st);
 void launch_rg_zero(double* x, size_t n, hipStream_t st);
 void launch_add_scalar_norms(const Geo& g, double* r, double a, const double* S, int slot, double* p0, double* p1,
                              hipStream_t st);

@@ -305,6 +305,346 @@ __global__ __launch_bounds__(256) void k_add_scalar_norms(Geo g, double* __restr
   }
 }
 
+// ------------------------------------------------------------- small levels
+// On levels and grids of up to RG_TILE_CELLS cells a sweep is bound by its
+// launch (2.8 us for a few thousand cells), and the V-cycle takes 46 of them.
+//
+// k_rg_down / k_rg_up do a level's four sweeps with its residual and
+// restriction, or with the prolongation before them, in one launch: a block
+// owns an 8^3 tile, holds it with a halo of 4 in LDS (two copies, as Jacobi
+// reads the old values) and repeats its neighbours' work there, each sweep on
+// a region one cell smaller. k_rg_tail does all levels that fit one
+// workgroup's LDS, from the first of them down to the coarsest sweeps and
+// back. Per cell the operations and their order are those of the sweeps above.
+// Bound by latency: 64x32x32 11 us down and 11 us up where nine launches took
+// 28 and 20 us; the 32x16x16 level 8 us each way against 20; the 38 sweeps of
+// the levels 16x8x8 and 8x8x8 19 us against 115.
+constexpr int RB_T = 8, RB_H = 4, RB_W = RB_T + 2 * RB_H, RB_N = RB_W * RB_W * RB_W;
+
+// FINE: the finest grid (row-split vectors, its own operator), else a level
+template <bool FINE, bool VAR>
+struct RgView {
+  Geo g;
+  BetaF gb;
+  RgLv L;
+  const double* b[3];
+  __device__ __forceinline__ int n(int d) const { return FINE ? g.n[d] : L.n[d]; }
+  __device__ __forceinline__ int per(int d) const { return FINE ? g.per[d] : L.per[d]; }
+  __device__ __forceinline__ size_t at(int i, int j, int k) const {
+    if constexpr (FINE) return idx(g, 0, j, k) + (size_t)spos(i, g.n[0]);
+    return ridx(L, i, j, k);
+  }
+  __device__ __forceinline__ RgCoef coef(int i, int j, int k) const {
+    if constexpr (FINE) {
+      const Coef c = VAR ? coef_var(g, gb.b, i, j, k) : coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k);
+      RgCoef r;
+#pragma unroll
+      for (int m = 0; m < 6; m++) r.a[m] = c.a[m];
+      r.diag = c.diag;
+      r.inv = 1. / c.diag;
+      return r;
+    }
+    return rg_coef(L, b[0], b[1], b[2], i, j, k);
+  }
+};
+// one sweep's new value at p of x, neighbours at p +- 1, +- sy, +- sz
+__device__ __forceinline__ double rg_relax(const double* x, int p, int sy, int sz, const RgCoef& c, double rhs) {
+  const double omega = RG_OMEGA;
+  const double s = c.a[0] * x[p + 1] + c.a[1] * x[p - 1] + c.a[2] * x[p + sy] + c.a[3] * x[p - sy] +
+                   c.a[4] * x[p + sz] + c.a[5] * x[p - sz];
+  return (1.0 - omega) * x[p] + omega * (s + rhs) * c.inv;
+}
+__device__ __forceinline__ int rg_dist(int l) { return max(max(RB_H - l, l - (RB_H + RB_T - 1)), 0); }
+// image of v in 1..n of a periodic axis: -3 <= v <= n + 11, n >= 4
+__device__ __forceinline__ int rg_image(int v, int n) {
+  v += v < 1 ? n : 0;
+#pragma unroll
+  for (int u = 0; u < 3; u++) v -= v > n ? n : 0;
+  return v;
+}
+// The four cells of a thread in the box (planes lz = t >> 8, + 4, + 8, + 12)
+struct RgCell {
+  int i, j, k, d;  // in 1..n; cells outside the tile, 15 = none
+  bool own;        // in the tile and the grid, not an image
+};
+template <class V>
+__device__ __forceinline__ RgCell rg_box_cell(const V& v, const int o[3], int m) {
+  const int t = (int)threadIdx.x;
+  const int l[3] = {t & 15, (t >> 4) & 15, (t >> 8) + 4 * m};
+  int q[3];
+  RgCell c;
+  c.d = 0;
+  c.own = true;
+  bool ok = true;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int x = o[d] - RB_H + l[d];
+    const bool in = x >= 1 && x <= v.n(d);
+    c.d = max(c.d, rg_dist(l[d]));
+    c.own = c.own && in;
+    q[d] = v.per(d) ? rg_image(x, v.n(d)) : x;
+    ok = ok && (in || v.per(d));
+  }
+  c.own = c.own && c.d == 0;
+  if (!ok) c.d = 15;
+  c.i = q[0];
+  c.j = q[1];
+  c.k = q[2];
+  return c;
+}
+
+template <bool FINE, bool VAR>
+__global__ __launch_bounds__(1024) void k_rg_down(RgView<FINE, VAR> V, const double* __restrict__ rhs,
+                                                  double* __restrict__ q, RgLv C, double* __restrict__ crhs) {
+  __shared__ double X[2][RB_N];
+  constexpr int SY = RB_W, SZ = RB_W * RB_W;
+  const int t = (int)threadIdx.x;
+  const int o[3] = {1 + RB_T * (int)blockIdx.x, 1 + RB_T * (int)blockIdx.y, 1 + RB_T * (int)blockIdx.z};
+  RgCell c[4];
+  RgCoef k[4];
+  double f[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    c[m] = rg_box_cell(V, o, m);
+    f[m] = 0.0;
+    if (c[m].d <= 4) {
+      f[m] = rhs[V.at(c[m].i, c[m].j, c[m].k)];
+      k[m] = V.coef(c[m].i, c[m].j, c[m].k);
+    }
+  }
+  const double omega = RG_OMEGA;
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    // from zero: the neighbour sum is 0
+    X[0][t + 1024 * m] = c[m].d <= 4 ? (1.0 - omega) * 0.0 + omega * (0.0 + f[m]) * k[m].inv : 0.0;
+    X[1][t + 1024 * m] = 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      if (c[m].d <= 3 - s) X[(s + 1) & 1][t + 1024 * m] = rg_relax(X[s & 1], t + 1024 * m, SY, SZ, k[m], f[m]);
+    __syncthreads();
+  }
+  // the sweeps' result is in X[1]; residual of the tile's cells into X[0]
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    if (c[m].own) {
+      const int p = t + 1024 * m;
+      const double* x = X[1];
+      const double s = k[m].a[0] * x[p + 1] + k[m].a[1] * x[p - 1] + k[m].a[2] * x[p + SY] + k[m].a[3] * x[p - SY] +
+                       k[m].a[4] * x[p + SZ] + k[m].a[5] * x[p - SZ];
+      const double Ap = x[p] * k[m].diag - s;
+      X[0][p] = f[m] - Ap;
+      q[V.at(c[m].i, c[m].j, c[m].k)] = x[p];
+    }
+  }
+  __syncthreads();
+  const int w[3] = {C.co[0] ? RB_T / 2 : RB_T, C.co[1] ? RB_T / 2 : RB_T, C.co[2] ? RB_T / 2 : RB_T};
+  if (t < w[0] * w[1] * w[2]) {
+    const int a[3] = {t % w[0], (t / w[0]) % w[1], t / (w[0] * w[1])};
+    int Q[3], l0[3], R[3];
+    bool in = true;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      R[d] = C.co[d] ? 2 : 1;
+      l0[d] = RB_H + R[d] * a[d];
+      Q[d] = (C.co[d] ? (o[d] + 1) / 2 : o[d]) + a[d];
+      in = in && Q[d] <= C.n[d];
+    }
+    if (in) {
+      double count = 0., tmp = 0.;
+      for (int iz = 0; iz < R[2]; iz++)
+        for (int iy = 0; iy < R[1]; iy++)
+          for (int ix = 0; ix < R[0]; ix++) {
+            tmp += X[0][(l0[2] + iz) * SZ + (l0[1] + iy) * SY + l0[0] + ix];
+            count += 1.0;
+          }
+      crhs[ridx(C, Q[0], Q[1], Q[2])] = tmp / count;
+    }
+  }
+}
+
+template <bool FINE, bool VAR>
+__global__ __launch_bounds__(1024) void k_rg_up(RgView<FINE, VAR> V, RgLv C, const double* __restrict__ cq,
+                                                const double* __restrict__ qi, const double* __restrict__ rhs,
+                                                double* __restrict__ qo) {
+  __shared__ double X[2][RB_N];
+  constexpr int SY = RB_W, SZ = RB_W * RB_W;
+  const int t = (int)threadIdx.x;
+  const int o[3] = {1 + RB_T * (int)blockIdx.x, 1 + RB_T * (int)blockIdx.y, 1 + RB_T * (int)blockIdx.z};
+  RgCell c[4];
+  RgCoef k[4];
+  double f[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) {
+    c[m] = rg_box_cell(V, o, m);
+    f[m] = 0.0;
+    double x = 0.0;
+    if (c[m].d <= 4) {
+      const int ci = C.co[0] ? (c[m].i + 1) / 2 : c[m].i, cj = C.co[1] ? (c[m].j + 1) / 2 : c[m].j,
+                ck = C.co[2] ? (c[m].k + 1) / 2 : c[m].k;
+      x = qi[V.at(c[m].i, c[m].j, c[m].k)] + cq[ridx(C, ci, cj, ck)];
+    }
+    if (c[m].d <= 3) {
+      f[m] = rhs[V.at(c[m].i, c[m].j, c[m].k)];
+      k[m] = V.coef(c[m].i, c[m].j, c[m].k);
+    }
+    X[0][t + 1024 * m] = x;
+    X[1][t + 1024 * m] = 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+      if (c[m].d <= 3 - s) X[(s + 1) & 1][t + 1024 * m] = rg_relax(X[s & 1], t + 1024 * m, SY, SZ, k[m], f[m]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int m = 0; m < 4; m++)
+    if (c[m].own) qo[V.at(c[m].i, c[m].j, c[m].k)] = rg_relax(X[1], t + 1024 * m, SY, SZ, k[m], f[m]);
+}
+
+// Levels first..last in one workgroup: a thread owns the cells t, t + 1024, ..
+// of the current level (its coefficients in registers), the level's values lie
+// in LDS with a zero ghost layer, twice.
+template <int CPT>
+__global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T, int first, int last, int nf, int nc) {
+  __shared__ double X[2][RG_TAIL_PAD];
+  const int t = (int)threadIdx.x;
+  double a[CPT][6], inv[CPT], f[CPT];
+  int p[CPT], off[CPT][3];  // LDS index (-1: no cell); (+, -) neighbour offsets per axis, 16 bits each
+  size_t at[CPT];
+  int cur = 0;
+  // the level's coefficients and right-hand side, both copies of X zero
+  auto load = [&](int l) {
+    const RgTailLv& V = T[l];
+    const RgLv& L = V.L;
+    const int sy = L.n[0] + 2, sz = sy * (L.n[1] + 2), pad = sz * (L.n[2] + 2);
+    for (int e = t; e < pad; e += 1024) {
+      X[0][e] = 0.0;
+      X[1][e] = 0.0;
+    }
+    cur = 0;
+    const int nxy = L.n[0] * L.n[1], cells = nxy * L.n[2];
+#pragma unroll
+    for (int u = 0; u < CPT; u++) {
+      const int e = t + 1024 * u;
+      p[u] = -1;
+      f[u] = 0.0;
+      if (e < cells) {
+        const int i = e % L.n[0] + 1, j = (e / L.n[0]) % L.n[1] + 1, k = e / nxy + 1;
+        p[u] = k * sz + j * sy + i;
+        at[u] = ridx(L, i, j, k);
+        f[u] = V.rhs[at[u]];
+        const RgCoef c = rg_coef(L, V.b[0], V.b[1], V.b[2], i, j, k);
+#pragma unroll
+        for (int m = 0; m < 6; m++) a[u][m] = c.a[m];
+        inv[u] = c.inv;
+        const int q[3] = {i, j, k}, st[3] = {1, sy, sz};
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          const int hi = L.per[d] && q[d] == L.n[d] ? -(L.n[d] - 1) * st[d] : st[d];
+          const int lo = L.per[d] && q[d] == 1 ? (L.n[d] - 1) * st[d] : -st[d];
+          off[u][d] = (int)(((unsigned)lo << 16) | ((unsigned)hi & 0xffffu));
+        }
+      }
+    }
+  };
+  auto nbsum = [&](const double* x, int u) -> double {
+    const int q = p[u];
+    double v[6];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      v[2 * d] = x[q + (int)(short)(off[u][d] & 0xffff)];
+      v[2 * d + 1] = x[q + (off[u][d] >> 16)];
+    }
+    return a[u][0] * v[0] + a[u][1] * v[1] + a[u][2] * v[2] + a[u][3] * v[3] + a[u][4] * v[4] + a[u][5] * v[5];
+  };
+  auto sweeps = [&](int n) {
+    const double omega = RG_OMEGA;
+#pragma unroll 1
+    for (int it = 0; it < n; it++) {
+      const double* x = X[cur];
+      double* y = X[1 - cur];
+#pragma unroll
+      for (int u = 0; u < CPT; u++)
+        if (p[u] >= 0) y[p[u]] = (1.0 - omega) * x[p[u]] + omega * (nbsum(x, u) + f[u]) * inv[u];
+      cur = 1 - cur;
+      __syncthreads();
+    }
+  };
+  auto store = [&](int l) {
+#pragma unroll
+    for (int u = 0; u < CPT; u++)
+      if (p[u] >= 0) T[l].q[at[u]] = X[cur][p[u]];
+  };
+#pragma unroll 1
+  for (int l = first; l < last; l++) {
+    load(l);
+    __syncthreads();
+    sweeps(nf);
+    store(l);
+    double* res = X[1 - cur];
+#pragma unroll
+    for (int u = 0; u < CPT; u++)
+      if (p[u] >= 0) {
+        const double diag = (a[u][0] + a[u][1] + a[u][2] + a[u][3] + a[u][4] + a[u][5]);
+        const double Ap = X[cur][p[u]] * diag - nbsum(X[cur], u);
+        res[p[u]] = f[u] - Ap;
+      }
+    __syncthreads();
+    const RgLv& L = T[l].L;
+    const RgLv& C = T[l + 1].L;
+    const int sy = L.n[0] + 2, sz = sy * (L.n[1] + 2);
+    for (int e = t; e < C.n[0] * C.n[1] * C.n[2]; e += 1024) {
+      const int Q[3] = {e % C.n[0] + 1, (e / C.n[0]) % C.n[1] + 1, e / (C.n[0] * C.n[1]) + 1};
+      int B[3], R[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        B[d] = C.co[d] ? 2 * Q[d] - 1 : Q[d];
+        R[d] = C.co[d] ? 2 : 1;
+      }
+      double count = 0., tmp = 0.;
+      for (int iz = 0; iz < R[2]; iz++)
+        for (int iy = 0; iy < R[1]; iy++)
+          for (int ix = 0; ix < R[0]; ix++) {
+            tmp += res[(B[2] + iz) * sz + (B[1] + iy) * sy + B[0] + ix];
+            count += 1.0;
+          }
+      T[l + 1].rhs[ridx(C, Q[0], Q[1], Q[2])] = tmp / count;
+    }
+    __syncthreads();
+  }
+  load(last);
+  __syncthreads();
+  sweeps(nc);
+  store(last);
+  __syncthreads();
+#pragma unroll 1
+  for (int l = last - 1; l >= first; l--) {
+    load(l);
+    __syncthreads();
+    const RgTailLv& V = T[l];
+    const RgLv& C = T[l + 1].L;
+#pragma unroll
+    for (int u = 0; u < CPT; u++)
+      if (p[u] >= 0) {
+        const int e = t + 1024 * u;
+        int Q[3] = {e % V.L.n[0] + 1, (e / V.L.n[0]) % V.L.n[1] + 1, e / (V.L.n[0] * V.L.n[1]) + 1};
+#pragma unroll
+        for (int d = 0; d < 3; d++) Q[d] = C.co[d] ? (Q[d] + 1) / 2 : Q[d];
+        X[0][p[u]] = V.q[at[u]] + T[l + 1].q[ridx(C, Q[0], Q[1], Q[2])];
+      }
+    __syncthreads();
+    sweeps(nf);
+    store(l);
+    __syncthreads();
+  }
+}
+
 dim3 cells_grid(const RgLv& L) {
   size_t n = (size_t)L.n[0] * L.n[1] * L.n[2];
   return dim3((unsigned)((n + RGB - 1) / RGB));
@@ -342,6 +682,61 @@ void launch_rg_fine_res_restrict(const Geo& g, const BetaF* gb, const double* x,
 }
 void launch_rg_prolong_fine(const RgLv& C, const double* cq, const Geo& g, double* x, hipStream_t st) {
   hipLaunchKernelGGL(k_rg_prolong_fine, cells_grid(C), dim3(RGB), 0, st, C, cq, g, x);
+}
+static dim3 rg_tiles(const int n[3]) {
+  return dim3((unsigned)((n[0] + RB_T - 1) / RB_T), (unsigned)((n[1] + RB_T - 1) / RB_T),
+              (unsigned)((n[2] + RB_T - 1) / RB_T));
+}
+// every axis at least 4 cells (the box's periodic images), few enough of them
+bool rg_tile_applies(const int n[3]) {
+  return n[0] >= 4 && n[1] >= 4 && n[2] >= 4 && (size_t)n[0] * n[1] * n[2] <= RG_TILE_CELLS;
+}
+bool rg_tail_applies(const RgLv& L) {
+  return L.n[0] * L.n[1] * L.n[2] <= RG_TAIL_CELLS && (L.n[0] + 2) * (L.n[1] + 2) * (L.n[2] + 2) <= RG_TAIL_PAD;
+}
+void launch_rg_down(const RgLv& L, double* const b[3], const double* rhs, double* q, const RgLv& C, double* crhs,
+                    hipStream_t st) {
+  RgView<false, true> V{};
+  V.L = L;
+  for (int d = 0; d < 3; d++) V.b[d] = b[d];
+  hipLaunchKernelGGL((k_rg_down<false, true>), rg_tiles(L.n), dim3(1024), 0, st, V, rhs, q, C, crhs);
+}
+void launch_rg_up(const RgLv& L, double* const b[3], const RgLv& C, const double* cq, const double* qi,
+                  const double* rhs, double* qo, hipStream_t st) {
+  RgView<false, true> V{};
+  V.L = L;
+  for (int d = 0; d < 3; d++) V.b[d] = b[d];
+  hipLaunchKernelGGL((k_rg_up<false, true>), rg_tiles(L.n), dim3(1024), 0, st, V, C, cq, qi, rhs, qo);
+}
+void launch_rg_fine_down(const Geo& g, const BetaF* gb, const double* r, double* x, const RgLv& C, double* crhs,
+                         hipStream_t st) {
+  if (gb) {
+    RgView<true, true> V{};
+    V.g = g;
+    V.gb = *gb;
+    hipLaunchKernelGGL((k_rg_down<true, true>), rg_tiles(g.n), dim3(1024), 0, st, V, r, x, C, crhs);
+  } else {
+    RgView<true, false> V{};
+    V.g = g;
+    hipLaunchKernelGGL((k_rg_down<true, false>), rg_tiles(g.n), dim3(1024), 0, st, V, r, x, C, crhs);
+  }
+}
+void launch_rg_fine_up(const Geo& g, const BetaF* gb, const RgLv& C, const double* cq, const double* xi,
+                       const double* r, double* xo, hipStream_t st) {
+  if (gb) {
+    RgView<true, true> V{};
+    V.g = g;
+    V.gb = *gb;
+    hipLaunchKernelGGL((k_rg_up<true, true>), rg_tiles(g.n), dim3(1024), 0, st, V, C, cq, xi, r, xo);
+  } else {
+    RgView<true, false> V{};
+    V.g = g;
+    hipLaunchKernelGGL((k_rg_up<true, false>), rg_tiles(g.n), dim3(1024), 0, st, V, C, cq, xi, r, xo);
+  }
+}
+void launch_rg_tail(const RgTailLv* T, int first, int last, int nf, int nc, int small, hipStream_t st) {
+  if (small) hipLaunchKernelGGL(k_rg_tail<1>, dim3(1), dim3(1024), 0, st, T, first, last, nf, nc);
+  else hipLaunchKernelGGL(k_rg_tail<4>, dim3(1), dim3(1024), 0, st, T, first, last, nf, nc);
 }
 void launch_rg_zero(double* x, size_t n, hipStream_t st) {
   hipLaunchKernelGGL(k_rg_zero, dim3((unsigned)((n + RGB - 1) / RGB)), dim3(RGB), 0, st, x, n);
