@@ -1,7 +1,7 @@
 // smac_adjoint.hip -- adjoint (vector-Jacobian product) of one SMAC step.
 //
 // Forward step, from (u^n, p^n):
-//   u*      = F(u^n) - dt beta G p^n           predictor (k_predict; F holds
+//   u*      = F(u^n) - dt beta G p^n           predictor (F holds
 //                                              the time, stress and MUSCL terms)
 //   b       = -(1/dt) D u*                     RHS
 //   dp      = A^+ (b - mean b)                 pressure solve

@@ -1,9 +1,10 @@
 // smac_kernels.hip -- gfx950 kernels of the SMAC projection step (FP64 form).
 //
-//   predictor        k_predict<A>      per face of component A (MUSCL-minmod
-//                                      advection + variable-mu stress + old dp/dx);
+//   predictor        k_predict_rim, k_predict_inner   MUSCL-minmod advection +
+//                                      variable-mu stress + old dp/dx, walls or
+//                                      property arrays, also the two-way
+//                                      (CFD-DEM) form;
 //                    k_predict_tile    triply periodic one-phase grids (z-march);
-//                    k_predict_tw<A>   the two-way (CFD-DEM) form
 //   star BC          k_star_bc         wall faces of u*, v*, w*
 //   Poisson RHS      k_rhs, k_rhs_eps  b = -(1/dt) div u* (+ the volume-fraction form)
 //   PCG vectors      k_init_r, k_add_scalar, k_jacobi, k_copy_dot, k_sum,
@@ -26,128 +27,48 @@
 
 namespace smac {
 
-// grid: x = face index along i (block 64), y = j (block 4), z = k
-template <class BC, class PR, class MF, int A>
-__global__ __launch_bounds__(256) void k_predict(Geo g, Props P, Vel V, VofF M, const double* __restrict__ p,
-                                                 double* __restrict__ ustar, double dt) {
-  int lo[3] = {1, 1, 1}, hi[3] = {g.n[0], g.n[1], g.n[2]};
-  lo[A] = g.per[A] ? 1 : 2;
-  int i = lo[0] + (int)(blockIdx.x * 64 + threadIdx.x);
-  int j = lo[1] + (int)(blockIdx.y * 4 + threadIdx.y);
-  int k = lo[2] + (int)blockIdx.z;
-  if (i > hi[0] || j > hi[1] || k > hi[2]) return;
-  I3 q = mk(i, j, k);
-  ustar[IX(g, q)] = predict_face<BC, PR, MF, A>(g, P, V, M, p, q, dt);
-}
-
-// ------------------------------------------------------- two-way (CFD-DEM)
-// Mass flux of k_compute_mass_flux_from_alpha_flux_two_way
-// (CFD/G_SMACSolver_VoF.cu:2472-2557): mf = rho0 (eps_f u_f) + (rho1-rho0) F h/dt
-// on the faces 1..N+1 of axis E and 0 outside them, eps_f the t^{n+1/2}
-// volume fraction of the face -- the mean of its two cells, the inner cell on
-// faces 1 and N+1 (d_get_void_fraction_half_*face, 1954-1967). F enters when
-// a VoF transport preceded (M.F[E] != nullptr).
-struct MfEps {
-  template <int E>
-  static __device__ __forceinline__ double mf(const Geo& g, const VofF& M, I3 r, double fv) {
-    const int m = r.v[E];
-    if (m < 1 || m > g.n[E] + 1) return 0.0;
-    double ef;
-    if (m == 1) {
-      ef = M.eps_half[IX(g, r)];
-    } else if (m == g.n[E] + 1) {
-      ef = M.eps_half[IX(g, sh(r, E, -1))];
-    } else {
-      ef = 0.5 * (M.eps_half[IX(g, sh(r, E, -1))] + M.eps_half[IX(g, r)]);
-    }
-    const double q = ef * fv;
-    if (!M.F[E]) return g.rho0 * q;
-    return g.rho0 * q + M.drho * (M.F[E][IX(g, wr(g, r))] * M.hbydt[E]);
+// The faces of a grid with walls, or of a periodic one with properties in
+// arrays: the inner box 4..n-2 of every axis, whose stencils (two faces either
+// way) meet no wall and no wrap, and the rim around it. Both kernels read the
+// whole stencil before any branch; the rim's replaces the values at and beyond
+// the walls by selects and wraps the indices. Bound by the array reads of the
+// inner box (256x128x128 with properties and alpha flux: 244 us, 0.6 GB) and the
+// latency of the rim's x slabs, which take a line per face (87 us). Before, one
+// kernel per component with the boundary getters of the reference, each of whose
+// loads waits on the face type before it: 1250 us for the three; in all,
+// 96x48x80 160 -> 44 us, two-way 80x48x64 340 -> 52, 21x17x13 60 -> 13.
+// Every box with an inner part is split; one of up to RIM cells along an axis is
+// all rim.
+constexpr int IN_LO = 4, IN_HI = 2;  // inner cells: IN_LO .. n - IN_HI
+constexpr int RIM = IN_LO - 1 + IN_HI;
+// rim cell t of the n box: z slabs, then y slabs, then x slabs; on a box too
+// small to have an inner part every cell
+__device__ __forceinline__ bool rim_cell(const Geo& g, unsigned t, I3& q) {
+  const unsigned nx = (unsigned)g.n[0], ny = (unsigned)g.n[1], nz = (unsigned)g.n[2];
+  if (nx <= RIM || ny <= RIM || nz <= RIM) {
+    if (t >= nx * ny * nz) return false;
+    q = mk((int)(t % nx) + 1, (int)(t / nx % ny) + 1, (int)(t / (nx * ny)) + 1);
+    return true;
   }
-};
-
-// Cross viscous term of the two-way predictor: the stresses of visc_cross,
-// each weighted by the t^n volume fraction of its edge, the mean of the four
-// cells around the edge summed in memory (x-fastest) order
-// (CFD/G_SMACSolver.cu:1608-1623, 1826-1844, 2044-2062).
-template <class BC, class PR, int A, int B>
-__device__ __forceinline__ double visc_cross_tw(const Geo& g, const Props& P, const Vel& V, const EpsF& E, I3 q,
-                                                double v0) {
-  double vbm = BC::dir(g, V, A, B, q, -1);
-  double vbp = BC::dir(g, V, A, B, q, +1);
-  double wpp = BC::face(g, V, B, sh(q, B, +1));
-  double wmp = BC::face(g, V, B, sh(sh(q, B, +1), A, -1));
-  double wp0 = BC::face(g, V, B, q);
-  double wm0 = BC::face(g, V, B, sh(q, A, -1));
-  double mu_p = PR::mu_edge(g, P, B, wr(g, sh(q, B, +1)), wr(g, sh(sh(q, B, +1), A, -1)));
-  double t_p = mu_p * ((wpp - wmp) * g.inv_d[A] + (vbp - v0) * g.inv_d[B]);
-  double mu_m = PR::mu_edge(g, P, B, wr(g, q), wr(g, sh(q, A, -1)));
-  double t_m = mu_m * ((wp0 - wm0) * g.inv_d[A] + (v0 - vbm) * g.inv_d[B]);
-  const double* eo = E.eps_old;
-  const I3 qa = sh(q, A, -1);
-  double ep, em;
-  if (B > A) {
-    ep = 0.25 * (eo[IX(g, qa)] + eo[IX(g, q)] + eo[IX(g, sh(qa, B, +1))] + eo[IX(g, sh(q, B, +1))]);
-    em = 0.25 * (eo[IX(g, sh(qa, B, -1))] + eo[IX(g, sh(q, B, -1))] + eo[IX(g, qa)] + eo[IX(g, q)]);
+  auto slab = [](unsigned s, unsigned n) { return (int)(s < IN_LO - 1 ? 1 + s : n - RIM + 1 + s); };
+  const unsigned cz = RIM * nx * ny, cy = RIM * nx * (nz - RIM), cx = RIM * (ny - RIM) * (nz - RIM);
+  if (t < cz) {
+    q = mk((int)(t % nx) + 1, (int)(t / nx % ny) + 1, slab(t / (nx * ny), nz));
+  } else if ((t -= cz) < cy) {
+    q = mk((int)(t % nx) + 1, slab(t / nx % RIM, ny), (int)(t / (nx * RIM)) + IN_LO);
+  } else if ((t -= cy) < cx) {
+    q = mk(slab(t % RIM, nx), (int)(t / RIM % (ny - RIM)) + IN_LO, (int)(t / (RIM * (ny - RIM))) + IN_LO);
   } else {
-    ep = 0.25 * (eo[IX(g, qa)] + eo[IX(g, sh(qa, B, +1))] + eo[IX(g, q)] + eo[IX(g, sh(q, B, +1))]);
-    em = 0.25 * (eo[IX(g, sh(qa, B, -1))] + eo[IX(g, qa)] + eo[IX(g, sh(q, B, -1))] + eo[IX(g, q)]);
+    return false;
   }
-  return (ep * t_p - em * t_m) * g.inv_d[B];
+  return true;
 }
-
-// One component of k_get_vof_vstar_rhouu_consistent_{x,y,z}_two_way
-// (CFD/G_SMACSolver.cu:1538-2194): the one-fluid predictor of predict_face
-// with the stresses weighted by the t^n volume fraction (cell values for the
-// own-direction stress, edge means for the cross stresses), the mass flux of
-// MfEps, the old pressure gradient weighted by the face mean of eps^n, and
-//   u* = (beta/eps^{n+1}_f) (eps^n_f rho^n_f u + dt tmp + J/V) + dt g
-// with J the particles' momentum impulse on the face. The IBM solid fraction
-// factor (1 - 0) of the reference is 1.
-template <class BC, class PR, class MF, int A>
-__device__ double predict_face_tw(const Geo& g, const Props& P, const Vel& V, const VofF& M, const EpsF& E,
-                                  const double* __restrict__ p, I3 q, double dt) {
-  constexpr int B1 = A == 0 ? 1 : 0;
-  constexpr int B2 = A == 2 ? 1 : 2;
-  double v0 = V.c[A][IX(g, q)];
-  double vp1 = BC::face(g, V, A, sh(q, A, +1));
-  double vm1 = BC::face(g, V, A, sh(q, A, -1));
-  const I3 cr = sh(q, A, -1);  // the minus cell at its raw index (volume fractions)
-  const I3 cm = wr(g, cr);
-  const double* eo = E.eps_old;
-
-  double tau_p = PR::mu(g, P, q) * (vp1 - v0);
-  double tau_m = PR::mu(g, P, cm) * (v0 - vm1);
-  double tmp = 2. * (eo[IX(g, q)] * tau_p - eo[IX(g, cr)] * tau_m) * g.inv_d2[A];
-  tmp += visc_cross_tw<BC, PR, A, B1>(g, P, V, E, q, v0);
-  tmp += visc_cross_tw<BC, PR, A, B2>(g, P, V, E, q, v0);
-  tmp -= conv_term<BC, MF, A, 0>(g, V, M, q, v0, vp1, vm1);
-  tmp -= conv_term<BC, MF, A, 1>(g, V, M, q, v0, vp1, vm1);
-  tmp -= conv_term<BC, MF, A, 2>(g, V, M, q, v0, vp1, vm1);
-
-  const double eo_f = 0.5 * (eo[IX(g, cr)] + eo[IX(g, q)]);
-  const double en_f = 0.5 * (E.eps[IX(g, cr)] + E.eps[IX(g, q)]);
-  tmp -= eo_f * (p[IX(g, q)] - p[IX(g, cm)]) * g.inv_d[A];
-  const double beta = PR::beta(g, P, A, q);
-  const double rho_old_f = PR::rho_old_f(g, P, q, cm);
-  const double jd = E.imp[A] ? E.imp[A][IX(g, q)] * E.inv_vol : 0.0;
-  const double inv_eps_rho = beta / en_f;
-  return inv_eps_rho * (eo_f * rho_old_f * v0 + dt * tmp + jd) + dt * g.g[A];
+static inline unsigned rim_cells(const Geo& g) {
+  const unsigned nx = (unsigned)g.n[0], ny = (unsigned)g.n[1], nz = (unsigned)g.n[2];
+  if (nx <= RIM || ny <= RIM || nz <= RIM) return nx * ny * nz;
+  return nx * ny * nz - (nx - RIM) * (ny - RIM) * (nz - RIM);
 }
-
-template <class BC, class PR, int A>
-__global__ __launch_bounds__(256) void k_predict_tw(Geo g, Props P, Vel V, VofF M, EpsF E,
-                                                    const double* __restrict__ p, double* __restrict__ ustar,
-                                                    double dt) {
-  int lo[3] = {1, 1, 1}, hi[3] = {g.n[0], g.n[1], g.n[2]};
-  lo[A] = g.per[A] ? 1 : 2;
-  int i = lo[0] + (int)(blockIdx.x * 64 + threadIdx.x);
-  int j = lo[1] + (int)(blockIdx.y * 4 + threadIdx.y);
-  int k = lo[2] + (int)blockIdx.z;
-  if (i > hi[0] || j > hi[1] || k > hi[2]) return;
-  I3 q = mk(i, j, k);
-  ustar[IX(g, q)] = predict_face_tw<BC, PR, MfEps, A>(g, P, V, M, E, p, q, dt);
-}
+static inline bool has_inner(const Geo& g) { return g.n[0] > RIM && g.n[1] > RIM && g.n[2] > RIM; }
 
 // Poisson face coefficients of a two-way grid (k_update_poisson_beta_two_way,
 // Coupling/G_CFDDEMCoupling.cu:419-455): on the faces 1..N+1 of axis A with
@@ -236,6 +157,248 @@ __device__ __forceinline__ double flux_minus(double m, const double c[5]) {
   double sl = minmod(dpv, dmv);
   int dir = sgn(m);
   return m * (uw + dir * 0.5 * sl);
+}
+
+// The value of a wall face of component a on side s (stored: the array's), as
+// get_face gives it
+__device__ __forceinline__ double wall_value(const Geo& g, int a, int s, double stored) {
+  const int bt = g.btype[s];
+  if (bt == BC_INFLOW) return (1. - 0.0) * g.bv[s][a];
+  if (bt == BC_OUTLET || (bt == BC_SLIP && a != 0)) return stored;
+  return 0.;
+}
+// Component a beyond the wall on side s of a tangential axis, next to the value
+// v, as get_dir gives it: both faces it averages lie on that side, so its wall
+// velocity is the side's
+__device__ __forceinline__ double wall_mirror(const Geo& g, int a, int s, double v) {
+  const int bt = g.btype[s];
+  return bt == BC_SLIP || bt == BC_OUTLET ? v : 2.0 * g.bv[s][a] - v;
+}
+
+// The convective flux through the + and the - side on the five values c[-2..2],
+// first-order where the upwind face is no interior one (flux_plus, flux_minus
+// with that case of conv_term)
+__device__ __forceinline__ double flux_plus_in(double m, const double c[5], bool in) {
+  const bool own = m > 0.;
+  const double uw = own ? c[2] : c[3];
+  const double sl = minmod(own ? c[3] - c[2] : c[4] - c[3], own ? c[2] - c[1] : c[3] - c[2]);
+  return m * (own || in ? uw + sgn(m) * 0.5 * sl : uw);
+}
+__device__ __forceinline__ double flux_minus_in(double m, const double c[5], bool in) {
+  const bool own = !(m > 0.);
+  const double uw = own ? c[2] : c[1];
+  const double sl = minmod(own ? c[3] - c[2] : c[2] - c[1], own ? c[2] - c[1] : c[1] - c[0]);
+  return m * (own || in ? uw + sgn(m) * 0.5 * sl : uw);
+}
+
+// The mass flux of a face
+enum MassFlux {
+  MF_RHO,  // rho0 u
+  MF_VOF,  // rho0 u + (rho1 - rho0) F h/dt (the alpha flux of a transport)
+  MF_EPS   // the two-way form (below)
+};
+// One face of component A of k_get_vof_vstar_rhouu_consistent_{x,y,z}
+// (CFD/G_SMACSolver.cu:139-392, 441-662, 763-1003), predict_face's terms in its
+// order; with MF_EPS of the two-way kernels (1538-2194): the stresses weighted
+// by the t^n volume fraction (cell values for the own-direction stress, the mean
+// of the four cells around the edge, summed in memory order, for the cross
+// stresses), the old pressure gradient by the face mean of eps^n, the mass flux
+// rho0 (eps_f u_f) + (rho1-rho0) F h/dt on the faces 1..N+1 of its axis and 0
+// outside them, eps_f the t^{n+1/2} volume fraction of the face -- the mean of its
+// two cells, the inner cell on faces 1 and N+1 (CFD/G_SMACSolver_VoF.cu:2472-2557,
+// 1954-1967) --, and u* = (beta/eps^{n+1}_f) (eps^n_f rho^n_f u + dt tmp + J/V) +
+// dt g with J the particles' momentum impulse on the face. Volume fractions are
+// read at the raw cell indices, ghosts included; the IBM solid fraction factor
+// (1 - 0) of the reference is 1.
+// VAR: properties from the arrays. RIM: the stencil may reach walls or wrap.
+template <int A, bool VAR, MassFlux MF, bool RIM_>
+__device__ __forceinline__ double face_direct(const Geo& g, const Props& P, const Vel& V, const VofF& M, const EpsF& E,
+                                              const double* __restrict__ p, I3 q, double dt) {
+  constexpr int B1 = A == 0 ? 1 : 0;
+  constexpr int B2 = A == 2 ? 1 : 2;
+  const long st[3] = {1, (long)g.px, (long)g.px * (long)g.py};
+  const size_t id = IX(g, q);
+  // array offsets of q + s e_d (wrapped on periodic axes; beyond a wall the
+  // array's own entries, whose values are replaced)
+  long off[3][5];
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int s = -2; s <= 2; s++) {
+      long o = s;
+      if (RIM_) {
+        if (g.per[d]) o = wrapi(q.v[d] + s, g.n[d]) - q.v[d];
+        else if (q.v[d] + s < 0) o = -q.v[d];
+      }
+      off[d][s + 2] = o * st[d];
+    }
+  auto at = [&](int d, int s) { return id + (size_t)off[d][s + 2]; };
+  auto at2 = [&](int d, int s, int e, int t) { return id + (size_t)(off[d][s + 2] + off[e][t + 2]); };
+  double c[3][5];  // component A along each axis
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int s = -2; s <= 2; s++) c[d][s + 2] = V.c[A][at(d, s)];
+  // component B on the faces around the edge: q + eB, q + eB - eA, q, q - eA
+  double wpp[3], wmp[3], wp0[3], wm0[3];
+#pragma unroll
+  for (int B = 0; B < 3; B++) {
+    if (B == A) continue;
+    const double* w = V.c[B];
+    wpp[B] = w[at(B, 1)];
+    wmp[B] = w[at2(B, 1, A, -1)];
+    wp0[B] = w[id];
+    wm0[B] = w[at(A, -1)];
+  }
+  bool inp[3] = {true, true, true}, inm[3] = {true, true, true};  // is q +- e_d an interior face?
+  if constexpr (RIM_) {
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      if (g.per[d]) continue;
+      const int x = q.v[d], n = g.n[d];
+      if (d == A) {
+        // own axis: faces 1 and n + 1 are the walls (the ghosts beyond are not used)
+        if (x == 2) c[d][1] = wall_value(g, A, 2 * d, c[d][1]);
+        if (x == 3) c[d][0] = wall_value(g, A, 2 * d, c[d][0]);
+        if (x == n) c[d][3] = wall_value(g, A, 2 * d + 1, c[d][3]);
+        if (x == n - 1) c[d][4] = wall_value(g, A, 2 * d + 1, c[d][4]);
+        inm[d] = x != 2;
+        inp[d] = x != n;
+      } else {
+        if (x == 1) c[d][1] = wall_mirror(g, A, 2 * d, c[d][2]);
+        if (x == 2) c[d][0] = wall_mirror(g, A, 2 * d, c[d][1]);
+        if (x == n) c[d][3] = wall_mirror(g, A, 2 * d + 1, c[d][2]);
+        if (x == n - 1) c[d][4] = wall_mirror(g, A, 2 * d + 1, c[d][3]);
+        inm[d] = x != 1;
+        inp[d] = x != n;
+        // component d on its own wall faces
+        if (x == 1) {
+          wp0[d] = wall_value(g, d, 2 * d, wp0[d]);
+          wm0[d] = wall_value(g, d, 2 * d, wm0[d]);
+        }
+        if (x == n) {
+          wpp[d] = wall_value(g, d, 2 * d + 1, wpp[d]);
+          wmp[d] = wall_value(g, d, 2 * d + 1, wmp[d]);
+        }
+      }
+    }
+  }
+  const double v0 = c[A][2];
+  const double rho0 = g.rho0;
+  // raw cell offsets (volume fractions)
+  const size_t rA = id - (size_t)st[A];
+  // mass flux of axis e at q + se e_e + sa e_A with face value v
+  auto mflux = [&](int e, int se, int sa, double v) -> double {
+    if constexpr (MF == MF_RHO) {
+      return rho0 * v;
+    } else {
+      const size_t r = e == A ? at(A, se) : at2(e, se, A, sa);
+      if constexpr (MF == MF_VOF) {
+        return rho0 * v + M.drho * (M.F[e][r] * M.hbydt[e]);
+      } else {
+        const size_t raw = id + (size_t)(se * st[e]) + (e == A ? 0 : (size_t)(sa * st[A]));
+        const int m = q.v[e] + se;  // 0 (a flux of 0) on a periodic axis: no cell before it
+        const double hi = M.eps_half[raw], lo = M.eps_half[raw - (RIM_ && m == 0 ? 0 : (size_t)st[e])];
+        double ef = 0.5 * (lo + hi);
+        if (RIM_ && m == 1) ef = hi;
+        if (RIM_ && m == g.n[e] + 1) ef = lo;
+        const double f = ef * v;
+        double mf = rho0 * f;
+        if (M.F[e]) mf = rho0 * f + M.drho * (M.F[e][r] * M.hbydt[e]);
+        if (RIM_ && (m < 1 || m > g.n[e] + 1)) mf = 0.0;
+        return mf;
+      }
+    }
+  };
+  constexpr bool TW = MF == MF_EPS;
+  const double* eo = E.eps_old;
+  double tmp;
+  {
+    const double mup = VAR ? P.mu[id] : g.mu0, mum = VAR ? P.mu[at(A, -1)] : g.mu0;
+    const double tau_p = mup * (c[A][3] - v0);
+    const double tau_m = mum * (v0 - c[A][1]);
+    if constexpr (TW) tmp = 2. * (eo[id] * tau_p - eo[rA] * tau_m) * g.inv_d2[A];
+    else tmp = 2. * (tau_p - tau_m) * g.inv_d2[A];
+  }
+  double mp[3], mm[3];
+  {
+    const double f0 = mflux(A, 0, 0, c[A][2]), fp = mflux(A, 1, 0, c[A][3]), fm = mflux(A, -1, 0, c[A][1]);
+    mp[A] = 0.5 * (f0 + fp);
+    mm[A] = 0.5 * (fm + f0);
+  }
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int B = e == 0 ? B1 : B2;
+    double mu_p = 0.5 * (g.mu0 + g.mu0), mu_m = mu_p;
+    if constexpr (VAR) {
+      mu_p = 0.5 * (P.muf[B][at(B, 1)] + P.muf[B][at2(B, 1, A, -1)]);
+      mu_m = 0.5 * (P.muf[B][id] + P.muf[B][at(A, -1)]);
+    }
+    const double t_p = mu_p * ((wpp[B] - wmp[B]) * g.inv_d[A] + (c[B][3] - v0) * g.inv_d[B]);
+    const double t_m = mu_m * ((wp0[B] - wm0[B]) * g.inv_d[A] + (v0 - c[B][1]) * g.inv_d[B]);
+    if constexpr (TW) {
+      const size_t sB = (size_t)st[B];
+      double ep, em;
+      if (B > A) {
+        ep = 0.25 * (eo[rA] + eo[id] + eo[rA + sB] + eo[id + sB]);
+        em = 0.25 * (eo[rA - sB] + eo[id - sB] + eo[rA] + eo[id]);
+      } else {
+        ep = 0.25 * (eo[rA] + eo[rA + sB] + eo[id] + eo[id + sB]);
+        em = 0.25 * (eo[rA - sB] + eo[rA] + eo[id - sB] + eo[id]);
+      }
+      tmp += (ep * t_p - em * t_m) * g.inv_d[B];
+    } else {
+      tmp += (t_p - t_m) * g.inv_d[B];
+    }
+    mp[B] = 0.5 * (mflux(B, 1, -1, wmp[B]) + mflux(B, 1, 0, wpp[B]));
+    mm[B] = 0.5 * (mflux(B, 0, 0, wp0[B]) + mflux(B, 0, -1, wm0[B]));
+  }
+#pragma unroll
+  for (int e = 0; e < 3; e++) {
+    const double Mp = RIM_ ? flux_plus_in(mp[e], c[e], inp[e]) : flux_plus(mp[e], c[e]);
+    const double Mm = RIM_ ? flux_minus_in(mm[e], c[e], inm[e]) : flux_minus(mm[e], c[e]);
+    tmp -= (Mp - Mm) * g.inv_d[e];
+  }
+  const size_t cm = at(A, -1);
+  const double beta = VAR ? P.beta[A][id] : g.beta0;
+  const double rho_old_f = VAR ? 0.5 * (P.rho_old[id] + P.rho_old[cm]) : 0.5 * (rho0 + rho0);
+  if constexpr (TW) {
+    const double eo_f = 0.5 * (eo[rA] + eo[id]);
+    const double en_f = 0.5 * (E.eps[rA] + E.eps[id]);
+    tmp -= eo_f * (p[id] - p[cm]) * g.inv_d[A];
+    const double jd = E.imp[A] ? E.imp[A][id] * E.inv_vol : 0.0;
+    const double inv_eps_rho = beta / en_f;
+    return inv_eps_rho * (eo_f * rho_old_f * v0 + dt * tmp + jd) + dt * g.g[A];
+  } else {
+    tmp -= (p[id] - p[cm]) * g.inv_d[A];
+    return beta * (v0 * rho_old_f) + dt * (beta * tmp + g.g[A]);
+  }
+}
+template <bool VAR, MassFlux MF>
+__global__ __launch_bounds__(256) void k_predict_inner(Geo g, Props P, Vel V, VofF M, EpsF E,
+                                                       const double* __restrict__ p, double* __restrict__ us0,
+                                                       double* __restrict__ us1, double* __restrict__ us2, double dt) {
+  const I3 q = mk(IN_LO + (int)(blockIdx.x * 64 + threadIdx.x), IN_LO + (int)(blockIdx.y * 4 + threadIdx.y),
+                  IN_LO + (int)blockIdx.z);
+  if (q.v[0] > g.n[0] - IN_HI || q.v[1] > g.n[1] - IN_HI) return;
+  const size_t id = IX(g, q);
+  us0[id] = face_direct<0, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+  us1[id] = face_direct<1, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+  us2[id] = face_direct<2, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+}
+// blockIdx.y: the component
+template <bool VAR, MassFlux MF>
+__global__ __launch_bounds__(256) void k_predict_rim(Geo g, Props P, Vel V, VofF M, EpsF E,
+                                                     const double* __restrict__ p, double* __restrict__ us0,
+                                                     double* __restrict__ us1, double* __restrict__ us2, double dt) {
+  I3 q;
+  if (!rim_cell(g, blockIdx.x * 256 + threadIdx.x, q)) return;
+  const int a = (int)blockIdx.y;
+  if (!g.per[a] && (a == 0 ? q.v[0] : (a == 1 ? q.v[1] : q.v[2])) < 2) return;  // wall face 1
+  const size_t id = IX(g, q);
+  if (a == 0) us0[id] = face_direct<0, VAR, MF, true>(g, P, V, M, E, p, q, dt);
+  else if (a == 1) us1[id] = face_direct<1, VAR, MF, true>(g, P, V, M, E, p, q, dt);
+  else us2[id] = face_direct<2, VAR, MF, true>(g, P, V, M, E, p, q, dt);
 }
 
 // ld(c, di, dj, dk) = component c (0..2 = u, v, w; 3 = p) at (i+di, j+dj, k+dk)
@@ -1896,18 +2059,14 @@ void launch_props(const Geo& g, const double* alpha, double* rho, double* rho_ol
   hipLaunchKernelGGL(k_props_faces<2>, fg, CELLB, 0, st, g, rho, mu, beta[2], muf[2]);
 }
 
-template <class BC, class PR, class MF>
-static void predict_components(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p,
-                               double* us[3], double dt, hipStream_t st) {
-  for (int a = 0; a < 3; a++) {
-    int lo = g.per[a] ? 1 : 2;
-    int nf[3] = {g.n[0], g.n[1], g.n[2]};
-    nf[a] = g.n[a] - lo + 1;
-    if (nf[0] <= 0 || nf[1] <= 0 || nf[2] <= 0) continue;
-    dim3 cg((unsigned)((nf[0] + 63) / 64), (unsigned)((nf[1] + 3) / 4), (unsigned)nf[2]);
-    if (a == 0) hipLaunchKernelGGL((k_predict<BC, PR, MF, 0>), cg, CELLB, 0, st, g, P, V, M, p, us[0], dt);
-    if (a == 1) hipLaunchKernelGGL((k_predict<BC, PR, MF, 1>), cg, CELLB, 0, st, g, P, V, M, p, us[1], dt);
-    if (a == 2) hipLaunchKernelGGL((k_predict<BC, PR, MF, 2>), cg, CELLB, 0, st, g, P, V, M, p, us[2], dt);
+template <bool VAR, MassFlux MF>
+static void predict_faces(const Geo& g, const Props& P, const Vel& V, const VofF& M, const EpsF& E, const double* p,
+                          double* us[3], double dt, hipStream_t st) {
+  hipLaunchKernelGGL((k_predict_rim<VAR, MF>), dim3((rim_cells(g) + 255) / 256, 3), dim3(256), 0, st, g, P, V, M, E, p,
+                     us[0], us[1], us[2], dt);
+  if (has_inner(g)) {
+    const dim3 grid((unsigned)((g.n[0] - RIM + 63) / 64), (unsigned)((g.n[1] - RIM + 3) / 4), (unsigned)(g.n[2] - RIM));
+    hipLaunchKernelGGL((k_predict_inner<VAR, MF>), grid, CELLB, 0, st, g, P, V, M, E, p, us[0], us[1], us[2], dt);
   }
 }
 
@@ -1918,12 +2077,10 @@ void launch_predict(const Geo& g, const Props* P, const Vel& V, const double* p,
   const VofF M0{};
   if (P && M) {
     // two-phase grids right after a VoF transport: mass flux with the alpha flux
-    if (allper) predict_components<PeriodicBC, VarP, MfVof>(g, *P, V, *M, p, us, dt, st);
-    else predict_components<WallBC, VarP, MfVof>(g, *P, V, *M, p, us, dt, st);
+    predict_faces<true, MF_VOF>(g, *P, V, *M, EpsF{}, p, us, dt, st);
   } else if (P) {
-    // two-phase grids: one kernel per component, properties from the arrays
-    if (allper) predict_components<PeriodicBC, VarP, MfRho0>(g, *P, V, M0, p, us, dt, st);
-    else predict_components<WallBC, VarP, MfRho0>(g, *P, V, M0, p, us, dt, st);
+    // two-phase grids: properties from the arrays
+    predict_faces<true, MF_RHO>(g, *P, V, M0, EpsF{}, p, us, dt, st);
   } else if (allper && g.n[0] % PT_X == 0 && g.n[1] % PT_Y == 0 && g.n[2] >= 3) {
     const int KT = 32;  // z-planes per block column
     dim3 grid((unsigned)(g.n[0] / PT_X), (unsigned)(g.n[1] / PT_Y), (unsigned)((g.n[2] + KT - 1) / KT));
@@ -1934,8 +2091,7 @@ void launch_predict(const Geo& g, const Props* P, const Vel& V, const double* p,
     hipLaunchKernelGGL(k_predict_fused<PeriodicBC>, grid, CELLB, 0, st, g, V, p, us[0], us[1], us[2], dt, KC);
     return;
   } else {
-    // walls: one kernel per component (the fused wall kernel exceeds the register file)
-    predict_components<WallBC, UniP, MfRho0>(g, Props{}, V, M0, p, us, dt, st);
+    predict_faces<false, MF_RHO>(g, Props{}, V, M0, EpsF{}, p, us, dt, st);
   }
   if (allper) return;
   int m = g.n[0] > g.n[1] ? g.n[0] : g.n[1];
@@ -1949,27 +2105,8 @@ void launch_predict_two_way(const Geo& g, const Props* P, const Vel& V, const do
   const bool allper = g.per[0] && g.per[1] && g.per[2];
   VofF MM{};
   if (M) MM = *M;
-  const Props PP = P ? *P : Props{};
-  for (int a = 0; a < 3; a++) {
-    int lo = g.per[a] ? 1 : 2;
-    int nf[3] = {g.n[0], g.n[1], g.n[2]};
-    nf[a] = g.n[a] - lo + 1;
-    if (nf[0] <= 0 || nf[1] <= 0 || nf[2] <= 0) continue;
-    dim3 cg((unsigned)((nf[0] + 63) / 64), (unsigned)((nf[1] + 3) / 4), (unsigned)nf[2]);
-#define SMAC_TW(BCT, PRT, AX) \
-  hipLaunchKernelGGL((k_predict_tw<BCT, PRT, AX>), cg, CELLB, 0, st, g, PP, V, MM, E, p, us[AX], dt)
-#define SMAC_TW_A(BCT, PRT)              \
-  if (a == 0) SMAC_TW(BCT, PRT, 0);      \
-  else if (a == 1) SMAC_TW(BCT, PRT, 1); \
-  else SMAC_TW(BCT, PRT, 2);
-    if (allper) {
-      if (P) { SMAC_TW_A(PeriodicBC, VarP) } else { SMAC_TW_A(PeriodicBC, UniP) }
-    } else {
-      if (P) { SMAC_TW_A(WallBC, VarP) } else { SMAC_TW_A(WallBC, UniP) }
-    }
-#undef SMAC_TW_A
-#undef SMAC_TW
-  }
+  if (P) predict_faces<true, MF_EPS>(g, *P, V, MM, E, p, us, dt, st);
+  else predict_faces<false, MF_EPS>(g, Props{}, V, MM, E, p, us, dt, st);
   if (allper) return;
   int m = g.n[0] > g.n[1] ? g.n[0] : g.n[1];
   m = m > g.n[2] ? m : g.n[2];
