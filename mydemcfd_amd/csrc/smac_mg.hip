@@ -1688,99 +1688,107 @@ __global__ __launch_bounds__(256) void k_pinv_panel(double* __restrict__ M, doub
 }
 
 // x_i = (y_i - l_{i+1,i} x_{i+1} - ... - l_{n-1,i} x_{n-1}) / l_ii, i = n-1..0,
-// for the CB columns c = CB blockIdx.x + lane of wave 0 (n <= NM); waves 1..3
-// stage the next G rows of L^T and of y. The chain's operands are read two
-// chunks of 16 ahead and its products formed one chunk ahead, past the end of a
-// row into zeros, so that its steps are subtractions only; of the newest x only
-// x_{i+1}, kept in a register, is younger than the loads.
-template <int CB, int G, int NM>
+// for the CB columns c = CB blockIdx.x + lane of wave 0 (n <= NM). Bound by the
+// n^2/2 dependent subtractions of a column, which only wave 0 does: while it works
+// on row i, waves 1..3 form the products of row i-1 with x_{i+1}.. into LDS (two
+// to a 16-byte read, zeros past the end of the row) and read row i-2 of L^T; the
+// product with x_i, still in a register, is the chain's own. 480 cells 650 us (6 ns
+// a subtraction), 92 cells 67; with the products formed by the chain's wave a chunk
+// ahead 1380 and 102. Four columns a block: with 32 (8 at 480 cells) the helpers'
+// products of a row took longer than its chain (92 cells 93 us, 480 698).
+constexpr int PCB = 4;
+template <int NM>
 __global__ __launch_bounds__(256) void k_pinv_back(const double* __restrict__ LT, const double* __restrict__ cshift,
                                                    int n, int singular, double* __restrict__ out) {
-  constexpr int U = 16, ST = NM + 5 * U;
-  __shared__ double xs[ST * CB];
-  __shared__ double ls[2 * G * ST];
-  __shared__ double ys[2 * G * CB];
-  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
-  const int c = CB * (int)blockIdx.x + lane;
+  constexpr int CB = PCB, U = 16, ST = NM + 4 * U, H = 192, NU = (NM * CB + 4 * H - 1) / (4 * H) * 4;
+  __shared__ double xs[NM * CB];
+  __shared__ __attribute__((aligned(16))) double ps[2][ST * CB];
+  __shared__ double hs[2][CB + 2];  // y_i of the columns, l_ii, l_{i+1,i}
+  const int t = (int)threadIdx.x, cb = CB * (int)blockIdx.x;
   const size_t ld = 2 * (size_t)n;
-  for (int e = (int)threadIdx.x; e < ST * CB; e += 256) xs[e] = 0.0;
-  for (int e = (int)threadIdx.x; e < 2 * G * ST; e += 256) ls[e] = 0.0;
-  __syncthreads();
-  // group g holds the rows i = hi(g) .. hi(g)-G+1, hi(g) = n-1-G g (row i at
-  // slot hi - i); wave wi of nw takes every nw-th row
-  auto stage = [&](int g, int wi, int nw) {
-    const int hi = n - 1 - G * g;
-    double* lb = ls + (g & 1) * G * ST;
-    double* yb = ys + (g & 1) * G * CB;
-    for (int s = wi; s < G && hi - s >= 0; s += nw) {
-      const int i = hi - s;
-      const double* src = LT + (size_t)i * ld;
-      for (int k = i + lane; k < n; k += 256) {
-        double v[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = k + 64 * u < n ? src[k + 64 * u] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-          if (k + 64 * u < n) lb[s * ST + k + 64 * u] = v[u];
-      }
-    }
-    for (int e = 64 * wi + lane; e < G * CB; e += 64 * nw) {
-      const int i = hi - e / CB, r = CB * (int)blockIdx.x + e % CB;
-      // y_i of column r is 0 before its own row
-      yb[e] = i >= r && r < n && i >= 0 ? LT[(size_t)i * ld + n + r] : 0.0;
-    }
+  for (int e = t; e < 2 * ST * CB; e += 256) ps[0][e] = 0.0;
+  // operand q of hs of row i, and whether it is in the matrix (y_i of column c is
+  // 0 before its own row)
+  auto head = [&](int i, int q) {
+    const int c = cb + q < n ? cb + q : n - 1, j = i < 0 ? 0 : i;
+    return LT[(size_t)j * ld + (q < CB ? n + c : q - CB + j)];
   };
-  stage(0, w, 4);
+  auto head_in = [&](int i, int q) { return q < CB ? cb + q < n && i >= cb + q : q == CB || i + 1 < n; };
+  if (t >= 64 && t - 64 < CB + 2) 
+    hs[(n - 1) & 1][t - 64] = head_in(n - 1, t - 64) ? head(n - 1, t - 64) : 0.0;
   __syncthreads();
   const double corr = singular ? 1.0 / (*cshift * (double)n * (double)n) : 0.0;
-  const int ng = (n + G - 1) / G;
-  double xl = 0.0;  // x_{i+1}
-  for (int g = 0; g < ng; g++) {
-    if (w > 0) {
-      if (g + 1 < ng) stage(g + 1, w - 1, 3);
-    } else if (lane < CB) {
-      const int hi = n - 1 - G * g;
-      const double* yb = ys + (g & 1) * G * CB + lane;
-      for (int s = 0; s < G && hi - s >= 0; s++) {
-        const int i = hi - s;
-        const double* l = ls + (g & 1) * G * ST + s * ST + i;
-        const double* x = xs + i * CB + lane;
-        double a0[U], b0[U], a1[U], b1[U], p0[U], p1[U];
-        auto rd = [&](double* a, double* b, int k) {
+  const int w = t - 64;
+  double xl = 0.0;  // wave 0: x_{i+1}
+  double l[NU] = {}, hv = 0.0;  // waves 1..3: their operands of the row after the next
+  // term q = (k - r - 2) CB + column of row r, of terms(r); four at a time, past
+  // the last the last one again
+  auto terms = [&](int r) { return r < 0 ? 0 : (n - 2 - r) * CB; };
+  auto term = [&](int u, int m) { return w + H * u < m ? w + H * u : m - 1; };
+  auto rdl = [&](int r) {
+    const int m = terms(r);
+    const double* row = LT + (size_t)(r < 0 ? 0 : r) * ld + (r + 2);
 #pragma unroll
-          for (int u = 0; u < U; u++) {
-            a[u] = l[k + u];
-            b[u] = x[(k + u) * CB];
-          }
-        };
-        double acc = yb[s * CB];
-        auto mul = [&](double* p, const double* a, const double* b) {
+    for (int u0 = 0; u0 < NU; u0 += 4) {
+      if (H * u0 >= m) break;
 #pragma unroll
-          for (int u = 0; u < U; u++) p[u] = a[u] * b[u];
-        };
-        auto sub = [&](const double* p) {
+      for (int u = u0; u < u0 + 4; u++) l[u] = row[term(u, m) / CB];
+    }
+    if (w < CB + 2) hv = head(r, w);
+  };
+  if (w >= 0) rdl(n - 2);
+  for (int i = n - 1; i >= 0; i--) {
+    if (w >= 0) {
+      const int r = i - 1, m = terms(r);
+      double* p = ps[r & 1];
+      if (w < CB + 2) hs[r & 1][w] = head_in(r, w) ? hv : 0.0;
+      const double* x = xs + (r + 2) * CB;
 #pragma unroll
-          for (int u = 0; u < U; u++) acc -= p[u];
-        };
-        const double dii = l[0];
-        rd(a0, b0, 2);
-        rd(a1, b1, 2 + U);
-        acc -= l[1] * xl;  // i = n-1: l[1] is 0
-        mul(p0, a0, b0);
-        for (int k = 2; k < n - i; k += 2 * U) {
-          rd(a0, b0, k + 2 * U);
-          mul(p1, a1, b1);
-          sub(p0);
-          __builtin_amdgcn_sched_barrier(0);
-          rd(a1, b1, k + 3 * U);
-          mul(p0, a0, b0);
-          sub(p1);
-          __builtin_amdgcn_sched_barrier(0);
+      for (int u0 = 0; u0 < NU; u0 += 4) {
+        if (H * u0 >= m) break;
+        double xv[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) xv[u] = x[term(u0 + u, m)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int q = w + H * (u0 + u), k = q / CB;
+          if (q < m) p[(k >> 1) * (2 * CB) + 2 * (q % CB) + (k & 1)] = l[u0 + u] * xv[u];
         }
-        xl = acc / dii;
-        xs[i * CB + lane] = xl;
-        if (c < n) out[(size_t)i * n + c] = singular ? xl - corr : xl;
       }
+      rdl(r - 1);
+    } else if (t < CB) {
+      const double2* p = (const double2*)ps[i & 1] + t;
+      const double* h = hs[i & 1];
+      double2 a[U / 2], b[U / 2];
+      auto rd = [&](double2* v, int k) {
+#pragma unroll
+        for (int u = 0; u < U / 2; u++) v[u] = p[(k / 2 + u) * CB];
+      };
+      double acc = h[t];
+      auto sub = [&](const double2* v) {
+#pragma unroll
+        for (int u = 0; u < U / 2; u++) {
+          acc -= v[u].x;
+          acc -= v[u].y;
+        }
+      };
+      const double dii = h[CB];
+      rd(a, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      rd(b, U);
+      __builtin_amdgcn_sched_barrier(0);
+      acc -= h[CB + 1] * xl;
+      for (int k = 0; k < n - 2 - i; k += 2 * U) {
+        sub(a);
+        rd(a, k + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        sub(b);
+        rd(b, k + 3 * U);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      xl = acc / dii;
+      xs[i * CB + t] = xl;
+      if (cb + t < n) out[(size_t)i * n + cb + t] = singular ? xl - corr : xl;
     }
     __syncthreads();
   }
@@ -1797,14 +1805,13 @@ void launch_dense_pinv(const Lv& C, int singular, double* work, double* out, hip
     const int ni = (2 * n - c1 + PB - 1) / PB, nj = c1 < n ? (n - c1 + PB - 1) / PB : 1;
     hipLaunchKernelGGL(k_pinv_panel, dim3((unsigned)ni, (unsigned)nj), dim3(256), 0, st, work, LT, n, c0);
   }
-  // the columns per wave and the rows staged ahead that fit the LDS
-#define SMAC_PBACK(CB, G, NM)                                                                                    \
-  hipLaunchKernelGGL((k_pinv_back<CB, G, NM>), dim3((unsigned)((n + CB - 1) / CB)), dim3(256), 0, st, LT, cs, n, \
-                     singular, out)
-  if (n <= 128) SMAC_PBACK(32, 16, 128);
-  else if (n <= 256) SMAC_PBACK(32, 8, 256);
-  else if (n <= 512) SMAC_PBACK(16, 8, 512);
-  else SMAC_PBACK(8, 4, 1024);
+#define SMAC_PBACK(NM)                                                                                              \
+  hipLaunchKernelGGL((k_pinv_back<NM>), dim3((unsigned)((n + PCB - 1) / PCB)), dim3(256), 0, st, LT, cs, n, singular, \
+                     out)
+  if (n <= 128) SMAC_PBACK(128);
+  else if (n <= 256) SMAC_PBACK(256);
+  else if (n <= 512) SMAC_PBACK(512);
+  else SMAC_PBACK(1024);
 #undef SMAC_PBACK
 }
 
