@@ -14,11 +14,13 @@
 //   pb   = pb' + dt D_i(beta ub*)
 //   ub   = (dF/du)^T ub*  (+ ub' on wall faces)
 // (dF/du)^T is formed face by face: each interior face re-evaluates its
-// predictor stencil with tracked loads (value, source array, index, factor)
-// and scatters the partial derivatives of the branch the forward took
-// (upwind side, minmod slope) with FP64 atomics into ub. Sums over the
+// predictor stencil, sums the partial derivatives of the branch the forward took
+// (upwind side, minmod slope) per entry read, and adds them with FP64 atomics to
+// a tile in LDS, whose finished planes go to ub with FP64 atomics. Sums over the
 // scatter are therefore order-dependent in the last bits; every other stage is
 // a deterministic gather.
+#include <type_traits>
+
 #include "smac_internal.hpp"
 #include "smac_predict.hpp"
 
@@ -27,80 +29,6 @@ namespace smac {
 namespace {
 
 constexpr dim3 CELLB_A(64, 4);
-
-// A loaded value with its linear dependence on one input: v = f * u_c[i] + const
-// (c < 0: constant).
-struct TV {
-  double v;
-  int c;
-  size_t i;
-  double f;
-};
-__device__ __forceinline__ TV tconst(double v) { return TV{v, -1, 0, 0.0}; }
-__device__ __forceinline__ TV tmem(const Vel& V, int c, size_t i) { return TV{V.c[c][i], c, i, 1.0}; }
-
-// tracked forms of the boundary getters (same values as get_face / get_dir);
-// Fwd is the forward policy with the same getters
-struct WallT {
-  using Fwd = WallBC;
-  static __device__ __forceinline__ TV face(const Geo& g, const Vel& V, int a, I3 q) {
-    q = wr(g, q);
-    int t = face_type(g, a, q);
-    if (t == F_INTERIOR) return tmem(V, a, IX(g, q));
-    if (t == F_BOUNDARY) {
-      int s = face_slot(g, a, q);
-      int bt = btype_of(g, s);
-      if (bt == BC_INFLOW) return tconst((1. - 0.0) * bv_of(g, s, a));
-      if (bt == BC_NOSLIP) return tconst(0.);
-      if (bt == BC_OUTLET) return tmem(V, a, IX(g, q));
-      if (bt == BC_SLIP && a != 0) return tmem(V, a, IX(g, q));
-    }
-    return tconst(0.);
-  }
-  static __device__ __forceinline__ TV dir(const Geo& g, const Vel& V, int a, int b, I3 q, int s) {
-    q = wr(g, q);
-    const size_t iq = IX(g, q);
-    double vin = V.c[a][iq];
-    I3 q2 = wr(g, sh(q, b, s));
-    if (face_type(g, a, q2) == F_INTERIOR) return tmem(V, a, IX(g, q2));
-    I3 qf = q;
-    qf.v[b] = s > 0 ? q.v[b] + 1 : q.v[b];
-    double vw = 0.0;
-    int count = 0;
-    if (face_type(g, b, qf) == F_BOUNDARY) {
-      vw += bv_of(g, face_slot(g, b, qf), a);
-      count++;
-    }
-    I3 qf2 = wr(g, sh(qf, a, -1));
-    if (face_type(g, b, qf2) == F_BOUNDARY) {
-      vw += bv_of(g, face_slot(g, b, qf2), a);
-      count++;
-    }
-    if (count > 0) vw /= (double)count;
-    int bt = btype_of(g, face_slot(g, b, qf));
-    if (bt == BC_SLIP || bt == BC_OUTLET) return TV{vin, a, iq, 1.0};
-    return TV{2.0 * vw - vin, a, iq, -1.0};
-  }
-  static __device__ __forceinline__ bool interior(const Geo& g, int a, I3 q) {
-    return face_type(g, a, wr(g, q)) == F_INTERIOR;
-  }
-};
-struct PeriodicT {
-  using Fwd = PeriodicBC;
-  static __device__ __forceinline__ I3 w3(const Geo& g, I3 q) {
-    q.v[0] = wrapi(q.v[0], g.n[0]);
-    q.v[1] = wrapi(q.v[1], g.n[1]);
-    q.v[2] = wrapi(q.v[2], g.n[2]);
-    return q;
-  }
-  static __device__ __forceinline__ TV face(const Geo& g, const Vel& V, int a, I3 q) {
-    return tmem(V, a, IX(g, w3(g, q)));
-  }
-  static __device__ __forceinline__ TV dir(const Geo& g, const Vel& V, int a, int b, I3 q, int s) {
-    return tmem(V, a, IX(g, w3(g, sh(q, b, s))));
-  }
-  static __device__ __forceinline__ bool interior(const Geo&, int, I3) { return true; }
-};
 
 struct Acc {
   double* ub[3];
@@ -115,30 +43,6 @@ struct AccV {
   double* an;
   double drho, dmu;
 };
-__device__ __forceinline__ void aadd(double* base, size_t i, double v) {
-  if (v != 0.0) unsafeAtomicAdd(base + i, v);
-}
-__device__ __forceinline__ void scat(const Acc& U, const TV& t, double c) {
-  if (t.c >= 0 && c != 0.0) {
-    // select chain: a dynamic index into the by-value argument would force a scratch copy
-    double* base = t.c == 0 ? U.ub[0] : (t.c == 1 ? U.ub[1] : U.ub[2]);
-    unsafeAtomicAdd(base + t.i, t.f * c);
-  }
-}
-// mass-flux face value of conv_term (MfRho0 or MfVof, the same expression)
-template <bool VOF, int E>
-__device__ __forceinline__ double mflux(const Geo& g, const VofF& M, I3 r, const TV& f) {
-  if constexpr (VOF) return g.rho0 * f.v + M.drho * (M.F[E][IX(g, wr(g, r))] * M.hbydt[E]);
-  return g.rho0 * f.v;
-}
-// cotangent c of a mass-flux face value: rho0 c to the velocity, (for VOF)
-// drho h/dt c to the accumulated alpha flux at r
-template <bool VOF, int E>
-__device__ __forceinline__ void mflux_bar(const Geo& g, const VofF& M, const AccV& AV, const Acc& U, I3 r,
-                                          const TV& f, double c) {
-  scat(U, f, g.rho0 * c);
-  if constexpr (VOF) aadd(AV.Fb[E], IX(g, wr(g, r)), M.drho * M.hbydt[E] * c);
-}
 
 // branch of minmod(dpv, dmv): 0 -> 0, 1 -> dpv, 2 -> dmv (d_minmod,
 // CFD/G_SMACSolver.cu:67-88)
@@ -147,208 +51,242 @@ __device__ __forceinline__ int minmod_sel(double dp, double dm) {
   return 0;
 }
 
-// adjoint of one side of the convective flux: M = m * (uw + sgn(m) 0.5 s),
-// m = 0.5 (mf(f0) + mf(f1)) with the mass-flux faces at r0, r1; cM = cotangent of M
-template <bool VOF, int E>
-__device__ __forceinline__ void flux_vjp(const Geo& g, const VofF& M, const AccV& AV, const Acc& U, I3 r0,
-                                         const TV& f0, I3 r1, const TV& f1, const TV& uw, bool slope, const TV& sa,
-                                         const TV& sb, const TV& sc, double cM) {
-  const double m = 0.5 * (mflux<VOF, E>(g, M, r0, f0) + mflux<VOF, E>(g, M, r1, f1));
-  double s = 0.0;
-  int sel = 0;
-  if (slope) {
-    const double dpv = sa.v - sb.v, dmv = sb.v - sc.v;
-    sel = minmod_sel(dpv, dmv);
-    s = sel == 1 ? dpv : (sel == 2 ? dmv : 0.0);
-  }
+// adjoint of M = m (uw + sgn(m) 0.5 s) of one side on the five values c: cM =
+// cotangent of M; to the values in cb; returns that of m. hi: the side's minus
+// value is c[hi-1], its plus value c[hi] (3 for the + side, 2 for the -); mine:
+// the upwind value is c[2]; slope: is its slope used?
+template <int HI>
+__device__ __forceinline__ double flux_vjp(double m, const double c[5], bool inner, double cM, double cb[5]) {
+  const bool low = m > 0.;  // the upwind value is c[HI-1], else c[HI]
+  const bool slope = (HI == 3 ? low : !low) || inner;
+  const double uw = low ? c[HI - 1] : c[HI];
+  const double dpv = low ? c[HI] - c[HI - 1] : c[HI + 1] - c[HI];
+  const double dmv = low ? c[HI - 1] - c[HI - 2] : c[HI] - c[HI - 1];
+  const int sel = slope ? minmod_sel(dpv, dmv) : 0;
+  const double s = sel == 1 ? dpv : (sel == 2 ? dmv : 0.0);
   const int dir = sgn(m);
-  const double up = uw.v + dir * 0.5 * s;
-  // dM/dm = up; dm/dmf0 = dm/dmf1 = 0.5
-  mflux_bar<VOF, E>(g, M, AV, U, r0, f0, 0.5 * up * cM);
-  mflux_bar<VOF, E>(g, M, AV, U, r1, f1, 0.5 * up * cM);
-  // dM/duw = m; dM/ds = m sgn(m) 0.5
-  scat(U, uw, m * cM);
+  const double up = uw + dir * 0.5 * s;
+  // dM/dm = up; dM/duw = m; dM/ds = m sgn(m) 0.5, s = sa - sb (1) or sb - sc (2)
   const double cs = m * dir * 0.5 * cM;
-  if (sel == 1) {  // s = sa - sb
-    scat(U, sa, cs);
-    scat(U, sb, -cs);
-  } else if (sel == 2) {  // s = sb - sc
-    scat(U, sb, cs);
-    scat(U, sc, -cs);
-  }
+  const double sa = sel == 1 ? cs : 0.0, sc = sel == 2 ? -cs : 0.0;
+  const double sb = m * cM + (sel == 1 ? -cs : (sel == 2 ? cs : 0.0));
+  cb[HI + 1] += low ? 0.0 : sa;
+  cb[HI] += low ? sa : sb;
+  cb[HI - 1] += low ? sb : sc;
+  cb[HI - 2] += low ? sc : 0.0;
+  return up * cM;
 }
 
-// adjoint of conv_term<BC, MF, A, E> scaled by cot (cotangent of the term)
-template <class BC, bool VOF, int A, int E>
-__device__ __forceinline__ void conv_vjp(const Geo& g, const Vel& V, const VofF& M, const AccV& AV, const Acc& U, I3 q,
-                                         const TV& v0, const TV& vp1, const TV& vm1, double cot) {
-  const double cE = cot * g.inv_d[E];  // d(term)/dMp = inv_d, d/dMm = -inv_d
-  if (E == A) {
-    const I3 qp = sh(q, A, +1), qm = sh(q, A, -1);
-    const TV fa0 = BC::face(g, V, A, q), fap = BC::face(g, V, A, qp), fam = BC::face(g, V, A, qm);
-    const double mp = 0.5 * (mflux<VOF, A>(g, M, q, fa0) + mflux<VOF, A>(g, M, qp, fap));
-    const double mm = 0.5 * (mflux<VOF, A>(g, M, qm, fam) + mflux<VOF, A>(g, M, q, fa0));
-    {
-      const I3 up = mp > 0. ? q : qp;
-      const bool in = BC::interior(g, A, up);
-      const TV uw = mp > 0. ? v0 : vp1;
-      TV sa = tconst(0.), sb = tconst(0.), sc = tconst(0.);
-      if (in) {
-        sa = BC::face(g, V, A, sh(up, A, +1));
-        sb = BC::face(g, V, A, up);
-        sc = BC::face(g, V, A, sh(up, A, -1));
-      }
-      flux_vjp<VOF, A>(g, M, AV, U, q, fa0, qp, fap, uw, in, sa, sb, sc, cE);
-    }
-    {
-      const I3 up = mm > 0. ? qm : q;
-      const bool in = BC::interior(g, A, up);
-      const TV uw = mm > 0. ? vm1 : v0;
-      TV sa = tconst(0.), sb = tconst(0.), sc = tconst(0.);
-      if (in) {
-        sa = BC::face(g, V, A, sh(up, A, +1));
-        sb = BC::face(g, V, A, up);
-        sc = BC::face(g, V, A, sh(up, A, -1));
-      }
-      flux_vjp<VOF, A>(g, M, AV, U, qm, fam, q, fa0, uw, in, sa, sb, sc, -cE);
-    }
-  } else {
-    const TV vcm = BC::dir(g, V, A, E, q, -1), vcp = BC::dir(g, V, A, E, q, +1);
-    const I3 r1 = sh(sh(q, E, +1), A, -1), r2 = sh(q, E, +1), r3 = sh(q, A, -1);
-    const TV e1 = BC::face(g, V, E, r1), e2 = BC::face(g, V, E, r2);
-    const TV e3 = BC::face(g, V, E, q), e4 = BC::face(g, V, E, r3);
-    const double mp = 0.5 * (mflux<VOF, E>(g, M, r1, e1) + mflux<VOF, E>(g, M, r2, e2));
-    const double mm = 0.5 * (mflux<VOF, E>(g, M, q, e3) + mflux<VOF, E>(g, M, r3, e4));
-    {
-      const I3 upw = wr(g, mp > 0. ? q : sh(q, E, +1));
-      const bool in = BC::interior(g, A, upw);
-      const TV uw = mp > 0. ? v0 : vcp;
-      TV sa = tconst(0.), sb = tconst(0.), sc = tconst(0.);
-      if (in) {
-        sb = tmem(V, A, IX(g, upw));
-        sa = BC::dir(g, V, A, E, upw, +1);
-        sc = BC::dir(g, V, A, E, upw, -1);
-      }
-      flux_vjp<VOF, E>(g, M, AV, U, r1, e1, r2, e2, uw, in, sa, sb, sc, cE);
-    }
-    {
-      const I3 upw = wr(g, mm > 0. ? sh(q, E, -1) : q);
-      const bool in = BC::interior(g, A, upw);
-      const TV uw = mm > 0. ? vcm : v0;
-      TV sa = tconst(0.), sb = tconst(0.), sc = tconst(0.);
-      if (in) {
-        sb = tmem(V, A, IX(g, upw));
-        sa = BC::dir(g, V, A, E, upw, +1);
-        sc = BC::dir(g, V, A, E, upw, -1);
-      }
-      flux_vjp<VOF, E>(g, M, AV, U, q, e3, r3, e4, uw, in, sa, sb, sc, -cE);
-    }
-  }
-}
-
-// cotangent c of the face viscosity muf[B] at f (VOF): to the cells it is
-// formed from (k_props_faces: the mean of its two cells on an interior face,
-// the inner cell on a boundary face), then to alpha^{n+1} with dmu
-__device__ __forceinline__ void mu_face_bar(const Geo& g, const AccV& AV, int B, I3 f, double c) {
-  f = wr(g, f);
-  const int t = face_type(g, B, f);
-  if (t == F_INTERIOR) {
-    aadd(AV.anp1, IX(g, f), AV.dmu * (0.5 * c));
-    aadd(AV.anp1, IX(g, wr(g, sh(f, B, -1))), AV.dmu * (0.5 * c));
-  } else if (t == F_BOUNDARY) {
-    aadd(AV.anp1, IX(g, f.v[B] == 1 ? f : sh(f, B, -1)), AV.dmu * c);
-  }
-}
-
-// adjoint of visc_cross<BC, PR, A, B> scaled by cot (VOF: and of its edge
-// viscosities)
-template <class BC, class PR, bool VOF, int A, int B>
-__device__ __forceinline__ void visc_vjp(const Geo& g, const Props& P, const Vel& V, const Acc& U, const AccV& AV, I3 q,
-                                         const TV& v0, double cot) {
-  const TV vbm = BC::dir(g, V, A, B, q, -1), vbp = BC::dir(g, V, A, B, q, +1);
-  const TV wpp = BC::face(g, V, B, sh(q, B, +1)), wmp = BC::face(g, V, B, sh(sh(q, B, +1), A, -1));
-  const TV wp0 = BC::face(g, V, B, q), wm0 = BC::face(g, V, B, sh(q, A, -1));
-  const double mu_p = PR::mu_edge(g, P, B, wr(g, sh(q, B, +1)), wr(g, sh(sh(q, B, +1), A, -1)));
-  const double mu_m = PR::mu_edge(g, P, B, wr(g, q), wr(g, sh(q, A, -1)));
-  const double c = cot * g.inv_d[B];  // cotangent of t_p; -c of t_m
-  scat(U, wpp, c * mu_p * g.inv_d[A]);
-  scat(U, wmp, -c * mu_p * g.inv_d[A]);
-  scat(U, vbp, c * mu_p * g.inv_d[B]);
-  scat(U, v0, -c * mu_p * g.inv_d[B]);
-  scat(U, wp0, -c * mu_m * g.inv_d[A]);
-  scat(U, wm0, c * mu_m * g.inv_d[A]);
-  scat(U, v0, -c * mu_m * g.inv_d[B]);
-  scat(U, vbm, c * mu_m * g.inv_d[B]);
-  if constexpr (VOF) {
-    // t_p = mu_p X_p with mu_p = 0.5 (muf(f1) + muf(f2)); t_m likewise
-    const double xp = (wpp.v - wmp.v) * g.inv_d[A] + (vbp.v - v0.v) * g.inv_d[B];
-    const double xm = (wp0.v - wm0.v) * g.inv_d[A] + (v0.v - vbm.v) * g.inv_d[B];
-    mu_face_bar(g, AV, B, sh(q, B, +1), 0.5 * c * xp);
-    mu_face_bar(g, AV, B, sh(sh(q, B, +1), A, -1), 0.5 * c * xp);
-    mu_face_bar(g, AV, B, q, -0.5 * c * xm);
-    mu_face_bar(g, AV, B, sh(q, A, -1), -0.5 * c * xm);
-  }
-}
-
-// (d u*_A(q) / d u^n)^T w, scattered into U (the pressure term is separate).
+// (d u*_A(q) / d u^n)^T w (the pressure term is separate): addu(c, d, s, r, v)
+// adds v to component c at q + s e_d + r e_A, once per entry; an axis is finished
+// before the next, so that few sums are held at a time.
 // VOF: the step after a VoF transport -- mass flux with the accumulated alpha
-// flux (its cotangent to AV.Fb) and the property cotangents: beta = 1/rho_f
-// and mu of alpha^{n+1}, rho_old of alpha^n
-template <class BC, class PR, bool VOF, int A>
-__device__ void predict_face_vjp(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p,
-                                 const Acc& U, const AccV& AV, I3 q, double dt, double w) {
-  constexpr int B1 = A == 0 ? 1 : 0;
-  constexpr int B2 = A == 2 ? 1 : 2;
-  const TV v0 = tmem(V, A, IX(g, q));
-  const TV vp1 = BC::face(g, V, A, sh(q, A, +1));
-  const TV vm1 = BC::face(g, V, A, sh(q, A, -1));
-  const I3 cm = wr(g, sh(q, A, -1));
-  const double beta = PR::beta(g, P, A, q);
-  const double rho_old_f = PR::rho_old_f(g, P, q, cm);
+// flux and the property cotangents: beta = 1/rho_f and mu of alpha^{n+1},
+// rho_old of alpha^n; addq(f, d, s, r, v) likewise, f = the axis of the flux, 3 =
+// alpha^{n+1}, 4 = alpha^n
+template <int A, bool VAR, bool VOF, bool RIM, class AddU, class AddQ>
+__device__ __forceinline__ void face_vjp(const Geo& g, const Props& P, const VofF& M, const AccV& AV, const double* p,
+                                         const Face<A, RIM>& F, double dt, double w, AddU addu, AddQ addq) {
+  constexpr MassFlux MF = VOF ? MF_VOF : MF_RHO;
+  const double v0 = F.c[A][2], beta = F.template beta<VAR>(g, P), rho_old_f = F.template rho_old<VAR>(g, P);
+  double mp[3], mm[3];
+  F.template mass<MF>(g, M, mp, mm);
   // u* = beta (v0 rho_old_f) + dt (beta tmp + g)
-  scat(U, v0, beta * rho_old_f * w);
-  const double W = dt * beta * w;  // cotangent of tmp
-  const double muq = PR::mu(g, P, q), mucm = PR::mu(g, P, cm);
+  double c0 = beta * rho_old_f * w;  // cotangent of v0
+  const double W = dt * beta * w;    // cotangent of tmp
+  const double muq = VAR ? P.mu[F.id] : g.mu0, mucm = VAR ? P.mu[F.at(A, -1)] : g.mu0;
   const double k2 = 2. * g.inv_d2[A] * W;
-  scat(U, vp1, k2 * muq);
-  scat(U, v0, -k2 * muq - k2 * mucm);
-  scat(U, vm1, k2 * mucm);
-  visc_vjp<BC, PR, VOF, A, B1>(g, P, V, U, AV, q, v0, W);
-  visc_vjp<BC, PR, VOF, A, B2>(g, P, V, U, AV, q, v0, W);
-  conv_vjp<BC, VOF, A, 0>(g, V, M, AV, U, q, v0, vp1, vm1, -W);
-  conv_vjp<BC, VOF, A, 1>(g, V, M, AV, U, q, v0, vp1, vm1, -W);
-  conv_vjp<BC, VOF, A, 2>(g, V, M, AV, U, q, v0, vp1, vm1, -W);
+  double x0 = 0.0, xm = 0.0;  // cotangents of alpha^{n+1} in cells q and q - e_A
   if constexpr (VOF) {
-    const size_t iq = IX(g, q), ic = IX(g, cm);
     // beta = 1/(0.5 (rho_q + rho_cm)): d beta / d rho_c = -0.5 beta^2
-    const double tmp = predict_tmp<typename BC::Fwd, PR, MfVof, A>(g, P, V, M, p, q);
-    const double bb = w * (v0.v * rho_old_f + dt * tmp);
+    const double tmp = F.template bracket<VAR, MF>(g, P, M, nullptr, p, mp, mm);
+    const double bb = w * (v0 * rho_old_f + dt * tmp);
     const double kr = AV.drho * (-0.5 * beta * beta * bb);
-    aadd(AV.anp1, iq, kr);
-    aadd(AV.anp1, ic, kr);
-    // rho_old_f = 0.5 (rho_old_q + rho_old_cm)
-    const double ko = AV.drho * (0.5 * (w * beta * v0.v));
-    aadd(AV.an, iq, ko);
-    aadd(AV.an, ic, ko);
     // own-axis stresses mu_q (vp1 - v0) and mu_cm (v0 - vm1)
-    aadd(AV.anp1, iq, AV.dmu * (k2 * (vp1.v - v0.v)));
-    aadd(AV.anp1, ic, AV.dmu * (-k2 * (v0.v - vm1.v)));
+    x0 = kr + AV.dmu * (k2 * (F.c[A][3] - v0));
+    xm = kr + AV.dmu * (-k2 * (v0 - F.c[A][1]));
+    // rho_old_f = 0.5 (rho_old_q + rho_old_cm)
+    const double ko = AV.drho * (0.5 * (w * beta * v0));
+    addq(4, A, 0, 0, ko);
+    addq(4, A, 0, -1, ko);
+  }
+#pragma unroll
+  for (int B = 0; B < 3; B++) {
+    if (B == A) continue;
+    double mu_p, mu_m;
+    F.template mu_edge<VAR>(g, P, B, mu_p, mu_m);
+    const double k = W * g.inv_d[B];  // cotangent of t_p; -k of t_m
+    const double kp = k * mu_p, km = k * mu_m;
+    double c[5] = {0.0, km * g.inv_d[B], 0.0, kp * g.inv_d[B], 0.0};
+    c0 += -kp * g.inv_d[B] - km * g.inv_d[B];
+    // convection: -W (Mp - Mm) / h
+    const double bp = 0.5 * flux_vjp<3>(mp[B], F.c[B], F.inp[B], -k, c);
+    const double bm = 0.5 * flux_vjp<2>(mm[B], F.c[B], F.inm[B], k, c);
+    double wpp = kp * g.inv_d[A] + g.rho0 * bp, wmp = -kp * g.inv_d[A] + g.rho0 * bp;
+    double wp0 = -km * g.inv_d[A] + g.rho0 * bm, wm0 = km * g.inv_d[A] + g.rho0 * bm;
+    c0 += c[2];
+    const int x = F.q.v[B], n = g.n[B];
+    const bool wl = RIM && !g.per[B] && x == 1, wh = RIM && !g.per[B] && x == n;
+    if (RIM && !g.per[B]) {
+      // mirrored values pass their cotangent on, a wall's own are constants
+      const double fl = wall_even(g, 2 * B) ? 1.0 : -1.0, fh = wall_even(g, 2 * B + 1) ? 1.0 : -1.0;
+      if (x == n - 1) {
+        c[3] += fh * c[4];
+        c[4] = 0.0;
+      }
+      if (wh) {
+        c0 += fh * c[3];
+        c[3] = 0.0;
+        if (!wall_stored(g, B, 2 * B + 1)) wpp = wmp = 0.0;
+      }
+      if (x == 2) {
+        c[1] += fl * c[0];
+        c[0] = 0.0;
+      }
+      if (wl) {
+        c0 += fl * c[1];
+        c[1] = 0.0;
+        if (!wall_stored(g, B, 2 * B)) wp0 = wm0 = 0.0;
+      }
+    }
+    addu(A, B, -2, 0, c[0]);
+    addu(A, B, -1, 0, c[1]);
+    addu(A, B, 1, 0, c[3]);
+    addu(A, B, 2, 0, c[4]);
+    addu(B, B, 1, 0, wpp);
+    addu(B, B, 1, -1, wmp);
+    addu(B, B, 0, 0, wp0);
+    addu(B, B, 0, -1, wm0);
+    if constexpr (VOF) {
+      const double kf = M.drho * M.hbydt[B], fp = kf * bp, fm = kf * bm;
+      addq(B, B, 1, 0, fp);
+      addq(B, B, 1, -1, fp);
+      addq(B, B, 0, 0, fm);
+      addq(B, B, 0, -1, fm);
+      // mu_p = 0.5 (muf(q + e_B) + muf(q + e_B - e_A)), mu_m at q; muf is the mean
+      // of its two cells on an interior face, the inner cell on a boundary face
+      const double xp = AV.dmu * (0.5 * k * F.strain_p(g, B)), xq = AV.dmu * (-0.5 * k * F.strain_m(g, B));
+      const double both = (wh ? xp : 0.5 * xp) + (wl ? xq : 0.5 * xq);
+      x0 += both;
+      xm += both;
+      const double ap = wh ? 0.0 : 0.5 * xp, am = wl ? 0.0 : 0.5 * xq;
+      addq(3, B, 1, 0, ap);
+      addq(3, B, 1, -1, ap);
+      addq(3, B, -1, 0, am);
+      addq(3, B, -1, -1, am);
+    }
+  }
+  double c[5] = {0.0, k2 * mucm, 0.0, k2 * muq, 0.0};
+  const double k = W * g.inv_d[A];
+  const double bp = 0.5 * flux_vjp<3>(mp[A], F.c[A], F.inp[A], -k, c);
+  const double bm = 0.5 * flux_vjp<2>(mm[A], F.c[A], F.inm[A], k, c);
+  c[1] += g.rho0 * bm;
+  c[2] += g.rho0 * (bm + bp) + c0 - k2 * muq - k2 * mucm;
+  c[3] += g.rho0 * bp;
+  if (RIM && !g.per[A]) {
+    const int x = F.q.v[A], n = g.n[A];
+    const bool lo = wall_stored(g, A, 2 * A), hi = wall_stored(g, A, 2 * A + 1);
+    if (x == 2 && !lo) c[1] = 0.0;
+    if (x == 3 && !lo) c[0] = 0.0;
+    if (x == n && !hi) c[3] = 0.0;
+    if (x == n - 1 && !hi) c[4] = 0.0;
+  }
+#pragma unroll
+  for (int s = -2; s <= 2; s++) addu(A, A, s, 0, c[s + 2]);
+  if constexpr (VOF) {
+    const double kf = M.drho * M.hbydt[A];
+    addq(A, A, -1, 0, kf * bm);
+    addq(A, A, 0, 0, kf * (bm + bp));
+    addq(A, A, 1, 0, kf * bp);
+    addq(3, A, 0, 0, x0);
+    addq(3, A, 0, -1, xm);
   }
 }
 
-template <class BC, class PR, bool VOF, int A>
-__global__ __launch_bounds__(256) void k_predict_vjp(Geo g, Props P, Vel V, VofF M, const double* __restrict__ p,
-                                                     const double* __restrict__ wbar, Acc U, AccV AV, double dt) {
-  int lo[3] = {1, 1, 1}, hi[3] = {g.n[0], g.n[1], g.n[2]};
-  lo[A] = g.per[A] ? 1 : 2;
-  int i = lo[0] + (int)(blockIdx.x * 64 + threadIdx.x);
-  int j = lo[1] + (int)(blockIdx.y * 4 + threadIdx.y);
-  int k = lo[2] + (int)blockIdx.z;
-  if (i > hi[0] || j > hi[1] || k > hi[2]) return;
-  I3 q = mk(i, j, k);
-  const double w = wbar[IX(g, q)];
-  if (w == 0.0) return;
-  predict_face_vjp<BC, PR, VOF, A>(g, P, V, M, p, U, AV, q, dt, w);
+// (dF/du)^T ub*: a block marches a column of VX x VY cells through kc planes, the
+// three components side by side (four waves each). The cotangents are summed in
+// LDS, for the velocities in the five planes k-2 .. k+2 that plane k reaches, for
+// the VoF sinks in three; a finished plane goes out with one atomic per entry
+// touched. Each face's own sum over its ~50 partial derivatives is formed in
+// registers first (21 entries, with VOF 44). Bound by the latency of the stencil
+// reads and the LDS atomics: 128^3 204 us, 128x64x64 with VOF 182 us; one kernel
+// per component with a global atomic per partial derivative took 2300 and 2100.
+constexpr int VX = 64, VY = 4;
+template <bool VAR, bool VOF, bool RIM>
+__global__ __launch_bounds__(768) void k_predict_vjp(Geo g, Props P, Vel V, VofF M, const double* __restrict__ p,
+                                                     Vel wbar, Acc U, AccV AV, double dt, int kc) {
+  constexpr int PX = VX + 4, PL = PX * (VY + 4);  // velocity planes, two cells around
+  constexpr int QX = VX + 2, QL = QX * (VY + 2);  // VoF planes, one cell around
+  constexpr int NQ = VOF ? 3 * QL : 1;
+  __shared__ double su[3][5 * PL];
+  __shared__ double sf[VOF ? 5 : 1][NQ];  // Fb, anp1, an
+  const int t = (int)threadIdx.x;
+  const int x0 = 1 + VX * (int)blockIdx.x, y0 = 1 + VY * (int)blockIdx.y, z0 = 1 + kc * (int)blockIdx.z;
+  const int z1 = min(z0 + kc - 1, g.n[2]);
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), a = wv >> 2;
+  const int lx = t & 63, ly = wv & 3, i = x0 + lx, j = y0 + ly;
+  for (int e = t; e < 15 * PL; e += 768) su[0][e] = 0.0;
+  if constexpr (VOF)
+    for (int e = t; e < 5 * NQ; e += 768) sf[0][e] = 0.0;
+  // plane z of the velocity sums / of the VoF sums
+  auto pu = [&](int z) { return (z - z0 + 2) % 5 * PL; };
+  auto pq = [&](int z) { return (z - z0 + 1) % 3 * QL; };
+  auto face = [&](auto ac, int k) {
+    constexpr int A = decltype(ac)::value;
+    if (i > g.n[0] || j > g.n[1]) return;
+    const I3 q = mk(i, j, k);
+    if (!g.per[A] && q.v[A] < 2) return;
+    const double w = wbar.c[A][IX(g, q)];
+    if (w == 0.0) return;
+    const Face<A, RIM> F(g, V, q);
+    const int lo = ly * PX + lx, lq = ly * QX + lx;
+    auto addu = [&](int c, int d, int s, int r, double v) {
+      int o[3] = {0, 0, 0};
+      o[d] += s;
+      o[A] += r;
+      unsafeAtomicAdd(su[c] + pu(k + o[2]) + (o[1] + 2) * PX + (o[0] + 2) + lo, v);
+    };
+    auto addq = [&](int f, int d, int s, int r, double v) {
+      int o[3] = {0, 0, 0};
+      o[d] += s;
+      o[A] += r;
+      unsafeAtomicAdd(sf[f] + pq(k + o[2]) + (o[1] + 1) * QX + (o[0] + 1) + lq, v);
+    };
+    face_vjp<A, VAR, VOF, RIM>(g, P, M, AV, p, F, dt, w, addu, addq);
+  };
+  auto out = [&](double* base, double* s, int x, int y, int z) {
+    const double v = *s;
+    if (v == 0.0) return;
+    *s = 0.0;
+    unsafeAtomicAdd(base + idx(g, W(g, 0, x), W(g, 1, y), W(g, 2, z)), v);
+  };
+  auto flush_u = [&](int z) {
+    for (int e = t; e < 3 * PL; e += 768) {
+      const int c = e / PL, r = e - c * PL;
+      out(c == 0 ? U.ub[0] : (c == 1 ? U.ub[1] : U.ub[2]), su[c] + pu(z) + r, x0 - 2 + r % PX, y0 - 2 + r / PX, z);
+    }
+  };
+  auto flush_q = [&](int z) {
+    for (int e = t; e < 5 * QL; e += 768) {
+      const int f = e / QL, r = e - f * QL;
+      double* b = f == 0 ? AV.Fb[0] : (f == 1 ? AV.Fb[1] : (f == 2 ? AV.Fb[2] : (f == 3 ? AV.anp1 : AV.an)));
+      out(b, sf[f] + pq(z) + r, x0 - 1 + r % QX, y0 - 1 + r / QX, z);
+    }
+  };
+  for (int k = z0; k <= z1; k++) {
+    __syncthreads();
+    if (a == 0) face(std::integral_constant<int, 0>{}, k);
+    else if (a == 1) face(std::integral_constant<int, 1>{}, k);
+    else face(std::integral_constant<int, 2>{}, k);
+    __syncthreads();
+    flush_u(k - 2);
+    if constexpr (VOF) flush_q(k - 1);
+  }
+  for (int z = z1 - 1; z <= z1 + 2; z++) flush_u(z);
+  if constexpr (VOF) {
+    flush_q(z1);
+    flush_q(z1 + 1);
+  }
 }
 
 // out_c = pin_c + s * sum over the interior faces f of cell c of +-beta_f ub_f / h
@@ -423,22 +361,19 @@ __global__ __launch_bounds__(256) void k_rowsum_nat(Geo g, const double* __restr
   if (lane == 0) part0[row] = acc;
 }
 
-template <class BC, class PR, bool VOF>
-void predict_vjp_components(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p,
-                            double* const wbar[3], const Acc& U, const AccV& AV, double dt, hipStream_t st) {
-  for (int a = 0; a < 3; a++) {
-    int lo = g.per[a] ? 1 : 2;
-    int nf[3] = {g.n[0], g.n[1], g.n[2]};
-    nf[a] = g.n[a] - lo + 1;
-    if (nf[0] <= 0 || nf[1] <= 0 || nf[2] <= 0) continue;
-    dim3 cg((unsigned)((nf[0] + 63) / 64), (unsigned)((nf[1] + 3) / 4), (unsigned)nf[2]);
-    if (a == 0)
-      hipLaunchKernelGGL((k_predict_vjp<BC, PR, VOF, 0>), cg, CELLB_A, 0, st, g, P, V, M, p, wbar[0], U, AV, dt);
-    if (a == 1)
-      hipLaunchKernelGGL((k_predict_vjp<BC, PR, VOF, 1>), cg, CELLB_A, 0, st, g, P, V, M, p, wbar[1], U, AV, dt);
-    if (a == 2)
-      hipLaunchKernelGGL((k_predict_vjp<BC, PR, VOF, 2>), cg, CELLB_A, 0, st, g, P, V, M, p, wbar[2], U, AV, dt);
-  }
+// planes per block: at least VJP_BLOCKS blocks (two for each CU, which is what
+// their registers allow), as long as a block has four planes to share its edges
+constexpr unsigned VJP_BLOCKS = 512;
+template <bool VAR, bool VOF>
+void predict_vjp(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p, double* const wbar[3],
+                 const Acc& U, const AccV& AV, double dt, hipStream_t st) {
+  const unsigned bx = (unsigned)((g.n[0] + VX - 1) / VX), by = (unsigned)((g.n[1] + VY - 1) / VY);
+  int kc = 32;
+  while (kc > 4 && bx * by * (unsigned)((g.n[2] + kc - 1) / kc) < VJP_BLOCKS) kc /= 2;
+  Vel wb;
+  for (int d = 0; d < 3; d++) wb.c[d] = wbar[d];
+  hipLaunchKernelGGL((k_predict_vjp<VAR, VOF, true>), dim3(bx, by, (unsigned)((g.n[2] + kc - 1) / kc)), dim3(768), 0,
+                     st, g, P, V, M, p, wb, U, AV, dt, kc);
 }
 
 }  // namespace
@@ -449,14 +384,8 @@ void launch_predict_vjp(const Geo& g, const Props* P, const Vel& V, double* cons
   for (int d = 0; d < 3; d++) U.ub[d] = ub[d];
   const VofF M0{};
   const AccV AV0{};
-  const bool allper = g.per[0] && g.per[1] && g.per[2];
-  if (P) {
-    if (allper) predict_vjp_components<PeriodicT, VarP, false>(g, *P, V, M0, nullptr, wbar, U, AV0, dt, st);
-    else predict_vjp_components<WallT, VarP, false>(g, *P, V, M0, nullptr, wbar, U, AV0, dt, st);
-  } else {
-    if (allper) predict_vjp_components<PeriodicT, UniP, false>(g, Props{}, V, M0, nullptr, wbar, U, AV0, dt, st);
-    else predict_vjp_components<WallT, UniP, false>(g, Props{}, V, M0, nullptr, wbar, U, AV0, dt, st);
-  }
+  if (P) predict_vjp<true, false>(g, *P, V, M0, nullptr, wbar, U, AV0, dt, st);
+  else predict_vjp<false, false>(g, Props{}, V, M0, nullptr, wbar, U, AV0, dt, st);
 }
 
 void launch_predict_vjp_vof(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p,
@@ -472,9 +401,7 @@ void launch_predict_vjp_vof(const Geo& g, const Props& P, const Vel& V, const Vo
   AV.an = an;
   AV.drho = drho;
   AV.dmu = dmu;
-  const bool allper = g.per[0] && g.per[1] && g.per[2];
-  if (allper) predict_vjp_components<PeriodicT, VarP, true>(g, P, V, M, p, wbar, U, AV, dt, st);
-  else predict_vjp_components<WallT, VarP, true>(g, P, V, M, p, wbar, U, AV, dt, st);
+  predict_vjp<true, true>(g, P, V, M, p, wbar, U, AV, dt, st);
 }
 
 void launch_adj_div(const Geo& g, const BetaF* bf, double* const ub[3], const double* pin, double* out, double s,

@@ -235,32 +235,6 @@ struct Props {
   const double* muf[3];
 };
 
-// Property policies of the predictor and the correction. UniP: one phase,
-// constants from Geo (mu_f = 0.5(mu0+mu0), rho_f = 0.5(rho0+rho0), as the
-// face formulas give them); VarP: the arrays of Props.
-struct UniP {
-  static __device__ __forceinline__ double mu(const Geo& g, const Props&, I3) { return g.mu0; }
-  static __device__ __forceinline__ double mu_edge(const Geo& g, const Props&, int, I3, I3) {
-    return 0.5 * (g.mu0 + g.mu0);
-  }
-  static __device__ __forceinline__ double beta(const Geo& g, const Props&, int, I3) { return g.beta0; }
-  static __device__ __forceinline__ double rho_old_f(const Geo& g, const Props&, I3, I3) {
-    return 0.5 * (g.rho0 + g.rho0);
-  }
-};
-struct VarP {
-  static __device__ __forceinline__ double mu(const Geo& g, const Props& P, I3 c) { return P.mu[IX(g, c)]; }
-  static __device__ __forceinline__ double mu_edge(const Geo& g, const Props& P, int b, I3 f1, I3 f2) {
-    return 0.5 * (P.muf[b][IX(g, f1)] + P.muf[b][IX(g, f2)]);
-  }
-  static __device__ __forceinline__ double beta(const Geo& g, const Props& P, int a, I3 q) {
-    return P.beta[a][IX(g, q)];
-  }
-  static __device__ __forceinline__ double rho_old_f(const Geo& g, const Props& P, I3 q, I3 cm) {
-    return 0.5 * (P.rho_old[IX(g, q)] + P.rho_old[IX(g, cm)]);
-  }
-};
-
 // Storage traits of the multigrid vectors: storage type T, compute type C.
 // bf16 is kept as raw 16-bit words (upper half of an IEEE float), rounded to
 // nearest-even on store.

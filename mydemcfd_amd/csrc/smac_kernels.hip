@@ -97,12 +97,11 @@ __global__ __launch_bounds__(256) void k_pois_two_way(Geo g, const double* __res
   }
 }
 
-// Periodic one-phase form of predict_face<PeriodicBC, UniP, A> with the whole
-// stencil loaded before any branch: the own component at q + s e_d for
+// Periodic one-phase form of face_ustar: the own component at q + s e_d for
 // s = -2..2 along each axis, the two cross components on the four faces around
 // the edge, p on both sides. The upwind side and the minmod slope are then
 // register selects, so no load waits on another load's value. The arithmetic
-// is that of predict_face, term for term, so the results are bit-identical.
+// is that of face_ustar, term for term, so the results are bit-identical.
 struct PerIdx {
   int x[5], y[5], z[5];  // wrapped coordinates i-2..i+2, j-2..j+2, k-2..k+2
   int px, py;
@@ -124,256 +123,6 @@ __device__ __forceinline__ size_t per_at2(const PerIdx& X, int sb, int sa) {
   return X.at(o[0], o[1], o[2]);
 }
 
-// one side of the convective flux along E, MUSCL-minmod on the five values
-// c[-2..2] = u_A at q + s e_E (upwind side from the sign of m)
-__device__ __forceinline__ double flux_plus(double m, const double c[5]) {
-  // + face: up = q (c0) when m > 0, else q + e (c1)
-  double dpv, dmv, uw;
-  if (m > 0.) {
-    dpv = c[3] - c[2];
-    dmv = c[2] - c[1];
-    uw = c[2];
-  } else {
-    dpv = c[4] - c[3];
-    dmv = c[3] - c[2];
-    uw = c[3];
-  }
-  double sl = minmod(dpv, dmv);
-  int dir = sgn(m);
-  return m * (uw + dir * 0.5 * sl);
-}
-__device__ __forceinline__ double flux_minus(double m, const double c[5]) {
-  // - face: up = q - e (c-1) when m > 0, else q (c0)
-  double dpv, dmv, uw;
-  if (m > 0.) {
-    dpv = c[2] - c[1];
-    dmv = c[1] - c[0];
-    uw = c[1];
-  } else {
-    dpv = c[3] - c[2];
-    dmv = c[2] - c[1];
-    uw = c[2];
-  }
-  double sl = minmod(dpv, dmv);
-  int dir = sgn(m);
-  return m * (uw + dir * 0.5 * sl);
-}
-
-// The value of a wall face of component a on side s (stored: the array's), as
-// get_face gives it
-__device__ __forceinline__ double wall_value(const Geo& g, int a, int s, double stored) {
-  const int bt = g.btype[s];
-  if (bt == BC_INFLOW) return (1. - 0.0) * g.bv[s][a];
-  if (bt == BC_OUTLET || (bt == BC_SLIP && a != 0)) return stored;
-  return 0.;
-}
-// Component a beyond the wall on side s of a tangential axis, next to the value
-// v, as get_dir gives it: both faces it averages lie on that side, so its wall
-// velocity is the side's
-__device__ __forceinline__ double wall_mirror(const Geo& g, int a, int s, double v) {
-  const int bt = g.btype[s];
-  return bt == BC_SLIP || bt == BC_OUTLET ? v : 2.0 * g.bv[s][a] - v;
-}
-
-// The convective flux through the + and the - side on the five values c[-2..2],
-// first-order where the upwind face is no interior one (flux_plus, flux_minus
-// with that case of conv_term)
-__device__ __forceinline__ double flux_plus_in(double m, const double c[5], bool in) {
-  const bool own = m > 0.;
-  const double uw = own ? c[2] : c[3];
-  const double sl = minmod(own ? c[3] - c[2] : c[4] - c[3], own ? c[2] - c[1] : c[3] - c[2]);
-  return m * (own || in ? uw + sgn(m) * 0.5 * sl : uw);
-}
-__device__ __forceinline__ double flux_minus_in(double m, const double c[5], bool in) {
-  const bool own = !(m > 0.);
-  const double uw = own ? c[2] : c[1];
-  const double sl = minmod(own ? c[3] - c[2] : c[2] - c[1], own ? c[2] - c[1] : c[1] - c[0]);
-  return m * (own || in ? uw + sgn(m) * 0.5 * sl : uw);
-}
-
-// The mass flux of a face
-enum MassFlux {
-  MF_RHO,  // rho0 u
-  MF_VOF,  // rho0 u + (rho1 - rho0) F h/dt (the alpha flux of a transport)
-  MF_EPS   // the two-way form (below)
-};
-// One face of component A of k_get_vof_vstar_rhouu_consistent_{x,y,z}
-// (CFD/G_SMACSolver.cu:139-392, 441-662, 763-1003), predict_face's terms in its
-// order; with MF_EPS of the two-way kernels (1538-2194): the stresses weighted
-// by the t^n volume fraction (cell values for the own-direction stress, the mean
-// of the four cells around the edge, summed in memory order, for the cross
-// stresses), the old pressure gradient by the face mean of eps^n, the mass flux
-// rho0 (eps_f u_f) + (rho1-rho0) F h/dt on the faces 1..N+1 of its axis and 0
-// outside them, eps_f the t^{n+1/2} volume fraction of the face -- the mean of its
-// two cells, the inner cell on faces 1 and N+1 (CFD/G_SMACSolver_VoF.cu:2472-2557,
-// 1954-1967) --, and u* = (beta/eps^{n+1}_f) (eps^n_f rho^n_f u + dt tmp + J/V) +
-// dt g with J the particles' momentum impulse on the face. Volume fractions are
-// read at the raw cell indices, ghosts included; the IBM solid fraction factor
-// (1 - 0) of the reference is 1.
-// VAR: properties from the arrays. RIM: the stencil may reach walls or wrap.
-template <int A, bool VAR, MassFlux MF, bool RIM_>
-__device__ __forceinline__ double face_direct(const Geo& g, const Props& P, const Vel& V, const VofF& M, const EpsF& E,
-                                              const double* __restrict__ p, I3 q, double dt) {
-  constexpr int B1 = A == 0 ? 1 : 0;
-  constexpr int B2 = A == 2 ? 1 : 2;
-  const long st[3] = {1, (long)g.px, (long)g.px * (long)g.py};
-  const size_t id = IX(g, q);
-  // array offsets of q + s e_d (wrapped on periodic axes; beyond a wall the
-  // array's own entries, whose values are replaced)
-  long off[3][5];
-#pragma unroll
-  for (int d = 0; d < 3; d++)
-#pragma unroll
-    for (int s = -2; s <= 2; s++) {
-      long o = s;
-      if (RIM_) {
-        if (g.per[d]) o = wrapi(q.v[d] + s, g.n[d]) - q.v[d];
-        else if (q.v[d] + s < 0) o = -q.v[d];
-      }
-      off[d][s + 2] = o * st[d];
-    }
-  auto at = [&](int d, int s) { return id + (size_t)off[d][s + 2]; };
-  auto at2 = [&](int d, int s, int e, int t) { return id + (size_t)(off[d][s + 2] + off[e][t + 2]); };
-  double c[3][5];  // component A along each axis
-#pragma unroll
-  for (int d = 0; d < 3; d++)
-#pragma unroll
-    for (int s = -2; s <= 2; s++) c[d][s + 2] = V.c[A][at(d, s)];
-  // component B on the faces around the edge: q + eB, q + eB - eA, q, q - eA
-  double wpp[3], wmp[3], wp0[3], wm0[3];
-#pragma unroll
-  for (int B = 0; B < 3; B++) {
-    if (B == A) continue;
-    const double* w = V.c[B];
-    wpp[B] = w[at(B, 1)];
-    wmp[B] = w[at2(B, 1, A, -1)];
-    wp0[B] = w[id];
-    wm0[B] = w[at(A, -1)];
-  }
-  bool inp[3] = {true, true, true}, inm[3] = {true, true, true};  // is q +- e_d an interior face?
-  if constexpr (RIM_) {
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-      if (g.per[d]) continue;
-      const int x = q.v[d], n = g.n[d];
-      if (d == A) {
-        // own axis: faces 1 and n + 1 are the walls (the ghosts beyond are not used)
-        if (x == 2) c[d][1] = wall_value(g, A, 2 * d, c[d][1]);
-        if (x == 3) c[d][0] = wall_value(g, A, 2 * d, c[d][0]);
-        if (x == n) c[d][3] = wall_value(g, A, 2 * d + 1, c[d][3]);
-        if (x == n - 1) c[d][4] = wall_value(g, A, 2 * d + 1, c[d][4]);
-        inm[d] = x != 2;
-        inp[d] = x != n;
-      } else {
-        if (x == 1) c[d][1] = wall_mirror(g, A, 2 * d, c[d][2]);
-        if (x == 2) c[d][0] = wall_mirror(g, A, 2 * d, c[d][1]);
-        if (x == n) c[d][3] = wall_mirror(g, A, 2 * d + 1, c[d][2]);
-        if (x == n - 1) c[d][4] = wall_mirror(g, A, 2 * d + 1, c[d][3]);
-        inm[d] = x != 1;
-        inp[d] = x != n;
-        // component d on its own wall faces
-        if (x == 1) {
-          wp0[d] = wall_value(g, d, 2 * d, wp0[d]);
-          wm0[d] = wall_value(g, d, 2 * d, wm0[d]);
-        }
-        if (x == n) {
-          wpp[d] = wall_value(g, d, 2 * d + 1, wpp[d]);
-          wmp[d] = wall_value(g, d, 2 * d + 1, wmp[d]);
-        }
-      }
-    }
-  }
-  const double v0 = c[A][2];
-  const double rho0 = g.rho0;
-  // raw cell offsets (volume fractions)
-  const size_t rA = id - (size_t)st[A];
-  // mass flux of axis e at q + se e_e + sa e_A with face value v
-  auto mflux = [&](int e, int se, int sa, double v) -> double {
-    if constexpr (MF == MF_RHO) {
-      return rho0 * v;
-    } else {
-      const size_t r = e == A ? at(A, se) : at2(e, se, A, sa);
-      if constexpr (MF == MF_VOF) {
-        return rho0 * v + M.drho * (M.F[e][r] * M.hbydt[e]);
-      } else {
-        const size_t raw = id + (size_t)(se * st[e]) + (e == A ? 0 : (size_t)(sa * st[A]));
-        const int m = q.v[e] + se;  // 0 (a flux of 0) on a periodic axis: no cell before it
-        const double hi = M.eps_half[raw], lo = M.eps_half[raw - (RIM_ && m == 0 ? 0 : (size_t)st[e])];
-        double ef = 0.5 * (lo + hi);
-        if (RIM_ && m == 1) ef = hi;
-        if (RIM_ && m == g.n[e] + 1) ef = lo;
-        const double f = ef * v;
-        double mf = rho0 * f;
-        if (M.F[e]) mf = rho0 * f + M.drho * (M.F[e][r] * M.hbydt[e]);
-        if (RIM_ && (m < 1 || m > g.n[e] + 1)) mf = 0.0;
-        return mf;
-      }
-    }
-  };
-  constexpr bool TW = MF == MF_EPS;
-  const double* eo = E.eps_old;
-  double tmp;
-  {
-    const double mup = VAR ? P.mu[id] : g.mu0, mum = VAR ? P.mu[at(A, -1)] : g.mu0;
-    const double tau_p = mup * (c[A][3] - v0);
-    const double tau_m = mum * (v0 - c[A][1]);
-    if constexpr (TW) tmp = 2. * (eo[id] * tau_p - eo[rA] * tau_m) * g.inv_d2[A];
-    else tmp = 2. * (tau_p - tau_m) * g.inv_d2[A];
-  }
-  double mp[3], mm[3];
-  {
-    const double f0 = mflux(A, 0, 0, c[A][2]), fp = mflux(A, 1, 0, c[A][3]), fm = mflux(A, -1, 0, c[A][1]);
-    mp[A] = 0.5 * (f0 + fp);
-    mm[A] = 0.5 * (fm + f0);
-  }
-#pragma unroll
-  for (int e = 0; e < 2; e++) {
-    const int B = e == 0 ? B1 : B2;
-    double mu_p = 0.5 * (g.mu0 + g.mu0), mu_m = mu_p;
-    if constexpr (VAR) {
-      mu_p = 0.5 * (P.muf[B][at(B, 1)] + P.muf[B][at2(B, 1, A, -1)]);
-      mu_m = 0.5 * (P.muf[B][id] + P.muf[B][at(A, -1)]);
-    }
-    const double t_p = mu_p * ((wpp[B] - wmp[B]) * g.inv_d[A] + (c[B][3] - v0) * g.inv_d[B]);
-    const double t_m = mu_m * ((wp0[B] - wm0[B]) * g.inv_d[A] + (v0 - c[B][1]) * g.inv_d[B]);
-    if constexpr (TW) {
-      const size_t sB = (size_t)st[B];
-      double ep, em;
-      if (B > A) {
-        ep = 0.25 * (eo[rA] + eo[id] + eo[rA + sB] + eo[id + sB]);
-        em = 0.25 * (eo[rA - sB] + eo[id - sB] + eo[rA] + eo[id]);
-      } else {
-        ep = 0.25 * (eo[rA] + eo[rA + sB] + eo[id] + eo[id + sB]);
-        em = 0.25 * (eo[rA - sB] + eo[rA] + eo[id - sB] + eo[id]);
-      }
-      tmp += (ep * t_p - em * t_m) * g.inv_d[B];
-    } else {
-      tmp += (t_p - t_m) * g.inv_d[B];
-    }
-    mp[B] = 0.5 * (mflux(B, 1, -1, wmp[B]) + mflux(B, 1, 0, wpp[B]));
-    mm[B] = 0.5 * (mflux(B, 0, 0, wp0[B]) + mflux(B, 0, -1, wm0[B]));
-  }
-#pragma unroll
-  for (int e = 0; e < 3; e++) {
-    const double Mp = RIM_ ? flux_plus_in(mp[e], c[e], inp[e]) : flux_plus(mp[e], c[e]);
-    const double Mm = RIM_ ? flux_minus_in(mm[e], c[e], inm[e]) : flux_minus(mm[e], c[e]);
-    tmp -= (Mp - Mm) * g.inv_d[e];
-  }
-  const size_t cm = at(A, -1);
-  const double beta = VAR ? P.beta[A][id] : g.beta0;
-  const double rho_old_f = VAR ? 0.5 * (P.rho_old[id] + P.rho_old[cm]) : 0.5 * (rho0 + rho0);
-  if constexpr (TW) {
-    const double eo_f = 0.5 * (eo[rA] + eo[id]);
-    const double en_f = 0.5 * (E.eps[rA] + E.eps[id]);
-    tmp -= eo_f * (p[id] - p[cm]) * g.inv_d[A];
-    const double jd = E.imp[A] ? E.imp[A][id] * E.inv_vol : 0.0;
-    const double inv_eps_rho = beta / en_f;
-    return inv_eps_rho * (eo_f * rho_old_f * v0 + dt * tmp + jd) + dt * g.g[A];
-  } else {
-    tmp -= (p[id] - p[cm]) * g.inv_d[A];
-    return beta * (v0 * rho_old_f) + dt * (beta * tmp + g.g[A]);
-  }
-}
 template <bool VAR, MassFlux MF>
 __global__ __launch_bounds__(256) void k_predict_inner(Geo g, Props P, Vel V, VofF M, EpsF E,
                                                        const double* __restrict__ p, double* __restrict__ us0,
@@ -382,9 +131,9 @@ __global__ __launch_bounds__(256) void k_predict_inner(Geo g, Props P, Vel V, Vo
                   IN_LO + (int)blockIdx.z);
   if (q.v[0] > g.n[0] - IN_HI || q.v[1] > g.n[1] - IN_HI) return;
   const size_t id = IX(g, q);
-  us0[id] = face_direct<0, VAR, MF, false>(g, P, V, M, E, p, q, dt);
-  us1[id] = face_direct<1, VAR, MF, false>(g, P, V, M, E, p, q, dt);
-  us2[id] = face_direct<2, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+  us0[id] = face_ustar<0, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+  us1[id] = face_ustar<1, VAR, MF, false>(g, P, V, M, E, p, q, dt);
+  us2[id] = face_ustar<2, VAR, MF, false>(g, P, V, M, E, p, q, dt);
 }
 // blockIdx.y: the component
 template <bool VAR, MassFlux MF>
@@ -396,9 +145,9 @@ __global__ __launch_bounds__(256) void k_predict_rim(Geo g, Props P, Vel V, VofF
   const int a = (int)blockIdx.y;
   if (!g.per[a] && (a == 0 ? q.v[0] : (a == 1 ? q.v[1] : q.v[2])) < 2) return;  // wall face 1
   const size_t id = IX(g, q);
-  if (a == 0) us0[id] = face_direct<0, VAR, MF, true>(g, P, V, M, E, p, q, dt);
-  else if (a == 1) us1[id] = face_direct<1, VAR, MF, true>(g, P, V, M, E, p, q, dt);
-  else us2[id] = face_direct<2, VAR, MF, true>(g, P, V, M, E, p, q, dt);
+  if (a == 0) us0[id] = face_ustar<0, VAR, MF, true>(g, P, V, M, E, p, q, dt);
+  else if (a == 1) us1[id] = face_ustar<1, VAR, MF, true>(g, P, V, M, E, p, q, dt);
+  else us2[id] = face_ustar<2, VAR, MF, true>(g, P, V, M, E, p, q, dt);
 }
 
 // ld(c, di, dj, dk) = component c (0..2 = u, v, w; 3 = p) at (i+di, j+dj, k+dk)
@@ -818,9 +567,8 @@ __global__ __launch_bounds__(256, 3) void k_predict_tile(Geo g, Vel V, const dou
 // cell (i,j,k) computes u* on x-face i, v* on y-face j and w* on z-face k (the
 // cell's minus faces). The neighbourhoods of the three faces overlap, so their
 // loads are shared through L1; per face the arithmetic is exactly
-// predict_face<PeriodicBC, UniP, A>. Each thread marches KC planes in z so that
+// face_ustar's. Each thread marches KC planes in z so that
 // planes are reused while they are still in L2.
-template <class BC>
 __global__ __launch_bounds__(256) void k_predict_fused(Geo g, Vel V, const double* __restrict__ p,
                                                        double* __restrict__ us0, double* __restrict__ us1,
                                                        double* __restrict__ us2, double dt, int KC) {
@@ -2088,7 +1836,7 @@ void launch_predict(const Geo& g, const Props* P, const Vel& V, const double* p,
     return;
   } else if (allper) {
     dim3 grid((unsigned)((g.n[0] + 63) / 64), (unsigned)((g.n[1] + 3) / 4), (unsigned)((g.n[2] + KC - 1) / KC));
-    hipLaunchKernelGGL(k_predict_fused<PeriodicBC>, grid, CELLB, 0, st, g, V, p, us[0], us[1], us[2], dt, KC);
+    hipLaunchKernelGGL(k_predict_fused, grid, CELLB, 0, st, g, V, p, us[0], us[1], us[2], dt, KC);
     return;
   } else {
     predict_faces<false, MF_RHO>(g, Props{}, V, M0, EpsF{}, p, us, dt, st);
