@@ -67,6 +67,53 @@ __device__ __forceinline__ CoefC<C> level_coef(const Lv& L, int i, int j, int k)
   return r;
 }
 
+// level_coef<float, true> of the CPL active cells h = hb .. hb + CPL - 1 of a half
+// row (cells 2h - 1 where par, else 2h), the face coefficients of the 2 CPL cells
+// that the lane's pairs span read as 16-byte vectors (rows on 128-byte lines, hb =
+// 1 mod CPL). Half sweep of 256x128x128 13.0 us, of 128x64x64 4.1; with a load per
+// face and cell, whose lanes are 32 bytes apart and use 4 of them, 25.8 and 5.6.
+template <int CPL>
+__device__ __forceinline__ void level_coefs(const Lv& L, int par, int hb, int j, int k, CoefC<float> cv[CPL]) {
+  constexpr int N = 2 * CPL;
+  const int i0 = 2 * hb - 1;
+  const size_t r0 = lrow(L, j, k);
+  const size_t ry = lrow(L, LW(L, 1, j + 1), k), rz = lrow(L, j, LW(L, 2, k + 1));
+  float x[N + 1], ym[N], yp[N], zm[N], zp[N];
+#pragma unroll
+  for (int q = 0; q < N; q += 4) {
+    Vec<float, 4>::ld(L.bs[0] + r0 + i0 + q, x + q);
+    Vec<float, 4>::ld(L.bs[1] + r0 + i0 + q, ym + q);
+    Vec<float, 4>::ld(L.bs[1] + ry + i0 + q, yp + q);
+    Vec<float, 4>::ld(L.bs[2] + r0 + i0 + q, zm + q);
+    Vec<float, 4>::ld(L.bs[2] + rz + i0 + q, zp + q);
+  }
+  x[N] = L.bs[0][r0 + LW(L, 0, i0 + N)];
+  const bool wyp = wall_face(L.per[1], j + 1, L.n[1]), wym = wall_face(L.per[1], j, L.n[1]);
+  const bool wzp = wall_face(L.per[2], k + 1, L.n[2]), wzm = wall_face(L.per[2], k, L.n[2]);
+#pragma unroll
+  for (int t = 0; t < CPL; t++) {
+    const int o = 2 * t, e = o + 1;  // the odd and the even cell of the pair
+    const int i = i0 + (par ? o : e);
+    Coef c;
+    c.a[0] = (double)(par ? x[o + 1] : x[e + 1]) * L.inv_d2[0];
+    c.a[1] = (double)(par ? x[o] : x[e]) * L.inv_d2[0];
+    c.a[2] = (double)(par ? yp[o] : yp[e]) * L.inv_d2[1];
+    c.a[3] = (double)(par ? ym[o] : ym[e]) * L.inv_d2[1];
+    c.a[4] = (double)(par ? zp[o] : zp[e]) * L.inv_d2[2];
+    c.a[5] = (double)(par ? zm[o] : zm[e]) * L.inv_d2[2];
+    c.diag = c.a[0] + c.a[1] + c.a[2] + c.a[3] + c.a[4] + c.a[5];
+    if (wall_face(L.per[0], i + 1, L.n[0])) c.a[0] = 0.;
+    if (wall_face(L.per[0], i, L.n[0])) c.a[1] = 0.;
+    if (wyp) c.a[2] = 0.;
+    if (wym) c.a[3] = 0.;
+    if (wzp) c.a[4] = 0.;
+    if (wzm) c.a[5] = 0.;
+#pragma unroll
+    for (int m = 0; m < 6; m++) cv[t].a[m] = (float)c.a[m];
+    cv[t].diag = (float)c.diag;
+  }
+}
+
 // Red-black Gauss-Seidel half sweep of colour col ((i+j+k)&1 == col) on the
 // active half row: e = (f + S)/diag with S = sum of a_nb e_nb in the order
 // xp, xm, yp, ym, zp, zm. zero_start: e is zero on entry, so e = f/diag.
@@ -541,14 +588,16 @@ __global__ __launch_bounds__(256) void k_mg_rbgs_v2(Lv L, T* __restrict__ e, con
   };
   C fv[CPL];
   Vec<T, CPL>::ld(f + rb + off + p, fv);
+  CoefC<C> cv[VB ? CPL : 1];
   if (zero_start) {
     C ev[CPL];
+    if constexpr (VB && sizeof(C) == 4) level_coefs<CPL>(L, par, p, j, k, cv);
 #pragma unroll
     for (int t = 0; t < CPL; t++) {
       const int h = p + t;
       const int i = par ? 2 * h - 1 : 2 * h;
-      CoefC<C> c = coef(i);
-      ev[t] = sm_div(fv[t], c.diag);
+      const C diag = VB && sizeof(C) == 4 ? cv[VB ? t : 0].diag : coef(i).diag;
+      ev[t] = sm_div(fv[t], diag);
     }
     Vec<T, CPL>::st(e + rb + off + p, ev);
     return;
@@ -560,8 +609,9 @@ __global__ __launch_bounds__(256) void k_mg_rbgs_v2(Lv L, T* __restrict__ e, con
   Vec<T, CPL>::ld(e + zmr + off + p, zm);
   if (lo || hi) Vec<T, CPL>::ld(e + (lo ? ymr : ypr) + off + p, hv);
   // variable coefficients: read with the values, ahead of the barrier
-  CoefC<C> cv[VB ? CPL : 1];
-  if constexpr (VB) {
+  if constexpr (VB && sizeof(C) == 4) {
+    level_coefs<CPL>(L, par, p, j, k, cv);
+  } else if constexpr (VB) {
 #pragma unroll
     for (int t = 0; t < CPL; t++) {
       const int h = p + t;
@@ -846,7 +896,10 @@ __global__ __launch_bounds__(256) void k_mg_resid_rx(Lv F, Lv Cl, const T* __res
       // of the barrier
       constexpr bool HC = VB && sizeof(C) == 4;
       CoefC<C> cv[HC ? NM : 1][HC ? CPL : 1];
-      if constexpr (HC) {
+      if constexpr (HC && (CPL == 4 || CPL == 2)) {
+#pragma unroll
+        for (int m = 0; m < NM; m++) level_coefs<CPL>(L, par, 1 + CPL * lane + 64 * CPL * m, j, k, cv[m]);
+      } else if constexpr (HC) {
 #pragma unroll
         for (int m = 0; m < NM; m++)
 #pragma unroll
