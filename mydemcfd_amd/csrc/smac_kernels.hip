@@ -805,6 +805,41 @@ struct DirArgs {
   double a = 0.0;
 };
 
+// Face coefficients of the four natural cells i0 .. i0 + 3 of a row (i0 = 1 mod 4,
+// rows on 128-byte lines), read as 16-byte vectors, and coef_var of one of them. A
+// load per face and cell has lanes 32 bytes apart, of which each uses 8: with the
+// direction update 256x128x128 took 65 us, now 55 (0.25 GB).
+struct Coef4 {
+  double x[5], yp[4], ym[4], zp[4], zm[4];
+  __device__ __forceinline__ void load(const Geo& g, const BetaF& bf, int i0, int j, int k) {
+    const size_t r0 = idx(g, i0, j, k), ry = idx(g, i0, W(g, 1, j + 1), k), rz = idx(g, i0, j, W(g, 2, k + 1));
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) {
+      Vec<double, 2>::ld(bf.b[0] + r0 + q, x + q);
+      Vec<double, 2>::ld(bf.b[1] + r0 + q, ym + q);
+      Vec<double, 2>::ld(bf.b[1] + ry + q, yp + q);
+      Vec<double, 2>::ld(bf.b[2] + r0 + q, zm + q);
+      Vec<double, 2>::ld(bf.b[2] + rz + q, zp + q);
+    }
+    x[4] = bf.b[0][idx(g, W(g, 0, i0 + 4), j, k)];
+  }
+  template <int Q>
+  __device__ __forceinline__ Coef at(const Geo& g, int i, int j, int k) const {
+    const double f[6] = {x[Q + 1], x[Q], yp[Q], ym[Q], zp[Q], zm[Q]};
+    const int q[3] = {i, j, k};
+    Coef c;
+#pragma unroll
+    for (int m = 0; m < 6; m++) c.a[m] = f[m] * g.inv_d2[m / 2];
+    c.diag = c.a[0] + c.a[1] + c.a[2] + c.a[3] + c.a[4] + c.a[5];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      if (wall_face(g.per[d], q[d] + 1, g.n[d])) c.a[2 * d] = 0.;
+      if (wall_face(g.per[d], q[d], g.n[d])) c.a[2 * d + 1] = 0.;
+    }
+    return c;
+  }
+};
+
 // Ad = A d, part0 <- sum d*Ad (k_make_pAp, G_PCGSolver.cu:87-124), the dot in
 // pair order (lane l: split positions 1+2l+128m, then +1; the oracle's
 // RED_DOT_S2). NM = nx/128 in {2, 4}, rows aligned (FAST): the lane holds its
@@ -849,6 +884,11 @@ __global__ __launch_bounds__(256) void k_spmv_dot(Geo g, BetaF bf, double* __res
     constexpr int NH = NM / 2;  // pair chunks per half row
     constexpr int NX = 128 * NM;
     double xc[NM][2], yp[NM][2], ym[NM][2], zp[NM][2], zm[NM][2];
+    Coef4 cf[VAR ? NH : 1];
+    if constexpr (VAR) {
+#pragma unroll
+      for (int m = 0; m < NH; m++) cf[m].load(g, bf, 4 * lane + 256 * m + 1, j, k);
+    }
     using ZC = typename St<Z>::C;
     const double beta = (DIR && !FIRST) ? da.S[da.slot_beta] : 0.0;
     const bool shift = FIRST && da.slot_beta >= 0;
@@ -996,8 +1036,13 @@ __global__ __launch_bounds__(256) void k_spmv_dot(Geo g, BetaF bf, double* __res
           xm = t == 1 ? xc[m - NH][0] : nb;
           if (!perx && i == 1) xm = 0.0;
         }
-        const Coef c = VAR ? coef_var(g, bf.b, i, j, k)
-                           : ((!perx && (i == 1 || i == nx)) ? coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k) : crow);
+        // cell 2q (of the first half row) is the odd-placed one of its pair
+        Coef c;
+        if constexpr (VAR)
+          c = m < NH ? (t == 0 ? cf[m % NH].template at<1>(g, i, j, k) : cf[m % NH].template at<3>(g, i, j, k))
+                     : (t == 0 ? cf[m % NH].template at<0>(g, i, j, k) : cf[m % NH].template at<2>(g, i, j, k));
+        else
+          c = (!perx && (i == 1 || i == nx)) ? coef_uniform(g.n, g.per, g.inv_d2, g.beta0, i, j, k) : crow;
         double s = c.a[0] * xp + c.a[1] * xm + c.a[2] * yp[m][t] + c.a[3] * ym[m][t] + c.a[4] * zp[m][t] +
                    c.a[5] * zm[m][t];
         double v = c.diag * xc[m][t] - s;
