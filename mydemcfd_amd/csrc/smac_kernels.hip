@@ -1344,37 +1344,42 @@ __global__ __launch_bounds__(256) void k_xpay_ch(Geo g, const Z* __restrict__ z,
 // --------------------------------------------------------------- finalize
 // Reduce up to four row-partial arrays with the canonical 1024-lane tree
 // (kind 0 = sum, 1 = max) into S[out[m]], then apply one scalar op.
-// lane t of the canonical tree accumulates rows t, t+1024, ... in order;
-// loads are issued in batches (64 in the multi-block first stage, 16 in the
-// single-block kernel) so their latencies overlap; the summation order is
-// unchanged
-// B: loads in flight per lane (the adds stay sequential)
-template <int B>
-__device__ __forceinline__ double fin_lane(const double* __restrict__ part, int kind, int nrows, int t) {
-  double acc = 0.0;
-  int r = t;
-  for (; r + (B - 1) * 1024 < nrows; r += B * 1024) {
-    double v[B];
+// lane t of the canonical tree accumulates rows t, t+1024, ... in order, B loads
+// of each of the CNT arrays in flight (past the end the last row again, not added)
+template <int CNT, int B>
+__device__ __forceinline__ void fin_lane(const double* const* part, const int* kind, int nrows, int t,
+                                         double (&acc)[CNT]) {
 #pragma unroll
-    for (int u = 0; u < B; u++) v[u] = part[r + u * 1024];
+  for (int m = 0; m < CNT; m++) acc[m] = 0.0;
+  auto take = [&](int m, double v) {
+    if (kind[m] == 0) acc[m] += v;
+    else if (v > acc[m] || v != v) acc[m] = v;
+  };
+  int r0 = t;
+  for (; r0 + (B - 1) * 1024 < nrows; r0 += B * 1024) {
+    double v[CNT][B];
 #pragma unroll
-    for (int u = 0; u < B; u++) {
-      if (kind == 0) {
-        acc += v[u];
-      } else if (v[u] > acc || v[u] != v[u]) {
-        acc = v[u];
-      }
-    }
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < B; u++) v[m][u] = part[m][r0 + 1024 * u];
+#pragma unroll
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < B; u++) take(m, v[m][u]);
   }
-  for (; r < nrows; r += 1024) {
-    double v = part[r];
-    if (kind == 0) {
-      acc += v;
-    } else if (v > acc || v != v) {
-      acc = v;
-    }
+  constexpr int R = B < 8 ? B : 8;
+  for (; r0 < nrows; r0 += R * 1024) {
+    double v[CNT][R];
+#pragma unroll
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < R; u++) v[m][u] = part[m][min(r0 + 1024 * u, nrows - 1)];
+#pragma unroll
+    for (int m = 0; m < CNT; m++)
+#pragma unroll
+      for (int u = 0; u < R; u++)
+        if (r0 + 1024 * u < nrows) take(m, v[m][u]);
   }
-  return acc;
 }
 
 // first stage of a large reduction: the 1024 lane sums of array blockIdx.y,
@@ -1382,55 +1387,77 @@ __device__ __forceinline__ double fin_lane(const double* __restrict__ part, int 
 __global__ __launch_bounds__(64) void k_fin_lanes(FinalizeArgs fa) {
   const int m = blockIdx.y;
   const int t = (int)blockIdx.x * 64 + (int)threadIdx.x;
-  fa.stage[m * 1024 + t] = fin_lane<64>(fa.part[m], fa.kind[m], fa.nrows, t);
+  const double* part[1] = {fa.part[m]};
+  const int kind[1] = {fa.kind[m]};
+  double acc[1];
+  fin_lane<1, 64>(part, kind, fa.nrows, t, acc);
+  fa.stage[m * 1024 + t] = acc[0];
 }
 
+// The arrays side by side: all their loads in flight, then a wave each for the
+// rest of the tree. Bound by latency: after k_fin_lanes 2.7 us, 3.6 with the host's
+// copy (one array after the other, a barrier per level of the tree: 3.7 and 4.7);
+// k_fin_lanes 3.9 us at 16384 rows (6.5 when its last 16 rows came one by one).
+template <int CNT>
 __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs fa, double* __restrict__ S) {
-  __shared__ double lds[1024];
-  const int t = threadIdx.x;
-  for (int m = 0; m < fa.count; m++) {
-    const int kind = fa.kind[m];
-    double acc = fa.stage ? fa.stage[m * 1024 + t] : fin_lane<16>(fa.part[m], kind, fa.nrows, t);
-    lds[t] = acc;
-    __syncthreads();
-    for (int s = 512; s >= 64; s >>= 1) {
-      if (t < s) {
-        if (kind == 0) {
-          lds[t] = lds[t] + lds[t + s];
-        } else {
-          double o = lds[t + s];
-          if (o > lds[t] || o != o) lds[t] = o;
-        }
-      }
-      __syncthreads();
+  __shared__ double lds[CNT][1024], sum[CNT];
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  {
+    double acc[CNT];
+    if (fa.stage) {
+#pragma unroll
+      for (int m = 0; m < CNT; m++) acc[m] = fa.stage[m * 1024 + t];
+    } else {
+      fin_lane<CNT, 16>(fa.part, fa.kind, fa.nrows, t, acc);
     }
-    if (t < 64) {
-      double v = lds[t];
-      v = kind == 0 ? wave_tree_sum(v) : wave_max(v);
-      if (t == 0) {
-        S[fa.out[m]] = v;
-        if (fa.host) fa.host[fa.out[m]] = v;
-      }
-    }
-    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < CNT; m++) lds[m][t] = acc[m];
   }
-  if (t == 0 && fa.host)  // the values above before the number the host waits for
+  __syncthreads();
+  if (w < CNT) {
+    double x[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) x[u] = lds[w][lane + 64 * u];
+    double v;
+    if (fa.kind[w] == 0) {
+#pragma unroll
+      for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+        for (int u = 0; u < h; u++) x[u] = x[u] + x[u + h];
+      v = wave_tree_sum(x[0]);
+    } else {
+#pragma unroll
+      for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+        for (int u = 0; u < h; u++)
+          if (x[u + h] > x[u] || x[u + h] != x[u + h]) x[u] = x[u + h];
+      v = wave_max(x[0]);
+    }
+    if (lane == 0) {
+      sum[w] = v;
+      S[fa.out[w]] = v;
+    }
+  }
+  __syncthreads();
+  if (t != 0) return;
+  if (fa.host) {  // the values before the number the host waits for
+#pragma unroll
+    for (int m = 0; m < CNT; m++) fa.host[fa.out[m]] = sum[m];
     __hip_atomic_store(reinterpret_cast<uint64_t*>(fa.host + S_COUNT), fa.seq, __ATOMIC_RELEASE,
                        __HIP_MEMORY_SCOPE_SYSTEM);
-  if (t == 0) {
-    switch (fa.op) {
-      case OP_MEAN:  // S[dst] = S[a] / c
-        S[fa.dst] = S[fa.sa] / fa.c;
-        break;
-      case OP_DIV:  // S[dst] = S[a] / S[b]
-        S[fa.dst] = S[fa.sa] / S[fa.sb];
-        break;
-      case OP_BETA_PR:  // S[dst] = (-S[alpha] * S[zad]) / S[rz]
-        S[fa.dst] = (-S[fa.sa] * S[fa.sb]) / S[fa.sc];
-        break;
-      default:
-        break;
-    }
+  }
+  switch (fa.op) {
+    case OP_MEAN:  // S[dst] = S[a] / c
+      S[fa.dst] = S[fa.sa] / fa.c;
+      break;
+    case OP_DIV:  // S[dst] = S[a] / S[b]
+      S[fa.dst] = S[fa.sa] / S[fa.sb];
+      break;
+    case OP_BETA_PR:  // S[dst] = (-S[alpha] * S[zad]) / S[rz]
+      S[fa.dst] = (-S[fa.sa] * S[fa.sb]) / S[fa.sc];
+      break;
+    default:
+      break;
   }
 }
 
@@ -2141,15 +2168,16 @@ SMAC_INST_Z(double)
 SMAC_INST_Z(float)
 SMAC_INST_Z(bf16s)
 void launch_finalize(const FinalizeArgs& fa, double* S, hipStream_t st) {
-  if (fa.stage && fa.count > 0 && fa.nrows >= 16384) {
-    // large reductions: lane sums on 16 blocks per array, then the tree
+  FinalizeArgs f1 = fa;
+  // large reductions: lane sums on 16 blocks per array, then the tree. At 16384
+  // rows (128 x 128) one block for all costs the same (8 us for two arrays, with
+  // the host's copy), at 65536 13 to 23 us against 10
+  if (fa.stage && fa.nrows >= 16384)
     hipLaunchKernelGGL(k_fin_lanes, dim3(16, (unsigned)fa.count), dim3(64), 0, st, fa);
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, st, fa, S);
-  } else {
-    FinalizeArgs f1 = fa;
+  else
     f1.stage = nullptr;
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, st, f1, S);
-  }
+  if (fa.count == 2) hipLaunchKernelGGL(k_finalize<2>, dim3(1), dim3(1024), 0, st, f1, S);
+  else if (fa.count == 1) hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(1024), 0, st, f1, S);
 }
 // 16 rows a block where there are rows enough for every CU, 4 below
 static inline int small_nt(const Geo& g) { return g.n[1] * g.n[2] > 1024 ? 1024 : 256; }
