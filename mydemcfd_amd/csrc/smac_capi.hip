@@ -1558,9 +1558,34 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   const bool jac = small && !mg && !refg;  // Jacobi and its dots ride on the residual update
   int rz = S_RZ, rzn = S_RZN;
   bool fresh = false;  // S_RR and S_LINF on the host are those of the last update
+  if (jac && pcg_one_applies(g, var)) {
+    // the smallest grids: the iterations in one launch, which ends where the checks
+    // below would (a bounded number of them, so that no launch runs for long)
+    const bool linf_rule = o.stop_rule == SMAC_STOP_REF_LINF_DT;
+    while (iter < o.max_iter && !conv && !nan) {
+      PcgOne po;
+      po.linf = linf_rule;
+      po.target = linf_rule ? o.tol : o.tol * bnorm;
+      po.scale = dt;
+      po.flexible = o.flexible;
+      po.check_every = o.check_every;
+      po.iter0 = iter;
+      po.iters = std::min(o.max_iter - iter, 512);
+      po.last = iter + po.iters == o.max_iter;
+      KT(c, "pcg_one", launch_pcg_one(g, bfp, c->dv, c->r, c->dp, c->S, po, c->Sh, ++c->seq, s));
+      HIPOK(hipGetLastError());
+      rc = wait_scalars(c);
+      if (rc) return rc;
+      iter += (int)c->Sh[S_ITER];
+      conv = c->Sh[S_END] == 1.0;
+      nan = c->Sh[S_END] == 2.0;
+      have_update = fresh = true;
+    }
+  }
+  const int first_iter = iter;  // the loop's, unless all is done
   bool near_end = false;
   double last = o.stop_rule == SMAC_STOP_REF_LINF_DT ? 0.0 : bnorm;  // the last check's norm
-  for (iter = 0; iter < o.max_iter && !conv && !nan; ++iter) {
+  for (iter = first_iter; iter < o.max_iter && !conv && !nan; ++iter) {
     if (!ad_ready) KT(c, "spmv_dot", launch_spmv_dot(g, bfp, c->dv, c->Ad, small ? P[4] : P[0], s));
     double* pap = ad_ready || small ? P[4] : P[0];
     ad_ready = false;

@@ -120,7 +120,7 @@ struct FinalizeArgs {
 // device scalar slots
 enum {
   S_SUMB = 0, S_MEANB, S_BB, S_SUMR, S_SUMZ, S_RZ, S_RZN, S_PAP, S_ALPHA, S_BETA,
-  S_RR, S_LINF, S_ZAD, S_CFLC, S_CFLV, S_COUNT = 32
+  S_RR, S_LINF, S_ZAD, S_CFLC, S_CFLV, S_ITER, S_END, S_COUNT = 32
 };
 
 // alpha flux of the VoF transport for the predictor's mass flux:
@@ -224,6 +224,19 @@ void launch_xpay(const Geo& g, const Z* z, double* d, double* dp, const double* 
 // <- |r|^2, max |r|, r.z, z.Ad (the last two with Jacobi)
 constexpr size_t PCG_SMALL_ROWS = 8192, PCG_SMALL_CELLS = (size_t)1 << 19;
 bool pcg_small_applies(const Geo& g);
+// The Jacobi PCG of the smallest grids in one launch: `iters` iterations from
+// iteration iter0 on, fewer where it stops (check_every, stop rule as the host's:
+// linf: max |r| scale < target, else sqrt(|r|^2) < target); last: none follow. From
+// d = z, r.z in S[S_RZ]; |r|^2, max |r|, the iterations done and 0 / 1 (converged) /
+// 2 (not finite) go to host, then seq
+struct PcgOne {
+  double target, scale;
+  int linf, flexible, check_every, iter0, iters, last;
+};
+constexpr int PCG_ONE_SLOTS = 4, PCG_ONE_SLOTS_VAR = 1;
+bool pcg_one_applies(const Geo& g, bool var);
+void launch_pcg_one(const Geo& g, const BetaF* bf, double* d, double* r, double* dp, double* S, const PcgOne& o,
+                    double* host, uint64_t seq, hipStream_t st);
 template <typename Z>
 void launch_pcg_dir(const Geo& g, const BetaF* bf, const double* p_rz, const double* p_zad, int flexible, double* S,
                     int rz_in, int rz_out, const Z* z, const double* dold, double* dnew, double* dp, double* Ad,

@@ -1709,6 +1709,240 @@ __global__ __launch_bounds__(NT) void k_pcg_res(Geo g, BetaF bf, const double* _
   }
 }
 
+// The whole Jacobi PCG in one workgroup, for the smallest grids, where an
+// iteration's launches are most of it. Row 1024 / G * slot + t / G of the grid
+// belongs to G lanes of a wave, two of its split positions to a lane (2l + 1 and
+// 2l + 2 of pair order); r, Ad and dp stay in registers, d in LDS. The sums
+// are the canonical ones: over a row's lanes, whose upper ones would hold zeros,
+// then the tree over the rows, in every wave from LDS; |r|^2 and max |r| only where
+// they are read.
+// Stops by itself where the host's check would, at the latest after `iters`
+// iterations (the host goes on from there), and leaves r, d and dp as the passes
+// above do, with the last update's dp += alpha d done.
+// Bound by the instructions of its one CU, so without branches: rows that are not
+// there and neighbours beyond a y or z wall are a row of zeros ahead of the others,
+// x neighbours beyond a wall have coefficient zero. 21x17x13: 5.2 us an iteration,
+// with branches for all of these 8.2, by the two passes 11.9.
+template <bool VAR, int G, int NP>
+__global__ __launch_bounds__(1024) void k_pcg_one(Geo g, BetaF bf, double* __restrict__ dg, double* __restrict__ rg,
+                                                  double* __restrict__ dpg, double* __restrict__ S, PcgOne o,
+                                                  double* __restrict__ host, uint64_t seq) {
+  constexpr int RP = 1024 / G;                // rows per slot
+  constexpr int U = (RP * NP + 63) / 64;      // row sums per lane of the tree
+  constexpr int PW = 64 * U;
+  extern __shared__ double sm1[];
+  double* part = sm1;                         // [4][PW]: d.Ad, r.r, r.z, z.Ad
+  double* tab = part + 4 * PW;                // uniform: diag and 1/diag by the axes at a wall
+  double* wmx = tab + 16;                     // the waves' max |r|
+  double* d = wmx + 16;                       // 2G zeros, the rows, 2G more (read, not used)
+  const int t = (int)threadIdx.x, lane = t & 63, l = t & (G - 1);
+  const int nx = g.n[0], ny = g.n[1], nz = g.n[2], nh = nx >> 1, nrows = ny * nz;
+  const bool perx = g.per[0] != 0, pery = g.per[1] != 0, perz = g.per[2] != 0;
+  const double A0 = g.beta0 * g.inv_d2[0], A1 = g.beta0 * g.inv_d2[1], A2 = g.beta0 * g.inv_d2[2];
+  // the lane's positions: their cells (0: none), x neighbours' positions and, on a
+  // uniform grid, coefficients
+  int ci[2], qp[2], qm[2];
+  double ap[2], am[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const int q = 2 * l + 1 + c, i = q <= nh ? 2 * q : 2 * (q - nh) - 1;
+    ci[c] = q <= nx ? i : 0;
+    const bool p = perx || i < nx, m = perx || i > 1;
+    qp[c] = ci[c] && p ? spos(i < nx ? i + 1 : 1, nx) - 1 : 0;
+    qm[c] = ci[c] && m ? spos(i > 1 ? i - 1 : nx, nx) - 1 : 0;
+    ap[c] = p ? A0 : 0.0;
+    am[c] = m ? A0 : 0.0;
+  }
+  for (int e = t; e < 4 * PW; e += 1024) part[e] = 0.0;
+  for (int e = t; e < 4 * G + nrows * nx; e += 1024) d[e] = 0.0;
+  if constexpr (!VAR) {
+    if (t < 8) {
+      // one face missing per axis of the mask: which side makes no difference
+      const double a[6] = {A0, t & 1 ? 0.0 : A0, A1, t & 2 ? 0.0 : A1, A2, t & 4 ? 0.0 : A2};
+      const double diag = a[0] + a[1] + a[2] + a[3] + a[4] + a[5];
+      tab[t] = diag;
+      tab[8 + t] = 1. / diag;
+    }
+  }
+  __syncthreads();
+  // by slot: the row's offset in d and its walls (bits 1, 2 of tab's index); the
+  // offsets of its y and z neighbours. Unpacked anew at each use: kept over the
+  // loop, what follows from them would fill the registers.
+  int ow[NP], oy[NP], oz[NP];
+  auto opaque = [](int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  double r[NP][2], ad[NP][2], dp[NP][2];
+#pragma unroll
+  for (int s = 0; s < NP; s++) {
+    const int row = RP * s + t / G, j = row % ny + 1, k = row / ny + 1;
+    const bool in = row < nrows;
+    auto off = [&](bool there, int rw) { return in && there ? 2 * G + rw * nx : 0; };
+    const bool yp = pery || j < ny, ym = pery || j > 1, zp = perz || k < nz, zm = perz || k > 1;
+    ow[s] = off(true, row) | ((yp && ym ? 0 : 2) + (zp && zm ? 0 : 4)) << 16;
+    oy[s] = off(yp, j < ny ? row + 1 : row + 1 - ny) | off(ym, j > 1 ? row - 1 : row - 1 + ny) << 16;
+    oz[s] = off(zp, k < nz ? row + ny : row + ny - nrows) | off(zm, k > 1 ? row - ny : row - ny + nrows) << 16;
+    const size_t rb = idx(g, 0, j, k);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      r[s][c] = ad[s][c] = dp[s][c] = 0.0;
+      if (in && ci[c]) {
+        r[s][c] = rg[rb + 2 * l + 1 + c];
+        d[2 * G + row * nx + 2 * l + c] = dg[rb + 2 * l + 1 + c];
+        dp[s][c] = dpg[rb + ci[c]];
+      }
+    }
+  }
+  // the coefficients of cell c of slot s (VAR)
+  auto coef = [&](int s, int c) {
+    const int row = RP * s + opaque(t) / G;
+    return row < nrows && ci[c] ? coef_var(g, bf.b, ci[c], row % ny + 1, row / ny + 1)
+                                : Coef{{0., 0., 0., 0., 0., 0.}, 1.};
+  };
+  // the canonical sum over a row's lanes, in its first lane
+  auto row_sum = [](double v) {
+    if constexpr (G >= 64) v = v + lane_down<32>(v);
+    if constexpr (G >= 32) v = v + lane_down<16>(v);
+    v = v + lane_down<8>(v);
+    v = v + lane_down<4>(v);
+    v = v + lane_down<2>(v);
+    return v + lane_down<1>(v);
+  };
+  // the canonical sum over the rows of part array a
+  auto total = [&](int a) {
+    double x[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) x[u] = part[a * PW + lane + 64 * u];
+#pragma unroll
+    for (int h = U / 2; h >= 1; h >>= 1)
+#pragma unroll
+      for (int u = 0; u < h; u++) x[u] = x[u] + x[u + h];
+    return lane_value(wave_tree_sum(x[0]), 0);
+  };
+  double rz = S[S_RZ], alpha = 0.0, rr = 0.0, mx = 0.0;
+  int it = 0, end = 0;  // end: 1 converged, 2 not finite
+  __syncthreads();
+  while (true) {
+    // Ad = A d, d.Ad
+#pragma unroll
+    for (int s = 0; s < NP; s++) {
+      const int w = opaque(ow[s]), wy = opaque(oy[s]), wz = opaque(oz[s]);
+      const double* dr = d + (w & 0xffff);
+      const double* dyp = d + (wy & 0xffff) + 2 * l;
+      const double* dym = d + (int)((unsigned)wy >> 16) + 2 * l;
+      const double* dzp = d + (wz & 0xffff) + 2 * l;
+      const double* dzm = d + (int)((unsigned)wz >> 16) + 2 * l;
+      double acc = 0.0;
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const double xc = dr[2 * l + c], xp = dr[qp[c]], xm = dr[qm[c]];
+        const double yp = dyp[c], ym = dym[c], zp = dzp[c], zm = dzm[c];
+        double sum, diag;
+        if constexpr (VAR) {
+          const Coef cf = coef(s, c);
+          sum = cf.a[0] * xp + cf.a[1] * xm + cf.a[2] * yp + cf.a[3] * ym + cf.a[4] * zp + cf.a[5] * zm;
+          diag = cf.diag;
+        } else {
+          sum = ap[c] * xp + am[c] * xm + A1 * yp + A1 * ym + A2 * zp + A2 * zm;
+          diag = tab[(w >> 16) + (ap[c] == 0.0 || am[c] == 0.0)];
+        }
+        const double v = ci[c] ? diag * xc - sum : 0.0;
+        ad[s][c] = v;
+        acc += xc * v;
+      }
+      acc = row_sum(acc);
+      if (l == 0) part[RP * s + t / G] = acc;
+    }
+    __syncthreads();
+    alpha = rz / total(0);
+    const int iter = o.iter0 + it;
+    it++;
+    const bool check = iter % o.check_every == 0, over = it == o.iters;
+    // r -= alpha Ad, z = r / diag, r.z, z.Ad; dp += alpha d. Ad gives way to z
+    double mw = 0.0;
+#pragma unroll
+    for (int s = 0; s < NP; s++) {
+      const int w = opaque(ow[s]);
+      const double* dr = d + (w & 0xffff) + 2 * l;
+      double a0 = 0.0, a2 = 0.0, a3 = 0.0;
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const double rn = r[s][c] - alpha * ad[s][c];
+        r[s][c] = rn;
+        a0 += rn * rn;
+        const double ar = fabs(rn);
+        mw = max_step(mw, ar);
+        const double inv = VAR ? 1. / coef(s, c).diag : tab[8 + (w >> 16) + (ap[c] == 0.0 || am[c] == 0.0)];
+        const double zz = inv * rn;
+        a2 += rn * zz;
+        if (o.flexible) a3 += zz * ad[s][c];
+        dp[s][c] = dp[s][c] + alpha * dr[c];
+        ad[s][c] = zz;
+      }
+      a2 = row_sum(a2);
+      if (l == 0) part[2 * PW + RP * s + t / G] = a2;
+      if (check || over) {
+        a0 = row_sum(a0);
+        if (l == 0) part[PW + RP * s + t / G] = a0;
+      }
+      if (o.flexible) {
+        a3 = row_sum(a3);
+        if (l == 0) part[3 * PW + RP * s + t / G] = a3;
+      }
+    }
+    if (check || over) {
+      mw = wave_max(mw);
+      if (lane == 0) wmx[t >> 6] = mw;
+    }
+    __syncthreads();
+    const double rzn = total(2);
+    const double beta = o.flexible ? (-alpha * total(3)) / rz : rzn / rz;
+    rz = rzn;
+    if (check || over) {
+      rr = total(1);
+      mx = lane_value(wave_max(wmx[lane & 15]), 0);
+      if (check) {
+        const double m = o.linf ? mx * o.scale : sqrt(rr);
+        if (!(rr - rr == 0.0) || !(mx - mx == 0.0)) end = 2;
+        else if (m < o.target) end = 1;
+      }
+      if (end || (over && o.last)) break;
+    }
+    // d = z + beta d
+#pragma unroll
+    for (int s = 0; s < NP; s++) {
+      double* dr = d + (opaque(ow[s]) & 0xffff) + 2 * l;
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+        if (ci[c]) dr[c] = ad[s][c] + beta * dr[c];
+    }
+    if (over) break;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int s = 0; s < NP; s++) {
+    const int row = RP * s + t / G, j = row % ny + 1, k = row / ny + 1;
+    const size_t rb = idx(g, 0, j, k);
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      if (row < nrows && ci[c]) {
+        rg[rb + 2 * l + 1 + c] = r[s][c];
+        dg[rb + 2 * l + 1 + c] = d[2 * G + row * nx + 2 * l + c];
+        dpg[rb + ci[c]] = dp[s][c];
+      }
+  }
+  if (t == 0) {
+    S[S_RZ] = rz;
+    S[S_ALPHA] = alpha;
+    host[S_RR] = rr;
+    host[S_LINF] = mx;
+    host[S_ITER] = (double)it;
+    host[S_END] = (double)end;
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(host + S_COUNT), seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // S[dst] = S[src] (e.g. rz <- rz_new)
 __global__ void k_scalar_copy(double* S, int dst, int src) { S[dst] = S[src]; }
 __global__ void k_scalar_set(double* S, int dst, double v) { S[dst] = v; }
@@ -2178,6 +2412,52 @@ void launch_finalize(const FinalizeArgs& fa, double* S, hipStream_t st) {
     f1.stage = nullptr;
   if (fa.count == 2) hipLaunchKernelGGL(k_finalize<2>, dim3(1), dim3(1024), 0, st, f1, S);
   else if (fa.count == 1) hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(1024), 0, st, f1, S);
+}
+// lanes per row and row slots of k_pcg_one, 0 where it does not take the grid. An
+// iteration, against 9.5 to 11 us of the two passes: one slot (64 rows of up to 32
+// cells, 32 of 64, 16 of 128) 2.3 us, two 3.2 to 3.6, four 5.3 to 6; eight would be
+// 15. With variable coefficients, read from the L2 in both halves, one slot 5.2 us;
+// two 9.4, against 10.
+static inline int pcg_one_lanes(const Geo& g) { return g.n[0] <= 32 ? 16 : (g.n[0] <= 64 ? 32 : (g.n[0] <= 128 ? 64 : 0)); }
+static inline int pcg_one_slots(const Geo& g, bool var) {
+  const int G = pcg_one_lanes(g), rows = g.n[1] * g.n[2];
+  if (!G) return 0;
+  for (int np = 1; np <= (var ? PCG_ONE_SLOTS_VAR : PCG_ONE_SLOTS); np *= 2)
+    if (rows * G <= 1024 * np) return np;
+  return 0;
+}
+bool pcg_one_applies(const Geo& g, bool var) { return pcg_one_slots(g, var) != 0; }
+void launch_pcg_one(const Geo& g, const BetaF* bf, double* d, double* r, double* dp, double* S, const PcgOne& o,
+                    double* host, uint64_t seq, hipStream_t st) {
+  const int G = pcg_one_lanes(g), np = pcg_one_slots(g, bf != nullptr);
+  const int U = (1024 / G * np + 63) / 64;
+  const size_t shm = (size_t)(4 * 64 * U + 16 + 16 + 4 * G + g.n[0] * g.n[1] * g.n[2]) * sizeof(double);
+#define SMAC_ONE(V, GG, P) \
+  hipLaunchKernelGGL((k_pcg_one<V, GG, P>), dim3(1), dim3(1024), shm, st, g, bf ? *bf : BetaF{}, d, r, dp, S, o, host, seq)
+#define SMAC_ONE_P(V, GG)                            \
+  if constexpr (V) {                                 \
+    SMAC_ONE(V, GG, 1);                              \
+  } else {                                           \
+    if (np == 1) SMAC_ONE(V, GG, 1);                 \
+    else if (np == 2) SMAC_ONE(V, GG, 2);            \
+    else SMAC_ONE(V, GG, 4);                         \
+  }
+#define SMAC_ONE_G(V)                            \
+  if (G == 16) {                                 \
+    SMAC_ONE_P(V, 16)                            \
+  } else if (G == 32) {                          \
+    SMAC_ONE_P(V, 32)                            \
+  } else {                                       \
+    SMAC_ONE_P(V, 64)                            \
+  }
+  if (bf) {
+    SMAC_ONE_G(true)
+  } else {
+    SMAC_ONE_G(false)
+  }
+#undef SMAC_ONE_G
+#undef SMAC_ONE_P
+#undef SMAC_ONE
 }
 // 16 rows a block where there are rows enough for every CU, 4 below
 static inline int small_nt(const Geo& g) { return g.n[1] * g.n[2] > 1024 ? 1024 : 256; }
