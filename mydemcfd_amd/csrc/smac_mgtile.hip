@@ -92,6 +92,51 @@ __device__ __forceinline__ TCoef<C> tcoef_var(const Lv& L, int i, int j, int k) 
   return tcast<C>(c);
 }
 
+// The coefficients of the cells i0 (odd) and i0 + 1 of a row, their faces read as
+// pairs; a load per face and cell (tcoef_var) has its lanes two cells apart. Down and
+// up on 64x32x32 FP32 9.8 and 7.4 us, with tcoef_var 11.9 and 8.7; on 48x24x40 FP64
+// 13.0 and 8.2, with it 14.4 and 8.9
+template <typename C>
+struct alignas(2 * sizeof(C)) Pair {
+  C v[2];
+};
+template <typename C>
+__device__ __forceinline__ void tcoef_pair(const Lv& L, int i0, int j, int k, TCoef<C> out[2]) {
+  const int jp = L.per[1] ? wrapi(j + 1, L.n[1]) : j + 1, kp = L.per[2] ? wrapi(k + 1, L.n[2]) : k + 1;
+  const unsigned r0 = ((unsigned)k * (unsigned)L.py + (unsigned)j) * (unsigned)L.px;
+  const unsigned ry = ((unsigned)k * (unsigned)L.py + (unsigned)jp) * (unsigned)L.px;
+  const unsigned rz = ((unsigned)kp * (unsigned)L.py + (unsigned)j) * (unsigned)L.px;
+  const C* b[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    if constexpr (sizeof(C) == 4) b[d] = L.bs[d];
+    else b[d] = L.b[d];
+  }
+  auto ld = [&](const C* p, unsigned at) { return *reinterpret_cast<const Pair<C>*>(p + at); };
+  const Pair<C> x = ld(b[0], r0 + (unsigned)i0);
+  const C x2 = b[0][r0 + (unsigned)(L.per[0] ? wrapi(i0 + 2, L.n[0]) : i0 + 2)];
+  const Pair<C> ym = ld(b[1], r0 + (unsigned)i0), yp = ld(b[1], ry + (unsigned)i0);
+  const Pair<C> zm = ld(b[2], r0 + (unsigned)i0), zp = ld(b[2], rz + (unsigned)i0);
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    Coef c;
+    c.a[0] = (double)(t ? x2 : x.v[1]) * L.inv_d2[0];
+    c.a[1] = (double)x.v[t] * L.inv_d2[0];
+    c.a[2] = (double)yp.v[t] * L.inv_d2[1];
+    c.a[3] = (double)ym.v[t] * L.inv_d2[1];
+    c.a[4] = (double)zp.v[t] * L.inv_d2[2];
+    c.a[5] = (double)zm.v[t] * L.inv_d2[2];
+    c.diag = c.a[0] + c.a[1] + c.a[2] + c.a[3] + c.a[4] + c.a[5];
+    const int q[3] = {i0 + t, j, k};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      if (wall_face(L.per[d], q[d] + 1, L.n[d])) c.a[2 * d] = 0.;
+      if (wall_face(L.per[d], q[d], L.n[d])) c.a[2 * d + 1] = 0.;
+    }
+    out[t] = tcast<C>(c);
+  }
+}
+
 // A block's box: the tile with a halo of 4, 16 cells per edge from o - 4, and
 // in LDS one more cell around it (lx, ly, lz = -1..16). A colour's values lie in
 // [z][y][pair]: pair (lx + 2) >> 1 of 10 holds one cell of each colour. Thread
@@ -287,10 +332,13 @@ __global__ __launch_bounds__(TT) void k_mg_down(Lv L, Lv Cl, const T* __restrict
   }
   if constexpr (VB) {
 #pragma unroll
-    for (int c = 0; c < 2; c++)
+    for (int m = 0; m < 2; m++)
+      if (P.on(0, m, 4) || P.on(1, m, 4)) {
+        TCoef<C> q[2];
+        tcoef_pair<C>(L, P.s[0] ? P.i[1] : P.i[0], P.j, P.k[m], q);
 #pragma unroll
-      for (int m = 0; m < 2; m++)
-        if (P.on(c, m, 4)) k[c][m] = tcoef_var<C>(L, P.i[c], P.j, P.k[m]);
+        for (int c = 0; c < 2; c++) k[c][m] = P.s[c] ? q[1] : q[0];
+      }
   }
   for (int q = t; q < RW * RW * RW; q += TT) res[q] = (C)0;
 #pragma unroll
@@ -409,8 +457,12 @@ __global__ __launch_bounds__(TT) void k_mg_up(Lv Cl, Lv L, const T* __restrict__
   if constexpr (VB) {
 #pragma unroll
     for (int m = 0; m < 2; m++) {
-      if (P.on(0, m, 2)) k[0][m] = tcoef_var<C>(L, P.i[0], P.j, P.k[m]);
-      if (P.on(1, m, 3)) k[1][m] = tcoef_var<C>(L, P.i[1], P.j, P.k[m]);
+      if (P.on(0, m, 2) || P.on(1, m, 3)) {
+        TCoef<C> q[2];
+        tcoef_pair<C>(L, P.s[0] ? P.i[1] : P.i[0], P.j, P.k[m], q);
+#pragma unroll
+        for (int c = 0; c < 2; c++) k[c][m] = P.s[c] ? q[1] : q[0];
+      }
     }
   }
   __syncthreads();
@@ -459,7 +511,7 @@ dim3 tile_grid(const Lv& L) {
 }  // namespace
 
 // Row kernels against the tile, down and up together: 32^3 uniform BF16 16 us
-// against 31, 64^3 29 against 45, 64x32x32 variable FP32 22 against 43; but
+// against 31, 64^3 29 against 45, 64x32x32 variable FP32 17 against 43; but
 // 128x64x64 variable FP32 78 against 65 and 96x48x80 variable FP64 70 against
 // 45, where the halo's work outweighs the launches.
 template <typename T>
