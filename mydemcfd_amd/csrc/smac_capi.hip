@@ -1539,12 +1539,14 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     launch_scalar_set(c->S, S_BETA, 0.0, s);
   }
   // the direction update of an iteration rides on the next iteration's SpMV
-  // where the rows have the pair form; pAp partials then come in P[4]
+  // where the rows have the pair form or the grid is not large; pAp partials then
+  // come in P[4]
   if (!c->dv2 && !nan && !conv) {
     rc = dalloc(&c->dv2, c->tot);
     if (rc) return rc;
   }
   const bool fuse = c->dv2 && dir_spmv_applies<T>(g, z, c->dv, c->dv2, c->dp, c->Ad);
+  const bool dir_rows = c->dv2 && dir_rows_applies(g);
   // the zero-start red half sweep of level 0 rides on the residual update
   // (uniform coefficients: pointwise f/diag)
   const int zs_mode = (mg && !var && o.nu1 >= 1 && !(o.nu1 == 2 && o.nu2 == 2 && mg_tile_applies<T>(c->lev[0].lv)))
@@ -1723,8 +1725,11 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     // (small grids, the last iteration: no direction is needed any more, and
     // the flush below adds its alpha d)
     if (small) continue;
-    if (fuse && more) {
-      KT(c, "dir_spmv", launch_dir_spmv<T>(g, bfp, z, c->dv, c->dv2, c->dp, c->Ad, P[4], c->S, S_ALPHA, S_BETA, s));
+    if ((fuse || dir_rows) && more) {
+      if (fuse)
+        KT(c, "dir_spmv", launch_dir_spmv<T>(g, bfp, z, c->dv, c->dv2, c->dp, c->Ad, P[4], c->S, S_ALPHA, S_BETA, s));
+      else
+        KT(c, "dir_spmv", launch_dir_rows<T>(g, bfp, z, c->dv, c->dv2, c->dp, c->Ad, P[4], c->S, s));
       std::swap(c->dv, c->dv2);
       ad_ready = true;
     } else {
