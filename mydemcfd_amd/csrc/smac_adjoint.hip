@@ -84,9 +84,9 @@ __device__ __forceinline__ double flux_vjp(double m, const double c[5], bool inn
 // flux and the property cotangents: beta = 1/rho_f and mu of alpha^{n+1},
 // rho_old of alpha^n; addq(f, d, s, r, v) likewise, f = the axis of the flux, 3 =
 // alpha^{n+1}, 4 = alpha^n
-template <int A, bool VAR, bool VOF, bool RIM, class AddU, class AddQ>
+template <int A, bool VAR, bool VOF, class AddU, class AddQ>
 __device__ __forceinline__ void face_vjp(const Geo& g, const Props& P, const VofF& M, const AccV& AV, const double* p,
-                                         const Face<A, RIM>& F, double dt, double w, AddU addu, AddQ addq) {
+                                         const Face<A, true>& F, double dt, double w, AddU addu, AddQ addq) {
   constexpr MassFlux MF = VOF ? MF_VOF : MF_RHO;
   const double v0 = F.c[A][2], beta = F.template beta<VAR>(g, P), rho_old_f = F.template rho_old<VAR>(g, P);
   double mp[3], mm[3];
@@ -126,8 +126,8 @@ __device__ __forceinline__ void face_vjp(const Geo& g, const Props& P, const Vof
     double wp0 = -km * g.inv_d[A] + g.rho0 * bm, wm0 = km * g.inv_d[A] + g.rho0 * bm;
     c0 += c[2];
     const int x = F.q.v[B], n = g.n[B];
-    const bool wl = RIM && !g.per[B] && x == 1, wh = RIM && !g.per[B] && x == n;
-    if (RIM && !g.per[B]) {
+    const bool wl = !g.per[B] && x == 1, wh = !g.per[B] && x == n;
+    if (!g.per[B]) {
       // mirrored values pass their cotangent on, a wall's own are constants
       const double fl = wall_even(g, 2 * B) ? 1.0 : -1.0, fh = wall_even(g, 2 * B + 1) ? 1.0 : -1.0;
       if (x == n - 1) {
@@ -183,7 +183,7 @@ __device__ __forceinline__ void face_vjp(const Geo& g, const Props& P, const Vof
   c[1] += g.rho0 * bm;
   c[2] += g.rho0 * (bm + bp) + c0 - k2 * muq - k2 * mucm;
   c[3] += g.rho0 * bp;
-  if (RIM && !g.per[A]) {
+  if (!g.per[A]) {
     const int x = F.q.v[A], n = g.n[A];
     const bool lo = wall_stored(g, A, 2 * A), hi = wall_stored(g, A, 2 * A + 1);
     if (x == 2 && !lo) c[1] = 0.0;
@@ -212,7 +212,7 @@ __device__ __forceinline__ void face_vjp(const Geo& g, const Props& P, const Vof
 // reads and the LDS atomics: 128^3 204 us, 128x64x64 with VOF 182 us; one kernel
 // per component with a global atomic per partial derivative took 2300 and 2100.
 constexpr int VX = 64, VY = 4;
-template <bool VAR, bool VOF, bool RIM>
+template <bool VAR, bool VOF>
 __global__ __launch_bounds__(768) void k_predict_vjp(Geo g, Props P, Vel V, VofF M, const double* __restrict__ p,
                                                      Vel wbar, Acc U, AccV AV, double dt, int kc) {
   constexpr int PX = VX + 4, PL = PX * (VY + 4);  // velocity planes, two cells around
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(768) void k_predict_vjp(Geo g, Props P, Vel V, VofF
     if (!g.per[A] && q.v[A] < 2) return;
     const double w = wbar.c[A][IX(g, q)];
     if (w == 0.0) return;
-    const Face<A, RIM> F(g, V, q);
+    const Face<A, true> F(g, V, q);
     const int lo = ly * PX + lx, lq = ly * QX + lx;
     auto addu = [&](int c, int d, int s, int r, double v) {
       int o[3] = {0, 0, 0};
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(768) void k_predict_vjp(Geo g, Props P, Vel V, VofF
       o[A] += r;
       unsafeAtomicAdd(sf[f] + pq(k + o[2]) + (o[1] + 1) * QX + (o[0] + 1) + lq, v);
     };
-    face_vjp<A, VAR, VOF, RIM>(g, P, M, AV, p, F, dt, w, addu, addq);
+    face_vjp<A, VAR, VOF>(g, P, M, AV, p, F, dt, w, addu, addq);
   };
   auto out = [&](double* base, double* s, int x, int y, int z) {
     const double v = *s;
@@ -361,8 +361,8 @@ __global__ __launch_bounds__(256) void k_rowsum_nat(Geo g, const double* __restr
   if (lane == 0) part0[row] = acc;
 }
 
-// planes per block: at least VJP_BLOCKS blocks (two for each CU, which is what
-// their registers allow), as long as a block has four planes to share its edges
+// planes per block: at least VJP_BLOCKS blocks, two for each CU in turn (one fits its
+// registers), as long as a block has four planes to share its edges
 constexpr unsigned VJP_BLOCKS = 512;
 template <bool VAR, bool VOF>
 void predict_vjp(const Geo& g, const Props& P, const Vel& V, const VofF& M, const double* p, double* const wbar[3],
@@ -372,7 +372,7 @@ void predict_vjp(const Geo& g, const Props& P, const Vel& V, const VofF& M, cons
   while (kc > 4 && bx * by * (unsigned)((g.n[2] + kc - 1) / kc) < VJP_BLOCKS) kc /= 2;
   Vel wb;
   for (int d = 0; d < 3; d++) wb.c[d] = wbar[d];
-  hipLaunchKernelGGL((k_predict_vjp<VAR, VOF, true>), dim3(bx, by, (unsigned)((g.n[2] + kc - 1) / kc)), dim3(768), 0,
+  hipLaunchKernelGGL((k_predict_vjp<VAR, VOF>), dim3(bx, by, (unsigned)((g.n[2] + kc - 1) / kc)), dim3(768), 0,
                      st, g, P, V, M, p, wb, U, AV, dt, kc);
 }
 
