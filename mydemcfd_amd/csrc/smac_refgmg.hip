@@ -318,7 +318,8 @@ __global__ __launch_bounds__(256) void k_add_scalar_norms(Geo g, double* __restr
 // back. Per cell the operations and their order are those of the sweeps above.
 // Bound by latency: 64x32x32 11 us down and 11 us up where nine launches took
 // 28 and 20 us; the 32x16x16 level 8 us each way against 20; the 38 sweeps of
-// the levels 16x8x8 and 8x8x8 19 us against 115.
+// the levels 16x8x8 and 8x8x8 16.6 us against 115 (18.8 while
+// each sweep formed its neighbours' places anew).
 constexpr int RB_T = 8, RB_H = 4, RB_W = RB_T + 2 * RB_H, RB_N = RB_W * RB_W * RB_W;
 
 // FINE: the finest grid (row-split vectors, its own operator), else a level
@@ -515,7 +516,10 @@ __global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T
   __shared__ double X[2][RG_TAIL_PAD];
   const int t = (int)threadIdx.x;
   double a[CPT][6], inv[CPT], f[CPT];
-  int p[CPT], off[CPT][3];  // LDS index (-1: no cell); (+, -) neighbour offsets per axis, 16 bits each
+  // LDS index (-1: no cell), the neighbours' (two to a word where the registers are short)
+  constexpr bool PACK = CPT > 1;
+  double own[PACK ? 1 : CPT];  // the cell's value in X[cur]
+  int p[CPT], nb[CPT][PACK ? 3 : 6];
   size_t at[CPT];
   int cur = 0;
   // the level's coefficients and right-hand side, both copies of X zero
@@ -534,6 +538,7 @@ __global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T
       const int e = t + 1024 * u;
       p[u] = -1;
       f[u] = 0.0;
+      if constexpr (!PACK) own[u] = 0.0;
       if (e < cells) {
         const int i = e % L.n[0] + 1, j = (e / L.n[0]) % L.n[1] + 1, k = e / nxy + 1;
         p[u] = k * sz + j * sy + i;
@@ -548,38 +553,64 @@ __global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T
         for (int d = 0; d < 3; d++) {
           const int hi = L.per[d] && q[d] == L.n[d] ? -(L.n[d] - 1) * st[d] : st[d];
           const int lo = L.per[d] && q[d] == 1 ? (L.n[d] - 1) * st[d] : -st[d];
-          off[u][d] = (int)(((unsigned)lo << 16) | ((unsigned)hi & 0xffffu));
+          if constexpr (PACK) {
+            nb[u][d] = (p[u] + hi) | (p[u] + lo) << 16;
+          } else {
+            nb[u][2 * d] = p[u] + hi;
+            nb[u][2 * d + 1] = p[u] + lo;
+          }
         }
       }
     }
   };
   auto nbsum = [&](const double* x, int u) -> double {
-    const int q = p[u];
     double v[6];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      v[2 * d] = x[q + (int)(short)(off[u][d] & 0xffff)];
-      v[2 * d + 1] = x[q + (off[u][d] >> 16)];
+    for (int m = 0; m < 6; m++) {
+      if constexpr (PACK) v[m] = x[m & 1 ? nb[u][m / 2] >> 16 : nb[u][m / 2] & 0xffff];
+      else v[m] = x[nb[u][m]];
     }
     return a[u][0] * v[0] + a[u][1] * v[1] + a[u][2] * v[2] + a[u][3] * v[3] + a[u][4] * v[4] + a[u][5] * v[5];
   };
-  auto sweeps = [&](int n) {
+  // the cell's value in x = X[cur]
+  auto val = [&](const double* x, int u) -> double {
+    if constexpr (PACK) return x[p[u]];
+    else return own[u];
+  };
+  auto sweep = [&](const double* x, double* y) {
     const double omega = RG_OMEGA;
-#pragma unroll 1
-    for (int it = 0; it < n; it++) {
-      const double* x = X[cur];
-      double* y = X[1 - cur];
 #pragma unroll
-      for (int u = 0; u < CPT; u++)
-        if (p[u] >= 0) y[p[u]] = (1.0 - omega) * x[p[u]] + omega * (nbsum(x, u) + f[u]) * inv[u];
-      cur = 1 - cur;
-      __syncthreads();
+    for (int u = 0; u < CPT; u++)
+      if (p[u] >= 0) {
+        const double v = (1.0 - omega) * val(x, u) + omega * (nbsum(x, u) + f[u]) * inv[u];
+        y[p[u]] = v;
+        if constexpr (!PACK) own[u] = v;
+      }
+    __syncthreads();
+  };
+  // n sweeps from X[0]; with one cell a thread two at a time, so that the copies'
+  // addresses are fixed (with four the longer loop costs more than it saves)
+  auto sweeps = [&](int n) {
+    if constexpr (PACK) {
+#pragma unroll 1
+      for (int it = 0; it < n; it++) {
+        sweep(X[cur], X[1 - cur]);
+        cur = 1 - cur;
+      }
+    } else {
+#pragma unroll 1
+      for (int it = 0; it + 1 < n; it += 2) {
+        sweep(X[0], X[1]);
+        sweep(X[1], X[0]);
+      }
+      if (n & 1) sweep(X[0], X[1]);
+      cur = n & 1;
     }
   };
   auto store = [&](int l) {
 #pragma unroll
     for (int u = 0; u < CPT; u++)
-      if (p[u] >= 0) T[l].q[at[u]] = X[cur][p[u]];
+      if (p[u] >= 0) T[l].q[at[u]] = val(X[cur], u);
   };
 #pragma unroll 1
   for (int l = first; l < last; l++) {
@@ -592,7 +623,7 @@ __global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T
     for (int u = 0; u < CPT; u++)
       if (p[u] >= 0) {
         const double diag = (a[u][0] + a[u][1] + a[u][2] + a[u][3] + a[u][4] + a[u][5]);
-        const double Ap = X[cur][p[u]] * diag - nbsum(X[cur], u);
+        const double Ap = val(X[cur], u) * diag - nbsum(X[cur], u);
         res[p[u]] = f[u] - Ap;
       }
     __syncthreads();
@@ -636,7 +667,9 @@ __global__ __launch_bounds__(1024) void k_rg_tail(const RgTailLv* __restrict__ T
         int Q[3] = {e % V.L.n[0] + 1, (e / V.L.n[0]) % V.L.n[1] + 1, e / (V.L.n[0] * V.L.n[1]) + 1};
 #pragma unroll
         for (int d = 0; d < 3; d++) Q[d] = C.co[d] ? (Q[d] + 1) / 2 : Q[d];
-        X[0][p[u]] = V.q[at[u]] + T[l + 1].q[ridx(C, Q[0], Q[1], Q[2])];
+        const double v = V.q[at[u]] + T[l + 1].q[ridx(C, Q[0], Q[1], Q[2])];
+        X[0][p[u]] = v;
+        if constexpr (!PACK) own[u] = v;
       }
     __syncthreads();
     sweeps(nf);
