@@ -208,7 +208,9 @@ int smac_set_fluid(smac_ctx* ctx, const smac_fluid_desc* fluid);
  * field in the reference layout (above). Synchronous. */
 int smac_upload(smac_ctx* ctx, int32_t field, const double* host, size_t count);
 int smac_download(smac_ctx* ctx, int32_t field, double* host, size_t count);
-/* Same, from/to a device buffer (e.g. a torch tensor) in the reference layout.
+/* Same, from/to a device buffer (e.g. a torch tensor) of the context's GPU in the
+ * reference layout. A buffer of another GPU or of pinned host memory goes through
+ * the runtime's copies, plane by plane.
  * The copy runs on the context's non-blocking stream, which is not ordered with
  * any other stream: finish the other streams' work on the buffer first (for a
  * torch tensor, torch.cuda.synchronize(); the caching allocator hands a freed

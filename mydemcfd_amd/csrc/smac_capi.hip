@@ -636,20 +636,8 @@ extern "C" size_t smac_field_count(const smac_ctx* c, int32_t f) {
   return (size_t)sh[0] * (size_t)sh[1] * (size_t)sh[2];
 }
 
-// a device field between the reference layout and the box, queued on the
-// context stream
-static int move_field(smac_ctx* c, int f, double* box, const double* ref, bool to_box) {
-  int sh[3];
-  field_shape(c, f, sh);
-  launch_field_copy(box, const_cast<double*>(ref), c->g.px, c->g.py, sh, to_box ? 1 : 0, c->st);
-  HIPOK(hipGetLastError());
-  return SMAC_OK;
-}
-static int field_in(smac_ctx* c, int f, double* box, const double* ref) { return move_field(c, f, box, ref, true); }
-static int field_out(smac_ctx* c, int f, double* ref, double* box) { return move_field(c, f, box, ref, false); }
-
-// copy between a host array in the reference layout (src pitch sh0, plane
-// sh0*sh1) and the padded box, one 2-D copy per z-plane
+// copy between an array in the reference layout (src pitch sh0, plane sh0*sh1)
+// and the padded box by the runtime, one 2-D copy per z-plane
 static int copy_field(smac_ctx* c, int f, double* dst_box, const double* src_ref, bool to_box, hipMemcpyKind kind,
                       double* dst_ref, const double* src_box) {
   int sh[3];
@@ -669,6 +657,46 @@ static int copy_field(smac_ctx* c, int f, double* dst_box, const double* src_ref
   HIPOK(hipStreamSynchronize(c->st));
   return SMAC_OK;
 }
+
+// does `p` lie in memory of the context's GPU (or managed memory of it)?
+static bool device_memory(const smac_ctx* c, const void* p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return (at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged) && at.device == c->dev;
+}
+// May a kernel of the context touch the `bytes` bytes at p? Only where they lie
+// whole, and aligned, in one allocation of its GPU. Everything else -- another
+// GPU's memory, host memory, a pointer or an extent that the runtime does not know --
+// is the runtime's, which stages it or refuses it; in a kernel it would be a fault.
+static bool kernel_reaches(const smac_ctx* c, const void* p, size_t bytes) {
+  if ((reinterpret_cast<uintptr_t>(p) & 7u) != 0 || !device_memory(c, p)) return false;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return (size_t)((const char*)p - (const char*)base) + bytes <= size;
+}
+// a device field between the reference layout and the box, queued on the
+// context stream (finished at return where the runtime copies)
+static int move_field(smac_ctx* c, int f, double* box, double* ref, bool to_box) {
+  int sh[3];
+  field_shape(c, f, sh);
+  if (!kernel_reaches(c, ref, (size_t)sh[0] * (size_t)sh[1] * (size_t)sh[2] * sizeof(double)))
+    return to_box ? copy_field(c, f, box, ref, true, hipMemcpyDeviceToDevice, nullptr, nullptr)
+                  : copy_field(c, f, nullptr, nullptr, false, hipMemcpyDeviceToDevice, ref, box);
+  KT(c, "field_copy", launch_field_copy(box, ref, c->g.px, c->g.py, sh, to_box ? 1 : 0, c->st));
+  HIPOK(hipGetLastError());
+  return SMAC_OK;
+}
+static int field_in(smac_ctx* c, int f, double* box, const double* ref) {
+  return move_field(c, f, box, const_cast<double*>(ref), true);
+}
+static int field_out(smac_ctx* c, int f, double* ref, double* box) { return move_field(c, f, box, ref, false); }
 
 // fill periodic images (ghost cells, duplicate faces) of a downloaded host array
 static void fill_periodic_images(const smac_ctx* c, int f, double* h) {
@@ -782,13 +810,7 @@ extern "C" int smac_bind_device(smac_ctx* c, int32_t f, double* dev, size_t coun
     return SMAC_OK;
   }
   if (count != c->tot || (reinterpret_cast<uintptr_t>(dev) & 255u) != 0) return SMAC_ERR_INVALID_ARG;
-  hipPointerAttribute_t at;
-  if (hipPointerGetAttributes(&at, dev) != hipSuccess) {
-    (void)hipGetLastError();
-    return SMAC_ERR_INVALID_ARG;
-  }
-  if ((at.type != hipMemoryTypeDevice && at.type != hipMemoryTypeManaged) || at.device != c->dev)
-    return SMAC_ERR_INVALID_ARG;
+  if (!device_memory(c, dev)) return SMAC_ERR_INVALID_ARG;
   HIPOK(hipStreamSynchronize(c->st));  // work queued on the old array ends first
   if (!c->bound[f]) c->own[f] = *slot;
   c->bound[f] = dev;
