@@ -1996,6 +1996,13 @@ extern "C" int smac_cell_output(smac_ctx* c, float* h, size_t count) {
   return SMAC_OK;
 }
 
+// The adjoints' copies from and to the caller's arrays are queued; none is left
+// when the call ends, on an error either (the caller may free the arrays then).
+struct StreamDrain {
+  hipStream_t st;
+  ~StreamDrain() { (void)hipStreamSynchronize(st); }
+};
+
 // Adjoint of one smac_step (see smac_adjoint.hip for the derivation).
 extern "C" int smac_adjoint_step(smac_ctx* c, double dt, const smac_solver_opts* opts, const double* const u_n[3],
                                  double* const ubar[3], double* pbar, smac_solve_stats* st) {
@@ -2022,6 +2029,7 @@ extern "C" int smac_adjoint_step(smac_ctx* c, double dt, const smac_solver_opts*
   double* pbo = c->adj[10];
   const Geo& g = c->g;
   hipStream_t s = c->st;
+  const StreamDrain drain{s};
   // the state of the step and the cotangents of its output, in the box layout
   for (int a = 0; a < 3; a++) {
     rc = field_in(c, SMAC_FIELD_U + a, c->u[a], u_n[a]);
@@ -2102,6 +2110,7 @@ extern "C" int smac_adjoint_vof_step(smac_ctx* c, double dt, int32_t S, int32_t 
   double* pbo = c->adj[10];
   const Geo& g = c->g;
   hipStream_t s = c->st;
+  const StreamDrain drain{s};
   const size_t bytes = c->tot * sizeof(double);
   // ---- the step again, from (alpha^n, u^n, p^n)
   rc = field_in(c, SMAC_FIELD_ALPHA, ral[0], alpha_n);

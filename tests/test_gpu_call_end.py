@@ -1,0 +1,40 @@
+"""GPU: what has ended when a call returns.
+
+* An adjoint step that fails (here: a level count that the grid does not have) leaves
+  no copy from the caller's arrays on the stream.
+"""
+import pytest
+
+from mydemcfd_amd import _abi, cases
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+F64 = torch.float64
+
+
+def _idle(ctx):
+    return torch.cuda.ExternalStream(ctx.lib.smac_stream(ctx.h)).query()
+
+
+@pytest.mark.parametrize("vof", [False, True])
+def test_failed_adjoint_leaves_nothing_queued(hip, vof):
+    n = (160, 160, 160)
+    print(f"case: failing adjoint step {n} vof={vof}", flush=True)
+    ctx = hip.SMACContext(**(cases.dam_break_desc(n) if vof else cases.cavity_desc(n)))
+    # the copies of the whole arrays take longer than the refusal behind them
+    vel = [torch.zeros(ctx.shape(f), dtype=F64, device="cuda") for f in "uvw"]
+    bar = [torch.zeros_like(t) for t in vel]
+    p = torch.zeros(ctx.shape("p"), dtype=F64, device="cuda")
+    q = [torch.zeros_like(p) for _ in range(3)]
+    torch.cuda.synchronize()
+    kw = dict(precond="mg", mg_levels=12)
+    for _ in range(2):  # the first call also allocates, which waits for the GPU
+        with pytest.raises(_abi.SmacError) as e:
+            if vof:
+                ctx.adjoint_vof_step(1e-3, 1, 0, q[0].data_ptr(), [t.data_ptr() for t in vel], p.data_ptr(),
+                                     q[1].data_ptr(), [t.data_ptr() for t in bar], q[2].data_ptr(), **kw)
+            else:
+                ctx.adjoint_step(1e-3, [t.data_ptr() for t in vel], [t.data_ptr() for t in bar], p.data_ptr(), **kw)
+        assert _idle(ctx)
+        assert e.value.status == _abi.SMAC_ERR_INVALID_GRID
