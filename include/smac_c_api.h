@@ -297,14 +297,15 @@ int smac_update_poisson_beta_two_way(smac_ctx* ctx);
  * preconditioned CG on A dp = b, dp starting from 0. Once SMAC_FIELD_EPS and
  * EPS_OLD are uploaded the RHS carries the volume fraction,
  * b = -(1/dt) D(eps_f u*) - (eps - eps_old)/dt^2 (the reference's general form;
- * without them eps = 1). */
+ * without them eps = 1). Has ended, with all its work on the device, at return. */
 int smac_pressure_solve(smac_ctx* ctx, double dt, const smac_solver_opts* opts,
                         smac_solve_stats* stats);
 /* G_SMACSolver::correct_vof_velocity (CFD/G_SMACSolver.cu:1072-1142,1269-1275):
  * u = u* - beta*dt*grad(dp) on interior faces, p += dp, dp = 0. */
 int smac_correct(smac_ctx* ctx, double dt);
 /* One whole step: properties (if variable), mass flux, predictor, solve, correct,
- * in the order of the driver loop CFD/main.cu:298-317. */
+ * in the order of the driver loop CFD/main.cu:298-317. Returns with the solve's
+ * statistics; the correction is queued on the context's stream (smac_sync). */
 int smac_step(smac_ctx* ctx, double dt, const smac_solver_opts* opts, smac_solve_stats* stats);
 /* G_SMACSolver::calc_cfl (CFD/G_SMACSolver.cu:1365-1430): convective and viscous
  * CFL numbers for time step dt. */

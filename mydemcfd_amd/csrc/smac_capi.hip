@@ -1802,7 +1802,12 @@ static int pressure_solve(smac_ctx* c, double dt, const smac_solver_opts* opts, 
                           bool rhs_given);
 
 extern "C" int smac_pressure_solve(smac_ctx* c, double dt, const smac_solver_opts* opts, smac_solve_stats* st) {
-  return pressure_solve(c, dt, opts, st, false);
+  const int rc = pressure_solve(c, dt, opts, st, false);
+  // the solve itself returns with its norms: the last update of dp, and a V-cycle or
+  // direction pass queued ahead of the check that ended it, may still run. A caller
+  // of the solve alone finds them done, and an error of theirs in this call.
+  if (c) HIPOK(hipStreamSynchronize(c->st));
+  return rc;
 }
 
 static int pressure_solve(smac_ctx* c, double dt, const smac_solver_opts* opts, smac_solve_stats* st,
@@ -1883,7 +1888,7 @@ extern "C" int smac_step(smac_ctx* c, double dt, const smac_solver_opts* o, smac
   double t_pred = prof_end(c, 0);
   prof_begin(c, 2);
   c->defer_dp = true;
-  rc = smac_pressure_solve(c, dt, o, sp);
+  rc = pressure_solve(c, dt, o, sp, false);
   c->defer_dp = false;
   if (rc) {
     if (c->dp_deferred) {  // leave dp complete on an error return

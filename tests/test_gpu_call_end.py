@@ -2,7 +2,10 @@
 
 * An adjoint step that fails (here: a level count that the grid does not have) leaves
   no copy from the caller's arrays on the stream.
+* A pressure solve has ended, also the V-cycle that was queued ahead of the check that
+  stopped it.
 """
+import numpy as np
 import pytest
 
 from mydemcfd_amd import _abi, cases
@@ -38,3 +41,23 @@ def test_failed_adjoint_leaves_nothing_queued(hip, vof):
                 ctx.adjoint_step(1e-3, [t.data_ptr() for t in vel], [t.data_ptr() for t in bar], p.data_ptr(), **kw)
         assert _idle(ctx)
         assert e.value.status == _abi.SMAC_ERR_INVALID_GRID
+
+
+@pytest.mark.parametrize("precond,kw", [("mg", dict(tol=0.9)), ("mg", dict(tol=0.0, max_iter=1)),
+                                        ("mg", dict(tol=0.9, precision="fp32", flexible=1)),
+                                        ("ref_gmg", dict(tol=0.9)), ("jacobi", dict(tol=0.0, max_iter=3))])
+def test_pressure_solve_has_ended(hip, precond, kw):
+    n = (192, 192, 192)
+    print(f"case: end of a solve {precond} {kw}", flush=True)
+    ctx = hip.SMACContext(**cases.periodic_desc(n))
+    rng = np.random.default_rng(4)
+    for f in ("ustar", "vstar", "wstar"):
+        ctx.upload(f, rng.standard_normal(ctx.shape(f)))
+    for _ in range(2):
+        ctx.pressure_solve(1e-3, precond=precond, **kw)
+        assert _idle(ctx)
+    ctx.upload("ustar", np.full(ctx.shape("ustar"), np.nan))
+    with pytest.raises(_abi.SmacError) as e:
+        ctx.pressure_solve(1e-3, precond=precond, **kw)
+    assert _idle(ctx)
+    assert e.value.status == _abi.SMAC_ERR_NAN
