@@ -500,8 +500,13 @@ extern "C" int smac_create(const smac_grid_desc* gd, const smac_fluid_desc* fl, 
   return SMAC_OK;
 }
 
+// A step returns while a V-cycle queued ahead of the check that ended its solve may
+// still run, so its graph (and, in mg_free, the arrays under it) can be in flight.
 static void graph_free(smac_ctx* c) {
-  if (c->cg_exec) (void)hipGraphExecDestroy(c->cg_exec);
+  if (c->cg_exec) {
+    (void)hipStreamSynchronize(c->st);
+    (void)hipGraphExecDestroy(c->cg_exec);
+  }
   c->cg_exec = nullptr;
   c->cg_nu[0] = c->cg_nu[1] = -1;
 }

@@ -4,6 +4,8 @@
   no copy from the caller's arrays on the stream.
 * A pressure solve has ended, also the V-cycle that was queued ahead of the check that
   stopped it.
+* Steps whose solver options change the hierarchy or its graph, taken while the last
+  step's work is still queued, give the fields of steps that each waited for the one before.
 """
 import numpy as np
 import pytest
@@ -61,3 +63,25 @@ def test_pressure_solve_has_ended(hip, precond, kw):
         ctx.pressure_solve(1e-3, precond=precond, **kw)
     assert _idle(ctx)
     assert e.value.status == _abi.SMAC_ERR_NAN
+
+
+def test_options_change_behind_a_queued_vcycle(hip):
+    n = (96, 96, 96)
+    print(f"case: changing V-cycle options behind queued work {n}", flush=True)
+    rng = np.random.default_rng(6)
+    fields = {}
+    ctxs = [hip.SMACContext(**cases.periodic_desc(n)) for _ in range(2)]
+    for f in "uvw":
+        fields[f] = rng.standard_normal(ctxs[0].shape(f))
+    for c in ctxs:
+        for f, a in fields.items():
+            c.upload(f, a)
+    # a tolerance that the first update meets: the V-cycle behind its check is queued
+    forms = [dict(), dict(nu1=1), dict(nu1=1, nu2=1), dict(precision="fp32", flexible=1), dict(mg_levels=6)] * 3
+    for kw in forms:
+        for wait, c in enumerate(ctxs):
+            c.step(1e-4, precond="mg", tol=0.9, **kw)
+            if wait:
+                c.sync()
+    for f in "uvwp":
+        assert np.array_equal(ctxs[0].download(f), ctxs[1].download(f)), f
