@@ -101,7 +101,7 @@ struct smac_ctx {
   // number of the last publication (waited for by wait_scalars)
   double* Sh = nullptr;
   uint64_t seq = 0;
-  double* fstage = nullptr;  // 3*1024 lane sums of the two-stage reductions
+  double* fstage = nullptr;  // FIN_ARRAYS * 1024 lane sums of the two-stage reductions
   std::vector<Level> lev;
   double* cinv = nullptr;
   double* cinv_ws = nullptr;  // work array of the coarsest inverse
@@ -484,7 +484,7 @@ extern "C" int smac_create(const smac_grid_desc* gd, const smac_fluid_desc* fl, 
     if (rc == SMAC_OK) rc = dalloc(a, c->tot);
   for (int m = 0; m < 5 && rc == SMAC_OK; m++) rc = dalloc(&c->part[m], (size_t)c->nrows);
   if (rc == SMAC_OK) rc = dalloc(&c->S, S_COUNT);
-  if (rc == SMAC_OK) rc = dalloc(&c->fstage, 3 * 1024);
+  if (rc == SMAC_OK) rc = dalloc(&c->fstage, FIN_ARRAYS * 1024);
   if (rc == SMAC_OK && hipHostMalloc((void**)&c->Sh, (S_COUNT + 1) * sizeof(double)) != hipSuccess) rc = SMAC_ERR_OOM;
   if (rc == SMAC_OK) memset(c->Sh, 0, (S_COUNT + 1) * sizeof(double));
   if (rc == SMAC_OK) {
@@ -1385,19 +1385,8 @@ static void rg_vcycle(smac_ctx* c, const smac_solver_opts& o) {
   // 2*nf sweeps: the result is back in z
 }
 
-static FinalizeArgs fin(const smac_ctx* c) {
-  FinalizeArgs fa;
-  memset(&fa, 0, sizeof(fa));
-  fa.nrows = c->nrows;
-  fa.stage = c->fstage;
-  return fa;
-}
-static void fin_add(FinalizeArgs& fa, const double* part, int kind, int out) {
-  fa.part[fa.count] = part;
-  fa.kind[fa.count] = kind;
-  fa.out[fa.count] = out;
-  fa.count++;
-}
+static FinalizeArgs fin(const smac_ctx* c, FinArray a) { return FinalizeArgs(c->nrows, c->fstage, a); }
+static FinalizeArgs fin(const smac_ctx* c, FinArray a, FinArray b) { return FinalizeArgs(c->nrows, c->fstage, a, b); }
 // The reduction fa also leaves its results in c->Sh: the host reads them after
 // wait_scalars, which waits for this kernel alone, not for what is queued
 // behind it.
@@ -1502,8 +1491,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     KT(c, "rhs", launch_rhs_eps(g, c->us, c->eps, c->eps_old, c->rhs, inv_dt, P[0], s));
   else KT(c, "rhs", launch_rhs(g, c->us, c->rhs, inv_dt, P[0], s));
   if (pure) {
-    FinalizeArgs fa = fin(c);
-    fin_add(fa, P[0], 0, S_SUMB);
+    FinalizeArgs fa = fin(c, {P[0], 0, S_SUMB});
     fa.op = OP_MEAN;
     fa.dst = S_MEANB;
     fa.sa = S_SUMB;
@@ -1519,9 +1507,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   launch_init_r<T>(g, c->rhs, c->r, f0, c->dp, zero_dp, c->S, pure ? S_MEANB : -1, 0.0, -1, P[0], P[1], 1,
                    pure ? 0 : 1, s);
   {
-    FinalizeArgs fa = fin(c);
-    fin_add(fa, P[0], 0, S_BB);
-    fin_add(fa, P[1], 0, S_SUMR);
+    FinalizeArgs fa = fin(c, {P[0], 0, S_BB}, {P[1], 0, S_SUMR});
     fin_publish(c, fa);  // read below, while the first V-cycle runs
     launch_finalize(fa, c->S, s);
   }
@@ -1531,8 +1517,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   precond();
   if (pure) {
     launch_sum<T>(g, z, P[0], s);
-    FinalizeArgs fa = fin(c);
-    fin_add(fa, P[0], 0, S_SUMZ);
+    FinalizeArgs fa = fin(c, {P[0], 0, S_SUMZ});
     launch_finalize(fa, c->S, s);
   }
   // z -= mean(z) (pure Neumann) in the same pass as d = z and r.z; rows of the
@@ -1544,8 +1529,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
   else
     launch_copy_dot<T>(g, z, c->dv, c->r, P[0], s, -1. * size_inv, c->S, pure ? S_SUMZ : -1);
   {
-    FinalizeArgs fa = fin(c);
-    fin_add(fa, P[0], 0, S_RZ);
+    FinalizeArgs fa = fin(c, {P[0], 0, S_RZ});
     launch_finalize(fa, c->S, s);
   }
   HIPOK(hipGetLastError());
@@ -1619,8 +1603,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     double* pap = ad_ready || small ? P[4] : P[0];
     ad_ready = false;
     if (!stat && !small) {
-      FinalizeArgs fa = fin(c);
-      fin_add(fa, pap, 0, S_PAP);
+      FinalizeArgs fa = fin(c, {pap, 0, S_PAP});
       fa.op = OP_DIV;
       fa.dst = S_ALPHA;
       fa.sa = S_RZ;
@@ -1641,8 +1624,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
       // solve_pureneumann_gmgpcg removes the mean of r after every update
       // (G_PCGSolver.cu:866); the check norms are taken after it
       launch_sum<double>(g, c->r, P[2], s);
-      FinalizeArgs fa = fin(c);
-      fin_add(fa, P[2], 0, S_SUMR);
+      FinalizeArgs fa = fin(c, {P[2], 0, S_SUMR});
       launch_finalize(fa, c->S, s);
       KT(c, "add_scalar_norms", launch_add_scalar_norms(g, c->r, -1. * size_inv, c->S, S_SUMR, P[0], P[1], s));
     }
@@ -1655,9 +1637,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     // for the direction pass' dp += alpha d, which is the flush's.
     const bool check = (iter % o.check_every) == 0;
     if (check) {
-      FinalizeArgs fa = fin(c);
-      fin_add(fa, P[0], 0, S_RR);
-      fin_add(fa, P[1], 1, S_LINF);
+      FinalizeArgs fa = fin(c, {P[0], 0, S_RR}, {P[1], 1, S_LINF});
       fin_publish(c, fa);
       launch_finalize(fa, c->S, s);
     }
@@ -1705,9 +1685,8 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     if (!stat && !c->dot_done && !jac)
       KT(c, "dot2", launch_dot2<T>(g, c->r, z, c->Ad, o.flexible, P[2], P[3], s));
     if (!stat && !small) {
-      FinalizeArgs fa = fin(c);
-      fin_add(fa, P[2], 0, S_RZN);
-      if (o.flexible) fin_add(fa, P[3], 0, S_ZAD);
+      const FinArray rzn_sum = {P[2], 0, S_RZN}, zad_sum = {P[3], 0, S_ZAD};
+      FinalizeArgs fa = o.flexible ? fin(c, rzn_sum, zad_sum) : fin(c, rzn_sum);
       if (o.flexible) {
         fa.op = OP_BETA_PR;
         fa.dst = S_BETA;
@@ -1781,9 +1760,7 @@ static int solve_t(smac_ctx* c, double dt, const smac_solver_opts& o, smac_solve
     st->bnorm = bnorm;
     if (have_update) {
       if (!fresh) {  // the last update was not checked
-        FinalizeArgs fa = fin(c);
-        fin_add(fa, P[0], 0, S_RR);
-        fin_add(fa, P[1], 1, S_LINF);
+        FinalizeArgs fa = fin(c, {P[0], 0, S_RR}, {P[1], 1, S_LINF});
         fin_publish(c, fa);
         launch_finalize(fa, c->S, s);
         rc = wait_scalars(c);
@@ -2211,9 +2188,7 @@ extern "C" int smac_calc_cfl(smac_ctx* c, double dt, double* cc, double* cv) {
   double visc = (1. / c->fl.rho0) * c->fl.mu0 * dt * (c->g.inv_d2[0] + c->g.inv_d2[1] + c->g.inv_d2[2]);
   const bool var = var_props(c);
   launch_cfl(c->g, V, dt, visc, var ? c->inv_rho : nullptr, var ? c->mu : nullptr, c->part[0], c->part[1], c->st);
-  FinalizeArgs fa = fin(c);
-  fin_add(fa, c->part[0], 1, S_CFLC);
-  fin_add(fa, c->part[1], 1, S_CFLV);
+  FinalizeArgs fa = fin(c, {c->part[0], 1, S_CFLC}, {c->part[1], 1, S_CFLV});
   fin_publish(c, fa);
   launch_finalize(fa, c->S, c->st);
   HIPOK(hipGetLastError());
@@ -2244,12 +2219,7 @@ extern "C" int smac_calc_cfl_noalloc(smac_ctx* c, double dt, double* cc, double*
   for (int a = 0; a < 3; a++) V.c[a] = c->u[a];
   double visc = (1. / c->fl.rho0) * c->fl.mu0 * dt * (c->g.inv_d2[0] + c->g.inv_d2[1] + c->g.inv_d2[2]);
   launch_cfl(c->g, V, dt, visc, var ? c->inv_rho : nullptr, var ? c->mu : nullptr, scr, scr + SCR_PART1, c->st);
-  FinalizeArgs fa;
-  memset(&fa, 0, sizeof(fa));
-  fa.nrows = c->nrows;
-  fa.stage = scr + SCR_STAGE;
-  fin_add(fa, scr, 1, 0);
-  fin_add(fa, scr + SCR_PART1, 1, 1);
+  FinalizeArgs fa(c->nrows, scr + SCR_STAGE, {scr, 1, 0}, {scr + SCR_PART1, 1, 1});
   launch_finalize(fa, scr + SCR_S, c->st);
   HIPOK(hipGetLastError());
   HIPOK(hipMemcpyAsync(c->Sh + S_CFLC, scr + SCR_S, 2 * sizeof(double), hipMemcpyDeviceToHost, c->st));

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "smac_dev.hpp"
 
 namespace smac {
@@ -102,20 +104,31 @@ inline int row_vpl(int n) { return n <= 64 ? 1 : (n <= 128 ? 2 : (n <= 256 ? 4 :
 
 enum { OP_NONE = 0, OP_MEAN = 1, OP_DIV = 2, OP_BETA_PR = 3 };
 
+// a reduction of row partials: kind 0 = sum, 1 = max, into slot out of S
+struct FinArray {
+  const double* part;
+  int kind, out;
+};
+// k_finalize's arguments, made from the one or the two arrays that it is built for
+constexpr int FIN_ARRAYS = 2;
 struct FinalizeArgs {
-  const double* part[3];
-  int kind[3];  // 0 = sum, 1 = max
-  int out[3];   // destination slots in S
-  int count;
+  FinalizeArgs(int rows, double* st, FinArray a) : FinalizeArgs(rows, st, a, a) { count = 1; }
+  FinalizeArgs(int rows, double* st, FinArray a, FinArray b)
+      : part{a.part, b.part}, kind{a.kind, b.kind}, out{a.out, b.out}, nrows(rows), stage(st) {}
+  const double* part[FIN_ARRAYS];
+  int kind[FIN_ARRAYS];
+  int out[FIN_ARRAYS];
+  int count = 2;
   int nrows;
-  int op, dst, sa, sb, sc;
-  double c;
-  double* stage;  // 3*1024 doubles: per-lane sums of large reductions (may be null)
+  int op = OP_NONE, dst = 0, sa = 0, sb = 0, sc = 0;
+  double c = 0.0;
+  double* stage;  // FIN_ARRAYS * 1024 doubles: lane sums of large reductions (may be null)
   // host != nullptr (pinned): the results also go to host[out[m]], then the
   // number `seq` to the word host[S_COUNT]
-  double* host;
-  uint64_t seq;
+  double* host = nullptr;
+  uint64_t seq = 0;
 };
+static_assert(!std::is_default_constructible<FinalizeArgs>::value, "a reduction has one array or two");
 
 // device scalar slots
 enum {

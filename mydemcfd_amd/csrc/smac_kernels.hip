@@ -1342,7 +1342,7 @@ __global__ __launch_bounds__(256) void k_xpay_ch(Geo g, const Z* __restrict__ z,
 }
 
 // --------------------------------------------------------------- finalize
-// Reduce up to four row-partial arrays with the canonical 1024-lane tree
+// Reduce one or two row-partial arrays with the canonical 1024-lane tree
 // (kind 0 = sum, 1 = max) into S[out[m]], then apply one scalar op.
 // lane t of the canonical tree accumulates rows t, t+1024, ... in order, B loads
 // of each of the CNT arrays in flight (past the end the last row again, not added)
@@ -2420,7 +2420,7 @@ void launch_finalize(const FinalizeArgs& fa, double* S, hipStream_t st) {
   else
     f1.stage = nullptr;
   if (fa.count == 2) hipLaunchKernelGGL(k_finalize<2>, dim3(1), dim3(1024), 0, st, f1, S);
-  else if (fa.count == 1) hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(1024), 0, st, f1, S);
+  else hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(1024), 0, st, f1, S);
 }
 // lanes per row and row slots of k_pcg_one, 0 where it does not take the grid. An
 // iteration, against 9.5 to 11 us of the two passes: one slot (64 rows of up to 32
