@@ -134,31 +134,6 @@ __device__ __forceinline__ double get_face(const Geo& g, const Vel& V, int a, I3
   return 0.;
 }
 
-// d_get_v{a}_{b}dir (CFD/G_BoundaryFunctions.h:100-367)
-__device__ __forceinline__ double get_dir(const Geo& g, const Vel& V, int a, int b, I3 q, int s) {
-  q = wr(g, q);
-  double vin = V.c[a][IX(g, q)];
-  I3 q2 = wr(g, sh(q, b, s));
-  if (face_type(g, a, q2) == F_INTERIOR) return V.c[a][IX(g, q2)];
-  I3 qf = q;
-  qf.v[b] = s > 0 ? q.v[b] + 1 : q.v[b];
-  double vw = 0.0;
-  int count = 0;
-  if (face_type(g, b, qf) == F_BOUNDARY) {
-    vw += bv_of(g, face_slot(g, b, qf), a);
-    count++;
-  }
-  I3 qf2 = wr(g, sh(qf, a, -1));
-  if (face_type(g, b, qf2) == F_BOUNDARY) {
-    vw += bv_of(g, face_slot(g, b, qf2), a);
-    count++;
-  }
-  if (count > 0) vw /= (double)count;
-  int bt = btype_of(g, face_slot(g, b, qf));
-  if (bt == BC_SLIP || bt == BC_OUTLET) return vin;
-  return 2.0 * vw - vin;
-}
-
 // d_minmod (CFD/G_SMACSolver.cu:67-88)
 __device__ __forceinline__ double minmod(double dp, double dm) {
   double prod = dp * dm;

@@ -195,18 +195,18 @@ void launch_spmv_dot(const Geo& g, const BetaF* bf, const double* d, double* Ad,
 // dp += alpha d_old, dnew = z + beta d_old and Ad = A dnew with its pair-order
 // row partials in one pass (slots of S hold alpha and beta), for rows of the
 // pair form (nx = 256 or 512, every array's rows aligned): dir_spmv_applies
-// the same for rows of any length, up to DIR_ROWS_CELLS cells
-constexpr size_t DIR_ROWS_CELLS = (size_t)1 << 22;
-bool dir_rows_applies(const Geo& g);
-template <typename Z>
-void launch_dir_rows(const Geo& g, const BetaF* bf, const Z* z, const double* dold, double* dnew, double* dp, double* Ad,
-                     double* part, double* S, hipStream_t st);
 template <typename Z>
 bool dir_spmv_applies(const Geo& g, const Z* z, const double* dold, const double* dnew, const double* dp,
                       const double* Ad);
 template <typename Z>
 void launch_dir_spmv(const Geo& g, const BetaF* bf, const Z* z, const double* dold, double* dnew, double* dp,
                      double* Ad, double* p0, const double* S, int slot_alpha, int slot_beta, hipStream_t st);
+// the same for rows of any length, up to DIR_ROWS_CELLS cells
+constexpr size_t DIR_ROWS_CELLS = (size_t)1 << 22;
+bool dir_rows_applies(const Geo& g);
+template <typename Z>
+void launch_dir_rows(const Geo& g, const BetaF* bf, const Z* z, const double* dold, double* dnew, double* dp, double* Ad,
+                     double* part, double* S, hipStream_t st);
 // k_copy_dot and the SpMV after it in one pass, the first SpMV of a solve:
 // d = z (slot >= 0: z + a S[slot] rounded to the storage of z), Ad = A d,
 // p_dad <- the rows' d.Ad and p_rz <- their r.d, both in pair order; the same

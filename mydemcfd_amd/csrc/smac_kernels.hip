@@ -1466,8 +1466,8 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs fa, double* __re
 // with Jacobi nine kernels of 1.7 to 5.5 us each on 64^3, three of them
 // reductions of a few thousand row partials in one block. Here every block of
 // the two kernels that need a scalar forms it for itself from the row partials
-// (32 KB at most 256 times from the L2), in the canonical order, so an
-// iteration is k_pcg_dir and k_pcg_res, with the V-cycle and its dots between
+// (from the L2, at most 64 KB an array and 512 blocks), in the canonical order, so
+// an iteration is k_pcg_dir and k_pcg_res, with the V-cycle and its dots between
 // them when there is one. Block 0 leaves the scalars in S for the next kernel;
 // r.z alternates between two slots, since its old value is read by every block
 // that may still be running.

@@ -1619,12 +1619,11 @@ __device__ void coarsest_coef(const Lv& L, int i, int j, int k, double a6[6], do
 // hold a row per lane in registers and broadcast by readlane, no barrier),
 // which costs less than a launch of its own per panel. The back substitution
 // subtracts l_ki x_k in increasing k, newest first, so it is one serial chain
-// of n^2/2 subtractions per column: a wave owns a few columns with x in LDS
-// and the other three waves stage the rows of L^T ahead of it. That chain is
-// the bound (12 ns a step of a lone wave). 512 cells 1.8 ms (16 panels of 14 to
-// 20 us, then 1.55 ms), 128 cells 0.23 ms, 90 cells 0.14 ms; one workgroup for
-// everything (a column at a time, operands from the L2) took 29.6 ms for 480
-// cells, 0.99 ms for 128 and 0.53 ms for 90.
+// of n^2/2 subtractions per column (k_pinv_back): that chain is the bound. 512
+// cells 1.0 ms (16 panels of 11 to 21 us, then 0.73 ms), 480 cells 0.89 ms, 128
+// cells 0.16 ms, 90 cells 0.12 ms; one workgroup for everything (a column at a
+// time, operands from the L2) took 29.6 ms for 480 cells, 0.99 ms for 128 and
+// 0.53 ms for 90.
 constexpr int PB = 32;       // panel and tile width
 constexpr int PINV_MAX = 1024;
 

@@ -510,10 +510,13 @@ dim3 tile_grid(const Lv& L) {
 
 }  // namespace
 
-// Row kernels against the tile, down and up together: 32^3 uniform BF16 16 us
-// against 31, 64^3 29 against 45, 64x32x32 variable FP32 17 against 43; but
-// 128x64x64 variable FP32 78 against 65 and 96x48x80 variable FP64 70 against
-// 45, where the halo's work outweighs the launches.
+// An iteration of the PCG with the level's half V-cycles by the tiles against by the
+// row kernels: uniform 32^3 BF16 51 us against 87, 64^3 BF16 80 against 94, FP32 76
+// against 91, FP64 87 against 90, 128x64x64 FP32 109 against 106, FP64 130 against 111;
+// variable 64x32x32 FP32 60 against 87, 128x64x32 FP32 88 against 94, BF16 92 against
+// 94, 128x64x64 FP32 136 against 113; variable FP64 64x64x32 74 against 90, 96x48x40 99
+// against 98, 128x64x32 98 against 96. Past the limits the halo's work outweighs the
+// launches.
 template <typename T>
 bool mg_tile_applies(const Lv& L) {
   const size_t cells = (size_t)L.n[0] * L.n[1] * L.n[2];

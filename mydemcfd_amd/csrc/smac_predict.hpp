@@ -52,9 +52,10 @@ __device__ __forceinline__ double wall_value(const Geo& g, int a, int s, double 
   if (wall_stored(g, a, s)) return stored;
   return g.btype[s] == BC_INFLOW ? (1. - 0.0) * g.bv[s][a] : 0.;
 }
-// Component a beyond the wall on side s of a tangential axis, next to the value
-// v, as get_dir gives it: both faces it averages lie on that side, so its wall
-// velocity is the side's
+// Component a beyond the wall on side s of a tangential axis, next to the value v
+// (d_get_v{a}_{b}dir, CFD/G_BoundaryFunctions.h:100-367): v itself at a slip or
+// outlet side, else mirrored about the wall velocity. That is there the mean of the
+// two wall faces next to it, which both lie on the side, so the side's
 __device__ __forceinline__ bool wall_even(const Geo& g, int s) {
   return g.btype[s] == BC_SLIP || g.btype[s] == BC_OUTLET;
 }
