@@ -485,7 +485,11 @@ extern "C" int smac_create(const smac_grid_desc* gd, const smac_fluid_desc* fl, 
   for (int m = 0; m < 5 && rc == SMAC_OK; m++) rc = dalloc(&c->part[m], (size_t)c->nrows);
   if (rc == SMAC_OK) rc = dalloc(&c->S, S_COUNT);
   if (rc == SMAC_OK) rc = dalloc(&c->fstage, FIN_ARRAYS * 1024);
-  if (rc == SMAC_OK && hipHostMalloc((void**)&c->Sh, (S_COUNT + 1) * sizeof(double)) != hipSuccess) rc = SMAC_ERR_OOM;
+  // coherent by request: the host reads what a kernel stored while later ones run
+  // (the default follows the environment's HIP_HOST_COHERENT)
+  if (rc == SMAC_OK &&
+      hipHostMalloc((void**)&c->Sh, (S_COUNT + 1) * sizeof(double), hipHostMallocCoherent) != hipSuccess)
+    rc = SMAC_ERR_OOM;
   if (rc == SMAC_OK) memset(c->Sh, 0, (S_COUNT + 1) * sizeof(double));
   if (rc == SMAC_OK) {
     c->ev_ok = true;
